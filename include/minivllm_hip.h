@@ -500,6 +500,30 @@ int mvllm_argmax(int64_t* out, const void* logits, int64_t rows, int64_t vocab,
  * Rows may hold up to 64 segments (1048576 logits). */
 uint64_t mvllm_argmax_workspace_bytes(int64_t rows, int64_t vocab);
 
+/* The distribution each row's token is drawn from (reference mini_vllm/sampler.py:71-124):
+ * softmax(logits / temperature) with the tokens outside top-k and top-p removed and the
+ * rest renormalised, in vocabulary order; a greedy row (temperature 0) is the one-hot of
+ * its mvllm_argmax. In descending order of logits / temperature (float32; equal values in
+ * vocabulary order) a token is kept while fewer than top_k tokens and less than top_p of
+ * the mass come before it, and the first always. A row holding NaN, or whose scaled
+ * maximum is not finite, is all NaN. No counterpart in mini_vllm_C (the reference sorts with
+ * torch).
+ *   probs [rows, vocab] float32; logits `rows` rows of `vocab` f32/f16/bf16, row_stride
+ *   elements apart; params: one per row, host memory, read before the call returns.
+ * vocab at most 1048576 (MVLLM_ERR_UNSUPPORTED beyond). Four launches per 128 rows. */
+typedef struct mvllm_sampling_row {
+  float temperature; /* >= 0 */
+  float top_p;       /* > 0; >= 1: no limit */
+  int32_t top_k;     /* <= 0 or >= vocab: no limit */
+} mvllm_sampling_row;
+int mvllm_sampling_probabilities(float* probs, const void* logits, int64_t rows, int64_t vocab,
+                                 int64_t row_stride, int32_t dtype,
+                                 const mvllm_sampling_row* params, void* workspace,
+                                 uint64_t workspace_bytes, void* stream);
+/* Its workspace (256-byte aligned, contents need not be initialised): about 2.4 bytes per
+ * logit of at most 128 rows. */
+uint64_t mvllm_sampling_workspace_bytes(int64_t rows, int64_t vocab);
+
 /* Read-only HBM probe for the benchmark's bandwidth ceiling (no counterpart in the
  * reference, whose ceiling is a device copy, mini_vllm/bench.py:448-466): reads
  * `num_pages` pages of `page_bytes` (4-64 KB, a multiple of 4 KB) from `base`, page i at

@@ -21,6 +21,7 @@
 #include "kv_write.hpp"
 #include "linear.hpp"
 #include "sampler.hpp"
+#include "sampling.hpp"
 #include "paged_attention.hpp"
 #include "probe.hpp"
 
@@ -572,7 +573,7 @@ extern "C" {
 
 const char* mvllm_last_error(void) { return g_error; }
 
-int mvllm_abi_version(void) { return 15; }
+int mvllm_abi_version(void) { return 16; }
 
 #ifndef MVLLM_SOURCE_HASH
 #define MVLLM_SOURCE_HASH "unstamped"
@@ -1017,6 +1018,60 @@ int mvllm_argmax(int64_t* out, const void* logits, int64_t rows, int64_t vocab,
   return hip_status(mvllm::launch_argmax(out, logits, rows, vocab, row_stride, dtype, workspace,
                                          static_cast<hipStream_t>(stream)),
                     "argmax: launch");
+}
+
+uint64_t mvllm_sampling_workspace_bytes(int64_t rows, int64_t vocab) {
+  if (rows < 1 || vocab < 1 || vocab > mvllm::sampling_max_vocab()) return 0;
+  return mvllm::sampling_workspace_bytes(rows, vocab);
+}
+int mvllm_sampling_probabilities(float* probs, const void* logits, int64_t rows, int64_t vocab,
+                                 int64_t row_stride, int32_t dtype,
+                                 const mvllm_sampling_row* params, void* workspace,
+                                 uint64_t workspace_bytes, void* stream) {
+  static_assert(sizeof(mvllm_sampling_row) == sizeof(mvllm::SamplingRow) &&
+                    offsetof(mvllm_sampling_row, top_p) == offsetof(mvllm::SamplingRow, top_p) &&
+                    offsetof(mvllm_sampling_row, top_k) == offsetof(mvllm::SamplingRow, top_k),
+                "the ABI's row is the launcher's");
+  g_error[0] = '\0';
+  if (dtype != mvllm::kF32 && dtype != mvllm::kF16 && dtype != mvllm::kBF16) {
+    return fail(MVLLM_ERR_UNSUPPORTED,
+                "sampling_probabilities: dtype code %d is not served (f32, f16, bf16)", dtype);
+  }
+  if (rows < 0 || rows >= (int64_t{1} << 31) || vocab <= 0 || row_stride < vocab) {
+    return fail(MVLLM_ERR_INVALID,
+                "sampling_probabilities: %lld rows of %lld logits, %lld apart: rows must be < "
+                "2^31, the row non-empty, the stride at least the row",
+                static_cast<long long>(rows), static_cast<long long>(vocab),
+                static_cast<long long>(row_stride));
+  }
+  if (vocab > mvllm::sampling_max_vocab()) {
+    return fail(MVLLM_ERR_UNSUPPORTED, "sampling_probabilities: rows of %lld logits, at most %lld",
+                static_cast<long long>(vocab), static_cast<long long>(mvllm::sampling_max_vocab()));
+  }
+  if (rows == 0) return MVLLM_OK;
+  if (probs == nullptr || logits == nullptr || params == nullptr) {
+    return fail(MVLLM_ERR_INVALID, "sampling_probabilities: a required pointer is NULL");
+  }
+  for (int64_t r = 0; r < rows; ++r) {
+    if (!(params[r].temperature >= 0.0f) || !(params[r].top_p > 0.0f)) {
+      return fail(MVLLM_ERR_INVALID,
+                  "sampling_probabilities: row %lld: temperature must be >= 0 and top_p > 0",
+                  static_cast<long long>(r));
+    }
+  }
+  const uint64_t need = mvllm::sampling_workspace_bytes(rows, vocab);
+  if (workspace == nullptr || workspace_bytes < need ||
+      reinterpret_cast<uintptr_t>(workspace) % 256 != 0) {
+    return fail(MVLLM_ERR_WORKSPACE,
+                "sampling_probabilities: needs %llu bytes of 256-byte aligned workspace "
+                "(mvllm_sampling_workspace_bytes), got %llu",
+                static_cast<unsigned long long>(need), static_cast<unsigned long long>(workspace_bytes));
+  }
+  return hip_status(mvllm::launch_sampling_probabilities(
+                        probs, logits, rows, vocab, row_stride, dtype,
+                        reinterpret_cast<const mvllm::SamplingRow*>(params), workspace,
+                        static_cast<hipStream_t>(stream)),
+                    "sampling_probabilities: launch");
 }
 
 int mvllm_rmsnorm(void* out, const void* x, const void* weight, int64_t rows, int64_t dim,

@@ -22,6 +22,7 @@ import ctypes
 import hashlib
 import math
 import os
+import struct
 import subprocess
 import sys
 import threading
@@ -68,7 +69,7 @@ EXTRA_FLAGS = {"elementwise.hip": ["-ffp-contract=off"], "linear.hip": ["-ffp-co
 # process that has imported torch the library binds to that copy.
 LINK_LIBS = ["-L/opt/rocm/lib", "-lhipblaslt"]
 
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 DTYPE_CODES: dict[torch.dtype, int] = {
     torch.float32: 0,
@@ -239,6 +240,9 @@ class _BlasChoice(ctypes.Structure):
     ]
 
 
+# ``mvllm_sampling_row`` of include/minivllm_hip.h: temperature, top_p, top_k.
+_SAMPLING_ROW = struct.Struct("@ffi")
+
 DECODE_MODES = {0: "none", 1: "stream", 2: "grid", 3: "by_row"}
 
 
@@ -300,6 +304,10 @@ def _bind(lib: ctypes.CDLL) -> None:
     lib.mvllm_argmax.argtypes = [p, p, i64, i64, i64, i32, p, u64, p]
     lib.mvllm_argmax_workspace_bytes.restype = u64
     lib.mvllm_argmax_workspace_bytes.argtypes = [i64, i64]
+    lib.mvllm_sampling_probabilities.restype = ctypes.c_int
+    lib.mvllm_sampling_probabilities.argtypes = [p, p, i64, i64, i64, i32, p, p, u64, p]
+    lib.mvllm_sampling_workspace_bytes.restype = u64
+    lib.mvllm_sampling_workspace_bytes.argtypes = [i64, i64]
     lib.mvllm_linear_pack.restype = ctypes.c_int
     lib.mvllm_linear_pack.argtypes = [p, p, i64, i64, i32, p]
     lib.mvllm_linear_workspace_bytes.restype = u64
@@ -351,6 +359,8 @@ EXPORTED_SYMBOLS = (
     "mvllm_qk_norm_rope_kv_write",
     "mvllm_paged_decode_qk_norm_rope",
     "mvllm_argmax_workspace_bytes",
+    "mvllm_sampling_probabilities",
+    "mvllm_sampling_workspace_bytes",
     "mvllm_dense_attention_plan",
     "mvllm_dense_attention",
     "mvllm_linear_pack",
@@ -1099,6 +1109,37 @@ class HipExtension:
                                           ws.data_ptr() if ws is not None else 0, need,
                                           _stream(logits.device)))
         return out
+
+    @staticmethod
+    def sampling_supported(logits: torch.Tensor) -> bool:
+        """Whether ``sampling_probabilities`` serves these logits: f32/f16/bf16
+        device rows of contiguous entries, 1 to 1048576 each. (One row of 8 logits takes
+        39 us against 212 us on torch's path, 20000 such rows 6.1 ms against 11.8 ms, 512
+        of 151936 0.55 ms against 7.6 ms.)"""
+        return (logits.is_cuda and logits.dim() == 2
+                and logits.dtype in (torch.float32, torch.float16, torch.bfloat16)
+                and logits.shape[0] > 0
+                and 0 < logits.shape[1] <= 1 << 20 and logits.stride(1) == 1
+                and (logits.shape[0] == 1 or logits.stride(0) >= logits.shape[1]))
+
+    def sampling_probabilities(self, logits: torch.Tensor, rows: list) -> torch.Tensor:
+        """The fp32 ``B x V`` distribution of each row of ``logits`` under its
+        ``(temperature, top_p, top_k)`` (``mvllm_sampling_probabilities``)."""
+        if not self.sampling_supported(logits):
+            raise RuntimeError(f"sampling_probabilities: logits {tuple(logits.shape)} "
+                               f"{logits.dtype} strides {logits.stride()} are not served")
+        batch, vocab = logits.shape
+        if len(rows) != batch:
+            raise RuntimeError(f"sampling_probabilities: {len(rows)} rows of parameters for "
+                               f"{batch} rows of logits")
+        packed = b"".join(_SAMPLING_ROW.pack(t, p, min(k, vocab)) for t, p, k in rows)
+        probs = torch.empty((batch, vocab), dtype=torch.float32, device=logits.device)
+        ws = self.workspace(logits.device, self.lib.mvllm_sampling_workspace_bytes(batch, vocab))
+        self._check(self.lib.mvllm_sampling_probabilities(
+            probs.data_ptr(), logits.data_ptr(), batch, vocab, max(logits.stride(0), vocab),
+            DTYPE_CODES[logits.dtype], packed, ws.data_ptr(), ws.numel(),
+            _stream(logits.device)))
+        return probs
 
     # -- dense-cache attention (reference csrc/decode_attention.cu, csrc/flash_prefill.cu)
     @staticmethod

@@ -71,6 +71,7 @@ __all__ = [
     "qk_norm_rope_kv_write",
     "rmsnorm",
     "rope",
+    "sampling_probabilities",
     "set_strict",
     "strict_kernels",
     "swiglu",
@@ -82,7 +83,7 @@ CUDA_KERNELS: dict[str, tuple[bool, str]] = {
     "rmsnorm": (True, "csrc/elementwise.hip"),
     "rope": (True, "csrc/elementwise.hip"),
     "swiglu": (True, "csrc/elementwise.hip"),
-    "argmax": (True, "csrc/sampler.hip"),
+    "argmax": (True, "csrc/sampler.hip, the sampling distribution csrc/sampling.hip"),
     "decode_attention": (True, "csrc/dense.hip over the paged decode kernels"),
     "flash_prefill": (True, "csrc/dense.hip over the paged prefill kernels"),
     "paged_attention": (True, "csrc/paged_decode.hip + csrc/paged_prefill.hip"),
@@ -353,6 +354,32 @@ def argmax(logits: torch.Tensor, use_cuda: bool = False,
     if out is None:
         return logits.argmax(dim=-1)
     return torch.argmax(logits, dim=-1, out=out)
+
+
+def sampling_probabilities(logits: torch.Tensor, rows, use_cuda: bool = False) -> torch.Tensor | None:
+    """The distribution each row of ``logits`` is drawn from under its parameters
+    (``rows``: objects with ``temperature``, ``top_k`` and ``top_p``, reference
+    sampler.py:71-124). Kernel: ``csrc/sampling.hip``. None where it does not serve the
+    call (the PyTorch path, float64 logits, logits that are traced or differentiated, a
+    temperature or top_p outside float32): the caller then sorts with torch."""
+    if not _use_kernel("argmax", use_cuda, logits) or not _plain(logits):
+        return None
+    ext = load_extension()
+    if not ext.sampling_supported(logits):
+        return None
+    params = [(float(r.temperature), float(r.top_p), int(r.top_k)) for r in rows]
+    if any(not (t == 0.0 or 1e-37 < t < 3e38) or p < 1e-37 for t, p, _ in params):
+        return None
+    return ext.sampling_probabilities(logits, params)
+
+
+def _plain(x: torch.Tensor) -> bool:
+    """A tensor whose memory a kernel may read in torch's place: not a subclass or a
+    functorch wrapper, not under a trace, and with no derivative asked for."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and torch.autograd.forward_ad._current_level < 0
+            and not (x.requires_grad and torch.is_grad_enabled()))
 
 
 @dataclass(frozen=True)

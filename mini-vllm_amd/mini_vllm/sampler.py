@@ -15,10 +15,11 @@ from, as the reference defines it:
 
 How it runs here: the whole batch stays on the device and nothing is read back by
 the host. Greedy-only batches never build probabilities (the argmax kernel,
-``ops.argmax``); batches without truncation take a softmax without sorting; only rows
-that truncate pay for a sort of the vocabulary, which is stable, so equal
-probabilities keep vocabulary order (lower token id first) and the kept set is
-deterministic. Draws take a ``torch.Generator`` (on the logits' device) and are
+``ops.argmax``). Device logits take ``csrc/sampling.hip``, which selects each row's last
+kept token without sorting. The PyTorch path (CPU tensors, float64 logits, logits under
+autograd) softmaxes rows without truncation and sorts the vocabulary of rows that
+truncate. Equal values keep vocabulary order (lower token id first) either way, so the
+kept set is deterministic. Draws take a ``torch.Generator`` (on the logits' device) and are
 reproducible under it.
 """
 
@@ -106,6 +107,10 @@ def sampling_probabilities(logits: torch.Tensor,
     batch, _ = logits.shape
     rows = _rows(params, batch)
     use_cuda = logits.is_cuda
+    if use_cuda:
+        probs = ops.sampling_probabilities(logits, rows, use_cuda=True)
+        if probs is not None:
+            return probs
     greedy = [r.is_greedy for r in rows]
     result = torch.empty(logits.shape, dtype=torch.float32, device=logits.device)
     if not all(greedy):

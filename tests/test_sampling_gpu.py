@@ -1,0 +1,99 @@
+"""The sampling distribution's kernels (``ops.sampling_probabilities``) on the MI355X
+(``-m gpu``), against the float64 oracle: the kept sets exactly, the probabilities within
+fp32 rounding: the scaled logit x and its distance from the maximum m are each rounded once
+(2^-24 of their size, an absolute error of the exponent), expf, the sum and the division add
+a few 2^-24, and the sum's own terms err as much again."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from mini_vllm.kernels import ops
+from mini_vllm.sampler import SamplingParams, sampling_probabilities
+from oracle import sampler as oracle
+
+pytestmark = pytest.mark.gpu
+
+PARAMS = [SamplingParams(0.7, 0, 0.9), SamplingParams(0.0), SamplingParams(1.3, 5, 1.0),
+          SamplingParams(1.0), SamplingParams(0.9, 40, 0.6), SamplingParams(1.0, 0, 1e-6),
+          SamplingParams(2.0, 3000, 0.999)]
+
+
+def check(logits, rows):
+    got = ops.sampling_probabilities(logits, rows, use_cuda=True)
+    assert got is not None and got.dtype == torch.float32 and got.shape == logits.shape
+    want = torch.from_numpy(oracle.sampling_probabilities(
+        logits.float().cpu().numpy(), [torch.tensor(r.temperature).item() for r in rows],
+        [r.top_k for r in rows], [torch.tensor(r.top_p).item() for r in rows]))
+    got = got.double().cpu()
+    tiny = want < 1e-30  # fp32 exponentials end there
+    assert torch.equal(got[~tiny] > 0, want[~tiny] > 0), "kept sets differ"
+    x = logits.float().cpu()
+    x = x / torch.tensor([r.temperature or 1.0 for r in rows])[:, None]
+    size = x[x.isfinite()].abs().max().item()
+    assert torch.allclose(got, want, rtol=2 * (3 * size + 8) * 2.0 ** -24, atol=1e-30)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vocab", [1, 3, 8, 511, 16384, 16385, 50257, 151936])
+def test_matches_the_oracle(device, vocab, dtype):
+    """Vocabularies around a chunk, a segment and several, aligned and not, rows of every
+    kind in one call; 16-bit logits tie often."""
+    gen = torch.Generator().manual_seed(vocab)
+    logits = (torch.randn(len(PARAMS), vocab, generator=gen) * 2.5).to(dtype).to(device)
+    check(logits, PARAMS)
+
+
+@pytest.mark.parametrize("vocab", [700, 151936])
+def test_many_tokens_at_the_boundary(device, vocab):
+    """Flat rows: every token in one bin, all equal (kept by index) or apart by less than
+    a bin, so the selection narrows thousands of tokens; a row far below its one peak."""
+    flat = torch.full((vocab,), 1.5)
+    close = torch.linspace(0.0, 0.05, vocab)[torch.randperm(vocab)]
+    peak = torch.full((vocab,), -200.0)
+    peak[vocab // 2] = 10.0
+    rows = [SamplingParams(1.0, 0, 0.37), SamplingParams(1.0, vocab // 3, 1.0),
+            SamplingParams(0.5, 0, 0.37), SamplingParams(1.0, vocab // 2, 0.9),
+            SamplingParams(1.0, 600, 1.0), SamplingParams(1.0, 0, 0.5)]
+    check(torch.stack([flat, flat, close, close, peak, peak]).to(device), rows)
+
+
+def test_strided_rows_many_rows_and_signed_zeros(device):
+    base = torch.randn(300, 1203, device=device)
+    base[:, ::2] = 0.0
+    base[:, 1::4] = -0.0
+    rows = [PARAMS[i % len(PARAMS)] for i in range(300)]
+    check(base[:, 3:1003], rows)
+
+
+def test_non_finite_rows(device):
+    """-inf tokens have no mass; a row holding NaN or +inf, or nothing but -inf, is all NaN
+    (as softmax gives it); its neighbours are untouched."""
+    x = torch.randn(6, 20000)
+    x[0, 7:] = float("-inf")
+    x[1, 19999] = float("nan")
+    x[2, 3] = float("inf")
+    x[3] = float("-inf")
+    rows = [SamplingParams(0.8, 4, 0.95), SamplingParams(0.8, 4, 0.95), SamplingParams(1.0),
+            SamplingParams(1.0, 0, 0.9), SamplingParams(0.0), SamplingParams(1.0, 2)]
+    got = ops.sampling_probabilities(x.to(device), rows, use_cuda=True).cpu()
+    assert bool(got[1:4].isnan().all())
+    keep = [0, 4, 5]
+    check(x[keep].to(device), [rows[i] for i in keep])
+    assert torch.equal(got[keep], ops.sampling_probabilities(
+        x[keep].to(device), [rows[i] for i in keep], use_cuda=True).cpu())
+
+
+def test_what_stays_on_the_torch_path(device):
+    """Autograd, float64 and parameters outside float32 keep the torch path and its
+    results."""
+    x = torch.randn(2, 50, device=device)
+    rows = [SamplingParams(0.7, 5, 0.9), SamplingParams()]
+    grad = x.clone().requires_grad_()
+    p = sampling_probabilities(grad, rows[:1] * 2)
+    assert p.requires_grad
+    assert torch.allclose(p.detach(), sampling_probabilities(x, rows[:1] * 2), rtol=1e-5)
+    assert ops.sampling_probabilities(x.double(), rows, use_cuda=True) is None
+    for odd in (SamplingParams(1e-40), SamplingParams(1e39), SamplingParams(1.0, 0, 1e-40)):
+        assert ops.sampling_probabilities(x, [odd, odd], use_cuda=True) is None

@@ -64,13 +64,14 @@ typedef struct mvllm_paged_plan {
   int32_t split_tokens;      /* grid modes: keys per split */
   int32_t prefill_mfma;      /* 1: prefill rows go to the MFMA prefill kernel */
   uint64_t workspace_bytes;  /* split partials and their index; 0 when none are needed */
-  int32_t prefill_workgroups; /* MFMA prefill: > 0 persistent workgroups with balanced
-                                 shares of all key tiles (cut items merged after);
-                                 0 one workgroup per (sequence, heads, query tile) */
-  int32_t prefill_pieces;     /* MFMA prefill on the grid: > 1 items longer than ~1.2x
-                                 the mean work per CU are cut into at most this many key
-                                 ranges, run in the same launch longest first and merged
-                                 by the last to finish; 0 every item whole */
+  int32_t prefill_workgroups; /* MFMA prefill: > 0 the stream schedule, balanced shares of
+                                 all key tiles for this many workgroups (cut items merged
+                                 after); 0 the grid, a workgroup per (sequence, heads,
+                                 query tile) */
+  int32_t prefill_pieces;     /* MFMA prefill on the grid: > 1 items longer than
+                                 prefill_piece_pct of the mean work per CU may be cut into
+                                 at most this many key ranges (merged after); 0 every item
+                                 whole */
 } mvllm_paged_plan;
 
 /* Explicit overrides of the planner's schedule choices, for measurement and for tests
@@ -98,12 +99,12 @@ typedef struct mvllm_plan_options {
                                   at least 50) */
 } mvllm_plan_options;
 
-/* The split prefill grid's arrival counters: regions taken on the current device (one
- * per stream that ran a split launch, at most 32), and the split launches (all devices)
- * that ran every item whole instead because no region was left or because their
- * stream was being captured into a graph (a captured launch must not name a stream's
- * counters: a replay on another stream could overlap it). No counterpart in the
- * reference. Any pointer may be NULL. */
+/* Prefills whose plan cut items on the grid but that ran every item whole because their
+ * stream was being captured into a graph (so a graph's result does not depend on how the
+ * lengths at capture would have been cut). The merge of cut items is a launch of its own
+ * over the caller's workspace: there are no arrival counters, so `regions_used` and
+ * `whole_no_region`, which described them, are 0. No counterpart in the reference. Any
+ * pointer may be NULL. */
 void mvllm_split_stats(int32_t* regions_used, int64_t* whole_no_region,
                        int64_t* whole_capturing);
 

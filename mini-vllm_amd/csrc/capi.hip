@@ -72,6 +72,7 @@ struct Options {
   int prefill_share_tiles = mvllm::kPrefillShareTiles;
   int prefill_staging = 0;
   int prefill_pieces = mvllm::kSplitDefaultPieces;
+  bool pieces_given = false;  // prefill_pieces is the caller's, not the default
   int prefill_piece_pct = mvllm::kSplitDefaultPct;
 };
 
@@ -95,6 +96,7 @@ int read_options(const mvllm_plan_options* o, Options& out) {
   if (o->prefill_share_tiles > 0) out.prefill_share_tiles = o->prefill_share_tiles;
   out.prefill_staging = o->prefill_staging;
   if (o->prefill_pieces > 0) out.prefill_pieces = o->prefill_pieces;
+  out.pieces_given = o->prefill_pieces > 0;
   if (o->prefill_piece_pct > 0) out.prefill_piece_pct = o->prefill_piece_pct;
   return MVLLM_OK;
 }
@@ -143,6 +145,9 @@ int check_paged_shape(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t 
   return MVLLM_OK;
 }
 
+// Pieces of one item on the stream schedule (as many as the grid's option allows).
+constexpr int kStreamPieces = 64;
+
 // A plan plus the workspace layout it implies.
 struct Plan {
   mvllm_paged_plan pub;
@@ -154,10 +159,16 @@ struct Plan {
   uint64_t off_pf = 0;      // stream prefill: [prefix][O partials][(m, l) partials]
   uint64_t off_pf_o = 0;
   uint64_t off_pf_ml = 0;
-  int split_ranks = 0;      // split prefill grid: rank extent, partial slots per column,
-  int split_slots = 0;      // piece length (percent of the mean tiles per CU)
+  // The pair prefill kernel's split schedule (paged_prefill.hip): pieces per item (<= 1:
+  // every item whole), rank extent, partial slots per column, piece length (percent of the
+  // mean tiles per workgroup of `split_wgs`); its slots and its ranks' records.
+  int split_pieces = 0;
+  int split_ranks = 0;
+  int split_slots = 0;
   int split_pct = 0;
-  uint64_t off_split = 0;   // split prefill grid: the partial slots
+  int split_wgs = 0;
+  uint64_t off_split = 0;
+  uint64_t off_rec = 0;
 };
 
 uint64_t align256(uint64_t v) { return (v + 255) / 256 * 256; }
@@ -166,67 +177,92 @@ void plan_decode(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, i
                  int32_t d, int32_t block_size, int32_t max_q, int32_t max_ctx, int32_t q_dtype,
                  int32_t kv_dtype, const Options& o);
 
-// The MFMA prefill's schedule. The grid (one workgroup per 128-query item) is chosen
-// when there are at least half as many items as CUs: the hardware dispatcher then
-// balances them, with no partials to merge (four 512-query chunks beside 28 decodes,
-// 136 items: grid 102 us, stream 110 us). With fewer items (one chunk of a long
-// prompt, 40 items: stream 104 us, grid 109 us) the grid would leave CUs idle behind a
-// few long items, so
-// the stream schedule is used: one persistent workgroup per CU (times the
-// prefill_wgs_per_cu option) with balanced shares of all key tiles, cut items merged
-// after (measured at 8K-16K contexts: 2.5-3x the grid). The item count is estimated
-// from host sizes: ceil(num_tokens / 128) query tiles per kv column. The
-// prefill_schedule option 1 / 2 forces stream / grid. The stream's workspace follows
-// the decode part's.
-// The grid's split (pieces of long items, merged in the same launch) where the
-// pipelined kernel runs it: D = 128, GQA pairs, pages of >= 16 keys, 16-bit or fp8
-// pools, and at most kSplitMaxItems items (bounded from host sizes: a sequence of L
-// queries has ceil(L / 128) items, so there are at most min(num_seqs * ceil(max_q /
-// 128), ceil(num_tokens / 128) + num_seqs)) over at most kSplitMaxCols columns.
-void plan_split(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t hk,
-                int32_t d, int32_t block_size, int32_t max_q, int32_t q_dtype, int32_t kv_dtype,
-                const Options& o) {
-  if (o.prefill_pieces < 2 || o.prefill_staging != 0 || d != 128 ||
-      mvllm::prefill_item_heads(hq / hk) != 2 || block_size < 16) {
-    return;
-  }
-  if (q_dtype != mvllm::kF16 && q_dtype != mvllm::kBF16) return;
-  if (kv_dtype != q_dtype && kv_dtype != mvllm::kFP8E4M3) return;
-  const int64_t q_tiles = (max_q + mvllm::kPrefillQueryTile - 1) / mvllm::kPrefillQueryTile;
-  const int64_t by_seqs = static_cast<int64_t>(num_seqs) * q_tiles;
-  const int64_t by_tokens =
-      (static_cast<int64_t>(num_tokens) + mvllm::kPrefillQueryTile - 1) / mvllm::kPrefillQueryTile +
-      num_seqs;
-  const int64_t items = by_seqs < by_tokens ? by_seqs : by_tokens;
-  const int cols = hq / 2;
-  if (items > mvllm::kSplitMaxItems || cols > mvllm::kSplitMaxCols) return;
-  const int cus = device_cus();
-  plan.pub.prefill_pieces = o.prefill_pieces;
-  plan.split_pct = o.prefill_piece_pct;
-  plan.split_ranks = static_cast<int>(items) + mvllm::split_extra_ranks(cus, cols, plan.split_pct);
-  plan.split_slots = mvllm::split_slots(cus, cols, plan.split_pct);
-  plan.off_split = align256(plan.pub.workspace_bytes);
-  plan.pub.workspace_bytes =
-      plan.off_split + static_cast<uint64_t>(plan.split_slots) * cols * mvllm::kSplitSlotFloats *
-                           sizeof(float);
+// Whether the pair prefill kernel serves these prefill rows (but for the sign of the
+// scale, which only the launch knows): D = 128, GQA pairs, pages of >= 16 keys, 16-bit
+// queries over a pool of their type or fp8.
+bool pair_prefill(int32_t hq, int32_t hk, int32_t d, int32_t block_size, int32_t q_dtype,
+                  int32_t kv_dtype, const Options& o) {
+  return o.prefill_staging == 0 && d == 128 && mvllm::prefill_item_heads(hq / hk) == 2 &&
+         block_size >= 16 && (q_dtype == mvllm::kF16 || q_dtype == mvllm::kBF16) &&
+         (kv_dtype == q_dtype || kv_dtype == mvllm::kFP8E4M3);
 }
 
+// Whether the pair kernel should cut its items. With few items the longest, of n = max_ctx /
+// 64 tiles at 0.93 us each, sets the time while CUs idle; cut, the tiles spread over all CUs
+// at 1.25 us each (every CU then streams its own keys), for 13 us more of schedule, partials
+// and merge. Whole against cut: one 512-token chunk (64 items) fresh 15 and 24 us, after
+// 1000 keys 28.3 and 27.4, after 8000 126 and 57; 63 tokens after 6393 (8 items) 97 and 23;
+// 1024 tokens after 4000 (128 items) 77 and 70; two 512-token chunks after 1000 (128 items) 29
+// and 36. With more items than half the CUs an even batch is best whole; only a sequence
+// far longer than the others gains, which the host cannot see, so several sequences with
+// contexts past 96 tiles are cut where an item exceeds the piece length (a 2048-token chunk
+// after 6000 keys, where none does: 131 us whole, 144 through the schedule and the empty merge).
+bool pair_wants_split(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max_ctx, int cus) {
+  const int64_t wgs = static_cast<int64_t>((num_tokens + mvllm::kPairQueryTile - 1) /
+                                           mvllm::kPairQueryTile) * (hq / 2);
+  const int64_t n = (static_cast<int64_t>(max_ctx) + mvllm::kPrefillKeyTile - 1) / mvllm::kPrefillKeyTile;
+  if (2 * wgs > cus) return num_seqs > 1 && n > 96;
+  return n * (93 * cus - 125 * wgs) > 1300 * static_cast<int64_t>(cus);
+}
+
+// The split's extents over `wgs` workgroups' shares: ranks are the items' bound (a
+// sequence of L queries has ceil(L / 64) items) plus the extra pieces'. Left whole past
+// kSplitMaxRanks: each position is a workgroup, and one without a piece still costs ~4 ns.
+void plan_split(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max_q,
+                int wgs, int pct, int pieces) {
+  const int64_t q_tiles = (max_q + mvllm::kPairQueryTile - 1) / mvllm::kPairQueryTile;
+  const int64_t by_seqs = static_cast<int64_t>(num_seqs) * q_tiles;
+  const int64_t by_tokens =
+      (static_cast<int64_t>(num_tokens) + mvllm::kPairQueryTile - 1) / mvllm::kPairQueryTile + num_seqs;
+  const int64_t items = by_seqs < by_tokens ? by_seqs : by_tokens;
+  const int cols = hq / 2;
+  const int64_t ranks = items + mvllm::split_extra_ranks(wgs, cols, pct);
+  if (ranks > mvllm::kSplitMaxRanks) return;
+  plan.split_pieces = pieces;
+  plan.split_ranks = static_cast<int>(ranks);
+  plan.split_slots = mvllm::split_slots(wgs, cols, pct);
+  plan.split_pct = pct;
+  plan.split_wgs = wgs;
+  plan.off_split = align256(plan.pub.workspace_bytes);
+  plan.off_rec = align256(plan.off_split + static_cast<uint64_t>(plan.split_slots) * cols *
+                                               mvllm::kPairSlotFloats * sizeof(float));
+  plan.pub.workspace_bytes = plan.off_rec + align256(static_cast<uint64_t>(ranks) * 32);
+}
+
+// The MFMA prefill's schedule, from host sizes: the grid where its 128-query items, ceil(
+// num_tokens / 128) query tiles per kv column, reach half the CU count, the stream schedule
+// (balanced shares of all key tiles) below; the prefill_schedule option 1 / 2 forces
+// stream / grid. The pair kernel runs both as its item grid or, where pair_wants_split or
+// an option says so, cut into pieces; the other kernels run the stream as one persistent
+// workgroup per CU (times the prefill_wgs_per_cu option), whose workspace follows the decode
+// part's (four 512-query chunks beside 28 decodes, 136 items: grid 102 us, stream 110 us;
+// one chunk of a long prompt, 40 items: stream 104 us, grid 109 us; 2.5-3x the grid at
+// 8K-16K contexts).
 void plan_prefill(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t hk,
-                  int32_t d, int32_t block_size, int32_t max_q, int32_t q_dtype,
+                  int32_t d, int32_t block_size, int32_t max_q, int32_t max_ctx, int32_t q_dtype,
                   int32_t kv_dtype, const Options& o) {
   if (!plan.pub.prefill_mfma) return;
   plan.register_staging = o.prefill_staging;
   plan.prefill_share_tiles = o.prefill_share_tiles;
   const int forced = o.prefill_schedule;
-  const int64_t items = static_cast<int64_t>((num_tokens + mvllm::kPrefillQueryTile - 1) /
-                                             mvllm::kPrefillQueryTile) *
-                        (hq / mvllm::prefill_item_heads(hq / hk));
-  if (num_seqs > mvllm::kMaxStreamSeqs || forced == 2 ||
-      (forced != 1 && 2 * items >= device_cus())) {
-    plan_split(plan, num_tokens, num_seqs, hq, hk, d, block_size, max_q, q_dtype, kv_dtype, o);
+  const int cus = device_cus();
+  const bool pair = pair_prefill(hq, hk, d, block_size, q_dtype, kv_dtype, o);
+  const int64_t qtiles = (static_cast<int64_t>(num_tokens) + mvllm::kPrefillQueryTile - 1) /
+                         mvllm::kPrefillQueryTile;
+  const int64_t items = qtiles * (hq / mvllm::prefill_item_heads(hq / hk));
+  if (num_seqs > mvllm::kMaxStreamSeqs || forced == 2 || (forced != 1 && 2 * items >= cus)) {
+    // The grid may cut at most kSplitMaxItems 128-query items (bounded as in plan_split).
+    const int64_t q_tiles = (max_q + mvllm::kPrefillQueryTile - 1) / mvllm::kPrefillQueryTile;
+    const int64_t by_seqs = num_seqs * q_tiles, by_tokens = qtiles + num_seqs;
+    if (pair && o.prefill_pieces > 1 && hq / 2 <= mvllm::kSplitMaxCols &&
+        (by_seqs < by_tokens ? by_seqs : by_tokens) <= mvllm::kSplitMaxItems) {
+      plan.pub.prefill_pieces = o.prefill_pieces;
+      plan_split(plan, num_tokens, num_seqs, hq, max_q, cus, o.prefill_piece_pct, o.prefill_pieces);
+      if (!o.pieces_given && !pair_wants_split(num_tokens, num_seqs, hq, max_ctx, cus)) plan.split_pieces = 0;
+    }
     return;
   }
-  int64_t wgs = static_cast<int64_t>(o.prefill_wgs_per_cu) * device_cus();
+  int64_t wgs = static_cast<int64_t>(o.prefill_wgs_per_cu) * cus;
   if (wgs > mvllm::kMaxPrefillWgs) wgs = mvllm::kMaxPrefillWgs;
   const uint64_t rows = static_cast<uint64_t>(2 * wgs) * mvllm::prefill_item_heads(hq / hk) *
                         mvllm::kPrefillQueryTile;
@@ -235,6 +271,13 @@ void plan_prefill(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, 
   plan.off_pf_o = plan.off_pf + align256(static_cast<uint64_t>(num_seqs + 1) * sizeof(int));
   plan.off_pf_ml = plan.off_pf_o + align256(rows * d * sizeof(float));
   plan.pub.workspace_bytes = plan.off_pf_ml + align256(rows * 2 * sizeof(float));
+  if (pair && (forced == 1 || pair_wants_split(num_tokens, num_seqs, hq, max_ctx, cus))) {
+    // (the stream's partial rows are not used then: the slots and records take their place)
+    const uint64_t end = plan.pub.workspace_bytes;
+    plan.pub.workspace_bytes = plan.off_pf_o;
+    plan_split(plan, num_tokens, num_seqs, hq, max_q, static_cast<int>(wgs), 100, kStreamPieces);
+    if (plan.pub.workspace_bytes < end) plan.pub.workspace_bytes = end;
+  }
 }
 
 Plan make_plan(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t hk, int32_t d,
@@ -243,7 +286,8 @@ Plan make_plan(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t hk, int
   Plan plan{};
   plan_decode(plan, num_tokens, num_seqs, hq, hk, d, block_size, max_q, max_ctx, q_dtype,
               kv_dtype, o);
-  plan_prefill(plan, num_tokens, num_seqs, hq, hk, d, block_size, max_q, q_dtype, kv_dtype, o);
+  plan_prefill(plan, num_tokens, num_seqs, hq, hk, d, block_size, max_q, max_ctx, q_dtype, kv_dtype,
+               o);
   return plan;
 }
 
@@ -313,56 +357,7 @@ void plan_decode(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, i
   }
 }
 
-// Arrival counters of the split prefill grid, in a static device array (each GPU holds
-// its own from the library's load until the process ends; it starts at zero and every
-// launch leaves its counters at zero). A stream takes one region of it on its first
-// split launch and keeps it, so launches that may overlap in time (other streams)
-// never share counters, while one stream's launches run in order. A stream beyond the
-// regions runs its prefill with every item whole, and so does a launch made while its
-// stream is being captured into a graph: the graph would carry the capture stream's
-// region in its kernel arguments, and a replay on another stream could then overlap a
-// launch still running on the capture stream over the same counters. Both cases are
-// counted (mvllm_split_stats). Host code never names the array itself: each device's
-// address comes from hipGetSymbolAddress, kept here.
-constexpr int kCounterRegions = 32;
-constexpr int kCounterInts = mvllm::kSplitMaxItems * mvllm::kSplitMaxCols;
-static __device__ __align__(256) int split_counters[kCounterRegions * kCounterInts];
-
-constexpr int kCounterDevices = 64;
-std::mutex g_counter_mutex;
-int* g_counter_base[kCounterDevices] = {};
-hipStream_t g_counter_owner[kCounterDevices][kCounterRegions] = {};
-bool g_counter_used[kCounterDevices][kCounterRegions] = {};
-std::atomic<int64_t> g_split_whole_no_region{0};   // split launches run whole: no region left
-std::atomic<int64_t> g_split_whole_capturing{0};   // split launches run whole: stream capturing
-
-// The counter region of (current device, stream), or nullptr when there is none to give.
-int* split_counters_for(hipStream_t stream) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kCounterDevices) return nullptr;
-  std::lock_guard<std::mutex> lock(g_counter_mutex);
-  if (g_counter_base[dev] == nullptr) {
-    void* ptr = nullptr;
-    if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(split_counters)) != hipSuccess || ptr == nullptr) {
-      return nullptr;
-    }
-    g_counter_base[dev] = static_cast<int*>(ptr);
-  }
-  int free_region = -1;
-  for (int r = 0; r < kCounterRegions; ++r) {
-    if (g_counter_used[dev][r] && g_counter_owner[dev][r] == stream) {
-      return g_counter_base[dev] + r * kCounterInts;
-    }
-    if (!g_counter_used[dev][r] && free_region < 0) free_region = r;
-  }
-  if (free_region < 0) {
-    g_split_whole_no_region.fetch_add(1, std::memory_order_relaxed);
-    return nullptr;
-  }
-  g_counter_used[dev][free_region] = true;
-  g_counter_owner[dev][free_region] = stream;
-  return g_counter_base[dev] + free_region * kCounterInts;
-}
+std::atomic<int64_t> g_split_whole_capturing{0};  // cut grid launches run whole: stream capturing
 
 // Fills the plan's schedule fields and workspace pointers into `p` and launches the
 // decode and prefill kernels the plan names (shared by the paged and dense entries).
@@ -375,6 +370,7 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
   p.by_row = plan.pub.decode_mode == MVLLM_DECODE_BY_ROW ? 1 : 0;
   p.pf_register_staging = plan.register_staging;
   p.pf_share_tiles = plan.prefill_share_tiles;
+  p.pf_cus = device_cus();
   if (plan.pub.workspace_bytes > 0) {
     char* ws = static_cast<char*>(workspace);
     if (plan.pub.decode_mode == MVLLM_DECODE_STREAM) p.seq_prefix = reinterpret_cast<int*>(ws);
@@ -386,23 +382,24 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
       p.pf_o = reinterpret_cast<float*>(ws + plan.off_pf_o);
       p.pf_ml = reinterpret_cast<float*>(ws + plan.off_pf_ml);
     }
-    if (plan.pub.prefill_pieces > 1) {
+    p.pf_pieces = plan.split_pieces;
+    if (plan.split_pieces > 1 && plan.pub.prefill_workgroups == 0) {
+      // The grid under graph capture runs its items whole: a graph's result does not depend
+      // on how a batch's lengths would cut them.
       hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
       if (hipStreamIsCapturing(s, &capture) != hipSuccess ||
           capture != hipStreamCaptureStatusNone) {
         g_split_whole_capturing.fetch_add(1, std::memory_order_relaxed);
-        p.pf_count = nullptr;  // items whole: a graph must not name a stream's counters
-      } else {
-        p.pf_count = split_counters_for(s);
+        p.pf_pieces = 0;
       }
-      if (p.pf_count != nullptr) {
-        p.pf_pieces = plan.pub.prefill_pieces;
-        p.pf_ranks = plan.split_ranks;
-        p.pf_slots = plan.split_slots;
-        p.pf_cus = device_cus();
-        p.pf_piece_pct = plan.split_pct;
-        p.pf_part = reinterpret_cast<float*>(ws + plan.off_split);
-      }
+    }
+    if (p.pf_pieces > 1) {
+      p.pf_ranks = plan.split_ranks;
+      p.pf_slots = plan.split_slots;
+      p.pf_piece_pct = plan.split_pct;
+      p.pf_cus = plan.split_wgs;
+      p.pf_part = reinterpret_cast<float*>(ws + plan.off_split);
+      p.pf_rec = reinterpret_cast<int4*>(ws + plan.off_rec);
     }
   }
   if (plan.pub.decode_mode != MVLLM_DECODE_NONE) {
@@ -582,14 +579,8 @@ const char* mvllm_build_id(void) { return MVLLM_SOURCE_HASH; }
 
 void mvllm_split_stats(int32_t* regions_used, int64_t* whole_no_region,
                        int64_t* whole_capturing) {
-  int dev = 0;
-  int used = 0;
-  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kCounterDevices) {
-    std::lock_guard<std::mutex> lock(g_counter_mutex);
-    for (int r = 0; r < kCounterRegions; ++r) used += g_counter_used[dev][r] ? 1 : 0;
-  }
-  if (regions_used != nullptr) *regions_used = used;
-  if (whole_no_region != nullptr) *whole_no_region = g_split_whole_no_region.load();
+  if (regions_used != nullptr) *regions_used = 0;
+  if (whole_no_region != nullptr) *whole_no_region = 0;
   if (whole_capturing != nullptr) *whole_capturing = g_split_whole_capturing.load();
 }
 

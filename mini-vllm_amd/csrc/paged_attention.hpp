@@ -40,21 +40,22 @@ __host__ __device__ inline int64_t prefill_stream_shares(int64_t total_units, in
 constexpr int kXcds = 8;
 constexpr int kPrefillKeyTile = 64;
 
-// Split grid (prefill): items longer than a piece length (a percentage of the mean work
-// per CU, kSplitDefaultPct by default) are cut into key
-// ranges ("pieces") run by workgroups of their own in one launch, longest piece first;
-// the last piece of an item to finish merges the others' (m, l, O) partials. Every
-// workgroup derives the same schedule from the sequences' sizes, one wave lane per
-// item, so the items of one call are at most kSplitMaxItems and the columns at most
-// kSplitMaxCols (the counters' extent).
+// The pair prefill kernel's items (64 query positions of two heads of a GQA group) and its
+// split schedule: items longer than a piece length (a percentage of the mean key tiles per
+// workgroup) are cut into key ranges ("pieces") run by workgroups of their own, whose (m, l,
+// O) partials a second kernel merges. Every workgroup derives the same schedule from the
+// sequences' sizes.
+constexpr int kPairQueryTile = 64;
+// Floats of one piece's partial: two heads x 64 rows x (128 of O + (m, l)).
+constexpr int kPairSlotFloats = 2 * kPairQueryTile * 130;
+// The grid plan cuts at most this many 128-query items over at most this many columns.
 constexpr int kSplitMaxItems = 64;
 constexpr int kSplitMaxCols = 64;
+constexpr int kSplitMaxRanks = 4096;
 constexpr int kSplitDefaultPieces = 8;
-// Floats of one piece's partial: 8 waves x 64 lanes x (64 of O + (m, l)).
-constexpr int kSplitSlotFloats = 8 * 64 * 66;
 constexpr int kSplitDefaultPct = 150;
-// Host bounds of the split grid over `cols` columns on `cus` CUs with pieces of at least
-// pct% of the mean work per CU: the extra pieces of one column number fewer than
+// Host bounds of the split over `cols` columns and `cus` workgroups with pieces of at least
+// pct% of the mean work per workgroup: the extra pieces of one column number fewer than
 // 100 cus / (pct cols); the partial slots of one column (every piece of a cut item
 // holds one) at most twice that.
 __host__ __device__ inline int split_extra_ranks(int cus, int cols, int pct) {
@@ -147,16 +148,15 @@ struct PagedParams {
                             // fewest key tiles per piece
   int pf_register_staging;  // 1: the register-staged prefill kernel even where the
                             // direct-to-LDS one serves (a plan option, for measurement)
-  int pf_pieces;      // split grid: > 1 cuts long items into at most this many pieces (a
+  int pf_pieces;      // pair prefill: > 1 cuts long items into at most this many pieces (a
                       // 1-D grid of pf_ranks x columns); otherwise the (column,
                       // sequence, query tile) grid with every item whole
-  int pf_ranks;       // split grid: grid extent in ranks (items + extra pieces bound)
-  int pf_slots;       // split grid: partial slots per column
-  int pf_cus;         // split grid: the device's CUs
-  int pf_piece_pct;   // split grid: piece length, percent of the mean tiles per CU
-  int* pf_count;      // split grid: [kSplitMaxItems][columns] arrival counters, zero
-                      // before the launch and left zero by it
-  float* pf_part;     // split grid: [pf_slots][columns] partials of kSplitSlotFloats
+  int pf_ranks;       // split: grid extent in ranks (items + extra pieces bound)
+  int pf_slots;       // split: partial slots per column
+  int pf_cus;         // the device's CUs; split: the workgroups the pieces are sized for
+  int pf_piece_pct;   // split: piece length, percent of the mean tiles per workgroup
+  float* pf_part;     // split: [pf_slots][columns] partials of kPairSlotFloats
+  int4* pf_rec;       // split: [pf_ranks][2], each position's piece for the merge
 };
 
 // Splits of one row: as many as its visible context needs at `split_tokens` keys

@@ -117,6 +117,15 @@ __device__ __forceinline__ u32x4 load16_untracked(const char* p) {
   return v;
 }
 
+// A 4-byte global load and its wait in one: for the rare load inside a loop whose other
+// copies the compiler does not track (a wait it placed itself, on a path that joins the
+// loop's, would drain them in every iteration).
+__device__ __forceinline__ int load_dword_now(const void* p) {
+  int v;
+  asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
+  return v;
+}
+
 // Eight consecutive pool elements -> eight 16-bit elements of the compute type.
 template <typename TQ, typename TKV> struct Stage;
 template <typename TQ> struct Stage<TQ, TQ> {
@@ -276,33 +285,6 @@ __device__ __forceinline__ bool prefill_work(const PagedParams& p, int cols, int
   return true;
 }
 
-// The split grid's piece at position `rank` (workgroup blockIdx.x / columns; the first
-// pf_ranks - (pieces) positions are empty, then the pieces in rank order), computed by one
-// wave from the sequences' sizes (no host read, no other launch; every workgroup
-// derives the same schedule). Items (sequence, query tile) are numbered sequence by
-// sequence, lane i holding item i:
-//  * piece length L = max(fewest tiles, ceil(pct% of the mean tiles per CU)); an item
-//    of nt tiles is cut into P = min(pieces, ceil(nt / L)) key ranges of floor-divided
-//    tiles (P - 1 < nt / L, so the extra pieces number fewer than 100 cus / (pct cols)
-//    and the cut items' pieces fewer than twice that: within the grid's ranks and
-//    slots; an item that would still pass them, counted with every earlier item's
-//    pieces, stays whole);
-//  * ranks go longest piece first (ties by item index), an item's pieces consecutive;
-//  * a cut item's pieces hold partial slots slot0 .. slot0 + P - 1 (prefix over the
-//    cut items in index order).
-// Scans are DPP; the all-pairs rank count reads every item's (longest piece,
-// pieces) from LDS with broadcast loads, so no step is a chain of per-item scalar reads.
-// False for an empty position (the grid is a host-side bound).
-struct SplitPiece {
-  int s, q, item, piece, pieces, slot0, tb, te;
-};
-
-struct SplitLds {
-  int4 rec[kSplitMaxItems];  // item i: (sequence, query tile, tiles, 0)
-  int2 kp[kSplitMaxItems];   // item i: (its longest piece, its pieces)
-  int out[10];               // the schedule's result for the other waves
-};
-
 // Inclusive prefix sum over the wave's 64 lanes: DPP row shifts 1, 2, 4, 8 (within
 // each 16-lane row; a lane whose source lies outside its row adds 0), then lane 15's
 // row total broadcast into rows 1 and 3 and lane 31's into rows 2 and 3.
@@ -316,113 +298,112 @@ __device__ __forceinline__ int wave_inclusive_scan(int v) {
   return v;
 }
 
-__device__ __forceinline__ bool split_piece_wave(const PagedParams& p, int cols, int rank,
-                                                 SplitLds& lds, SplitPiece& out) {
-  const int lane = threadIdx.x % kWave;
-  const int n = p.num_seqs;
-  // Items in sequence order: lane s of each 64-sequence chunk lists its query tiles.
-  // (One wave's LDS accesses complete in order, so its lanes read what others wrote.)
-  int items = 0;
-  for (int base = 0; base < n; base += kWave) {
-    int len = 0, ctx = 0;
-    if (base + lane < n) {
-      len = p.seq_lens[base + lane];
-      ctx = p.context_lens[base + lane];
-    }
-    const int qts = len > 1 ? (len + kPrefillQueryTile - 1) / kPrefillQueryTile : 0;
-    const int pre = items + wave_inclusive_scan(qts) - qts;
-    for (int q = 0; q < qts && pre + q < kSplitMaxItems; ++q) {
-      lds.rec[pre + q] = make_int4(base + lane, q, prefill_item_tiles(ctx, len, q), 0);
-    }
-    items = __builtin_amdgcn_readlane(pre + qts, kWave - 1);
-  }
-  items = min(items, kSplitMaxItems);  // the host bound rules out more
-  const bool have = lane < items;
-  const int4 r = have ? lds.rec[lane] : make_int4(0, 0, 0, 0);
-  const int nt = r.z;
-  const int total = __builtin_amdgcn_readlane(wave_inclusive_scan(nt), kWave - 1);
-  // pct percent of the mean tiles per CU, rounded up
-  const int64_t scaled = static_cast<int64_t>(p.pf_piece_pct) * total * cols;
-  int piece_len = static_cast<int>((scaled + 100 * p.pf_cus - 1) / (100 * p.pf_cus));
-  piece_len = max(piece_len, max(p.pf_share_tiles, 1));
-  int pcs = have ? max(min(p.pf_pieces, (nt + piece_len - 1) / piece_len), 1) : 0;
-  // Extra pieces (low 16 bits) and cut items' slots (high 16 bits) before this item;
-  // both stay below 64 x 64.
-  const int both = (have ? pcs - 1 : 0) | ((pcs > 1 ? pcs : 0) << 16);
-  const int before = wave_inclusive_scan(both) - both;
-  const int extra_before = before & 0xffff, slots_before = before >> 16;
-  if (pcs > 1 && (items + extra_before + pcs - 1 > p.pf_ranks || slots_before + pcs > p.pf_slots)) {
-    pcs = 1;
-  }
-  const int cut = pcs > 1 ? pcs : 0;
-  const int slot0 = wave_inclusive_scan(cut) - cut;
-  // The grid's first positions are the ranks it has beyond the pieces (empty): they
-  // end here, while every CU is still free, rather than after the last piece.
-  const int ranks = items + __builtin_amdgcn_readlane(wave_inclusive_scan(have ? pcs - 1 : 0), kWave - 1);
-  rank -= p.pf_ranks - ranks;
-  if (rank < 0) return false;
-  const int key = have ? (nt + pcs - 1) / pcs : 0;
-  lds.kp[lane] = make_int2(key, pcs);
-  // Pieces ranked before this item's first: every item's pair read with 16-byte
-  // broadcast loads, all of a half issued before any is used.
-  int start = 0;
-#pragma unroll
-  for (int h = 0; h < kSplitMaxItems; h += kSplitMaxItems / 2) {
-    int4 two[kSplitMaxItems / 4];
-#pragma unroll
-    for (int k = 0; k < kSplitMaxItems / 4; ++k) two[k] = *reinterpret_cast<const int4*>(&lds.kp[h + 2 * k]);
-#pragma unroll
-    for (int k = 0; k < kSplitMaxItems / 4; ++k) {
-      const int j = h + 2 * k;
-      if (two[k].x > key || (two[k].x == key && j < lane)) start += two[k].y;
-      if (two[k].z > key || (two[k].z == key && j + 1 < lane)) start += two[k].w;
-    }
-  }
-  const uint64_t mine = __builtin_amdgcn_ballot_w64(have && start <= rank && rank < start + pcs);
-  if (mine == 0) return false;
-  const int i = __builtin_ctzll(mine);
-  out.s = __builtin_amdgcn_readlane(r.x, i);
-  out.q = __builtin_amdgcn_readlane(r.y, i);
-  out.item = i;
-  out.pieces = __builtin_amdgcn_readlane(pcs, i);
-  out.piece = rank - __builtin_amdgcn_readlane(start, i);
-  out.slot0 = __builtin_amdgcn_readlane(slot0, i);
-  const int nti = __builtin_amdgcn_readlane(nt, i);
-  out.tb = out.piece * nti / out.pieces;
-  out.te = (out.piece + 1) * nti / out.pieces;
-  return true;
+// A piece of the pair kernel's work: key tiles [tb, te) of query tile q (of kPairQueryTile
+// positions) of sequence s, the `piece`th of the item's `pieces`, its partial in slot
+// slot0 + piece when there are several.
+struct PairPiece {
+  int s, q, piece, pieces, slot0, tb, te;
+};
+
+// Key tiles walked by an item of `qt` query positions.
+__device__ __forceinline__ int pair_item_tiles(int context, int len, int q, int qt) {
+  return (context - len + min((q + 1) * qt, len) + kTileKeys - 1) / kTileKeys;
 }
 
-// Every wave's copy of the schedule: wave 0 computes it, the workgroup's barrier
-// publishes it. False (for the whole workgroup) past the last piece.
-__device__ __forceinline__ bool split_piece(const PagedParams& p, int cols, int rank,
-                                            SplitLds& lds, SplitPiece& out) {
-  if (threadIdx.x < kWave) {
-    SplitPiece mine{};
-    const bool got = split_piece_wave(p, cols, rank, lds, mine);
-    if (threadIdx.x == 0) {
-      lds.out[0] = got ? 1 : 0;
-      lds.out[1] = mine.s;
-      lds.out[2] = mine.q;
-      lds.out[3] = mine.item;
-      lds.out[4] = mine.piece;
-      lds.out[5] = mine.pieces;
-      lds.out[6] = mine.slot0;
-      lds.out[7] = mine.tb;
-      lds.out[8] = mine.te;
-    }
+// The piece at position `rank` of the split schedule, computed by every wave for itself
+// from the sequences' sizes (no host read of device data, no launch before, no barrier).
+// The piece length is pct% of the mean key tiles per CU, at least pf_share_tiles; an item
+// of nt tiles is cut into P = min(pf_pieces, ceil(nt / length)) equal key ranges. P - 1 <
+// nt / length, so the pieces beyond one an item number fewer than 100 cus / (pct cols) and
+// the cut items' pieces fewer than twice that: the grid's extra ranks and the partial
+// slots. The positions past the last piece end here; they come last, so that the pieces
+// are dealt to empty CUs one each (first, they left some CUs two pieces and others none: a
+// 512-token chunk after 8000 keys 60 us against 57). Lane l holds sequence 64 i + l of the i-th chunk.
+__device__ __forceinline__ bool pair_piece(const PagedParams& p, int cols, int rank,
+                                           PairPiece& out) {
+  const int lane = threadIdx.x % kWave;
+  const int n = p.num_seqs;
+  int total = 0, items = 0;
+  int len = 0, ctx = 0, qts = 0;
+  auto load = [&](int base) __attribute__((always_inline)) {  // sequence base + lane
+    len = base + lane < n ? p.seq_lens[base + lane] : 0;
+    ctx = base + lane < n ? p.context_lens[base + lane] : 0;
+    qts = len > 1 ? (len + kPairQueryTile - 1) / kPairQueryTile : 0;
+  };
+  auto wave_total = [&](int v) __attribute__((always_inline)) -> int {
+    return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1);
+  };
+  for (int base = 0; base < n; base += kWave) {
+    load(base);
+    int tiles = 0;
+    for (int q = 0; q < qts; ++q) tiles += pair_item_tiles(ctx, len, q, kPairQueryTile);
+    total += wave_total(tiles);
+    items += wave_total(qts);
   }
-  __syncthreads();
-  if (__builtin_amdgcn_readfirstlane(lds.out[0]) == 0) return false;
-  out.s = __builtin_amdgcn_readfirstlane(lds.out[1]);
-  out.q = __builtin_amdgcn_readfirstlane(lds.out[2]);
-  out.item = __builtin_amdgcn_readfirstlane(lds.out[3]);
-  out.piece = __builtin_amdgcn_readfirstlane(lds.out[4]);
-  out.pieces = __builtin_amdgcn_readfirstlane(lds.out[5]);
-  out.slot0 = __builtin_amdgcn_readfirstlane(lds.out[6]);
-  out.tb = __builtin_amdgcn_readfirstlane(lds.out[7]);
-  out.te = __builtin_amdgcn_readfirstlane(lds.out[8]);
-  return true;
+  const int64_t scaled = static_cast<int64_t>(p.pf_piece_pct) * total * cols;
+  int length = static_cast<int>((scaled + 100 * p.pf_cus - 1) / (100 * p.pf_cus));
+  length = max(length, max(p.pf_share_tiles, 1));
+  auto pieces_of = [&](int nt) __attribute__((always_inline)) -> int {
+    return min(p.pf_pieces, (nt + length - 1) / length);
+  };
+  // Pieces (low half) and cut items' slots (high half; both below 2^15) of a sequence.
+  auto count = [&]() __attribute__((always_inline)) -> int {
+    int both = 0;
+    for (int q = 0; q < qts; ++q) {
+      const int pcs = pieces_of(pair_item_tiles(ctx, len, q, kPairQueryTile));
+      both += pcs | (pcs > 1 ? pcs << 16 : 0);
+    }
+    return both;
+  };
+  // Every piece at once: rounding each item's pieces up may pass the CUs by a few, whose two
+  // workgroups then take twice as long as the others (one 512-token chunk after 8000 keys,
+  // 272 pieces on 256 CUs: 68 us, 256 60 us), so the length grows until they fit.
+  int ranks = 0;
+  for (int i = 0; i < 12; ++i) {
+    ranks = 0;
+    for (int base = 0; base < n; base += kWave) {
+      if (n > kWave) load(base);
+      ranks += wave_total(count() & 0xffff);
+    }
+    if (ranks * cols <= p.pf_cus || ranks <= items || 2 * items * cols > p.pf_cus) break;
+    length += (length + 15) / 16;
+  }
+  if (rank >= ranks) return false;
+  int before = 0, slots = 0;
+  for (int base = 0; base < n; base += kWave) {
+    if (n > kWave) load(base);
+    const int both = count();
+    const int incl = wave_inclusive_scan(both);
+    const int all = __builtin_amdgcn_readlane(incl, kWave - 1);
+    const int first = before + ((incl - both) & 0xffff);
+    const uint64_t mine =
+        __builtin_amdgcn_ballot_w64(rank >= first && rank < first + (both & 0xffff));
+    if (mine != 0) {
+      const int i = __builtin_ctzll(mine);
+      const int len_i = __builtin_amdgcn_readlane(len, i), ctx_i = __builtin_amdgcn_readlane(ctx, i);
+      int r = rank - __builtin_amdgcn_readlane(first, i);
+      out.slot0 = slots + (__builtin_amdgcn_readlane(incl - both, i) >> 16);
+      out.s = base + i;
+      for (out.q = 0;; ++out.q) {
+        const int nt = pair_item_tiles(ctx_i, len_i, out.q, kPairQueryTile);
+        out.pieces = pieces_of(nt);
+        if (r < out.pieces) {
+          out.piece = r;
+          out.tb = r * nt / out.pieces;
+          out.te = (r + 1) * nt / out.pieces;
+          break;
+        }
+        r -= out.pieces;
+        if (out.pieces > 1) out.slot0 += out.pieces;
+      }
+      // (the bounds above rule this out; a slot is never written past the workspace)
+      if (out.pieces > 1 && out.slot0 + out.pieces > p.pf_slots) return false;
+      return true;
+    }
+    before += all & 0xffff;
+    slots += all >> 16;
+  }
+  return false;
 }
 
 }  // namespace
@@ -1231,74 +1212,61 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// The grid schedule's kernel for 16-bit pools at D = 128, a GQA pair per work item and
-// pages of >= 16 keys, software pipelined: the scores of tile t + 1 are computed
-// (S^T = K Q^T) while the softmax of tile t runs, so one wave keeps its MFMAs and its
-// vector work in flight together instead of alternating between them (with the two
-// waves of a SIMD meeting at every tile's barrier, both used to reach their softmax at
-// the same time and leave the matrix core idle). Per tile t, in order:
-//   wait for this wave's copies of tile t + 1; barrier (tile t + 1's K and raw V rows,
-//   and every wave's V^T rows of tile t, are then visible, and every wave is done with
-//   tile t - 1); transpose this wave's V rows of tile t + 1 into V^T buffer (t + 1) & 1;
-//   stage tile t + 3 into the slots tile t used (K read by S(t) one step earlier);
-//   S(t + 1) = K(t + 1) Q^T  ||  softmax of S(t) -> P(t);
-//   O^T += V^T(t) P^T(t)  ||  the rest of P(t), then the row maxima of S(t + 1).
-// (The maxima used to open the next step, ahead of its first MFMA, with a trip through LDS
-// for the other half's: under the last MFMAs and with a permlane swap instead, and one
-// packed conversion per pair of float16 probabilities, a 2048-token float16 chunk after
-// 14336 keys, 32 heads, went from 577 to 541 us, eight 512-token bf16 chunks from 61.1 to
-// 59.6 us.)
-// Staging maps and the softmax are those of paged_prefill_lds_kernel, except that K
-// rows are swizzled over 16 chunks (key & 15) instead of 8; K/V slots rotate by three and the score accumulators by two, so the loop is unrolled by
-// six with every buffer named at compile time.
-template <typename TQ, typename TKV, bool kSplit>
-__global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedParams p) {
+// The kernel of GQA pairs at D = 128 (pages of >= 16 keys, a positive scale, 16-bit and fp8
+// pools): a work item is kWaves * 16 query positions of two heads against one kv head, one
+// wave per (head, 32 positions).
+//
+// What bounds it: per wave and 64-key tile 32 MFMAs (1024 matrix cycles), ~130 vector
+// instructions of softmax (32 of them v_exp_f32), and 32 KB of K/V fragments from LDS, no two
+// of which overlap fully with the in-order issue of one or two waves per SIMD. Measured with
+// two waves per SIMD: 13.9 ns an MFMA alone, 15.6 beside the softmax's instructions, 16.2
+// beside its LDS reads, 22.5 beside both; the kernel runs at 28 without and 32 with the
+// copies of its tiles.
+//
+// Why this layout:
+//  * workgroups of four waves and 64 KB of LDS, two to a CU, not one of eight: twice the items
+//    (a 512-token chunk is 64 of them, not 32), one workgroup's waits, barriers, prologue
+//    and epilogue run beside the other's MFMAs, and four waves meet at a barrier
+//    instead of eight. Against the eight-wave kernel it replaced, which kept three staged tiles
+//    and a transposed copy of V in 128 KB: 8 x 512 tokens after up to 1536 keys 59.6 -> 52
+//    us, 4 x 512 after 1000 62 -> 33, one fresh 512-token chunk 35 -> 15, one fresh 2048-token
+//    chunk 60 -> 38, 2048 float16 tokens after 14336, 32 heads, 541 -> 510.
+//  * V is read transposed out of its row-major tile by ds_read_b64_tr_b16: no transposed copy
+//    (LDS for the second workgroup) and none of its permutes and writes per tile.
+//  * software pipelined: S(t + 1) = K(t + 1) Q^T is computed while the softmax of tile t
+//    runs, so a wave keeps MFMAs and vector work in flight together. Per tile t: wait for
+//    this wave's copies, barrier (K(t + 1) and V(t) visible, the slots of K(t) and V(t - 1)
+//    free); request V(t + 1) and K(t + 2); S(t + 1) || first half of P(t); O^T += V^T(t) P^T(t)
+//    || the rest of P(t), then the row maxima of S(t + 1). Two slots each of K and V and two
+//    of scores, the loop unrolled by two with every buffer named at compile time.
+//  * tried, no faster: copies with a step and a half to land (a second barrier per tile), six
+//    fragments read ahead, a raised wave priority in the MFMA phases.
+//  * fp8 pools: each wave's own rows are staged as codes and converted, times the page's
+//    scale, into the same buffers before the barrier.
+template <typename TQ, typename TKV, int kWaves, bool kSplit>
+__global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(const PagedParams p) {
   constexpr bool kFp8 = std::is_same_v<TKV, fp8_t>;
   constexpr int D = 128;
-  constexpr int kWaves = 8;
-  constexpr int HW = 2;                   // query heads per work item, one per wave set
-  constexpr int KW = kTileKeys / kWaves;  // keys of a tile staged by one wave
-  constexpr int kRawRow = kFp8 ? D : D * 2;  // bytes of one staged pool row
-  constexpr int kRowLanes = kRawRow / 16;    // lanes per staged row (16 bytes each)
-  constexpr int kCopies = KW * kRowLanes / kWave;  // direct loads per wave per tile (K and V each)
-  constexpr int KV = 2;                   // V keys per lane in the transpose
+  constexpr int QT = kWaves * 16;            // query positions: kWaves / 2 waves of 32 per head
+  constexpr int KW = kTileKeys / kWaves;     // keys of a tile staged by one wave
+  constexpr int kRawRow = kFp8 ? D : D * 2;  // bytes of one pool row
+  constexpr int kRowLanes = kRawRow / 16;
+  constexpr int kKeysPerCopy = kWave / kRowLanes;
+  constexpr int kCopies = KW / kKeysPerCopy;  // direct loads per wave per tile (K and V each)
   constexpr int kKSteps = D / 16;
   constexpr int kDBlocks = D / 32;
   constexpr int kRow = D * 2;
   constexpr int kTileBytes = kTileKeys * kRow;
-  constexpr int kRawTileBytes = kTileKeys * kRawRow;
-  constexpr int kVRow = kTileKeys * 2;
-  constexpr int kStageOps = 2 * kCopies;  // vector-memory ops of one tile's stage per lane
-  static_assert(KW == 8 && kTileKeys == 64 && 32 * 4 == kPrefillQueryTile, "tile sizes");
+  static_assert(KW <= 16 && kCopies >= 1, "a wave's keys lie in one page");
 
-  // Staging slots (raw pool rows: K and V of three tiles), the 16-bit K the MFMAs read
-  // (for 16-bit pools the staged K itself; for fp8 pools a converted copy, two tiles)
-  // and V^T (two tiles).
-  __shared__ __align__(16) char k_lds0[kRawTileBytes];
-  __shared__ __align__(16) char k_lds1[kRawTileBytes];
-  __shared__ __align__(16) char k_lds2[kRawTileBytes];
-  __shared__ __align__(16) char r_lds0[kRawTileBytes];
-  __shared__ __align__(16) char r_lds1[kRawTileBytes];
-  __shared__ __align__(16) char r_lds2[kRawTileBytes];
-  __shared__ __align__(16) char kc_lds0[kFp8 ? kTileBytes : 16];  // converted K, even tiles
-  __shared__ __align__(16) char kc_lds1[kFp8 ? kTileBytes : 16];  // converted K, odd tiles
-  __shared__ __align__(1024) char v_lds0[kTileBytes];  // V^T of even tiles
-  __shared__ __align__(1024) char v_lds1[kTileBytes];  // V^T of odd tiles
-  auto k_arr = [&](auto slot) __attribute__((always_inline)) -> char* {
-    constexpr int X = decltype(slot)::value;
-    if constexpr (X == 0) return k_lds0; else if constexpr (X == 1) return k_lds1; else return k_lds2;
-  };
-  // The K the MFMAs of tile t read: staging slot t % 3, or converted buffer t & 1.
-  auto kmma_arr = [&](auto slot, auto par) __attribute__((always_inline)) -> char* {
-    if constexpr (kFp8) {
-      if constexpr (decltype(par)::value == 0) return kc_lds0; else return kc_lds1;
-    } else {
-      return k_arr(slot);
-    }
-  };
-  auto r_arr = [&](auto slot) __attribute__((always_inline)) -> char* {
-    constexpr int X = decltype(slot)::value;
-    if constexpr (X == 0) return r_lds0; else if constexpr (X == 1) return r_lds1; else return r_lds2;
+  __shared__ __align__(1024) char k_lds0[kTileBytes];
+  __shared__ __align__(1024) char k_lds1[kTileBytes];
+  __shared__ __align__(1024) char v_lds0[kTileBytes];
+  __shared__ __align__(1024) char v_lds1[kTileBytes];
+  __shared__ __align__(16) char k_raw[kFp8 ? kTileKeys * D : 16];
+  __shared__ __align__(16) char v_raw[kFp8 ? kTileKeys * D : 16];
+  auto k_arr = [&](auto par) __attribute__((always_inline)) -> char* {
+    if constexpr (decltype(par)::value == 0) return k_lds0; else return k_lds1;
   };
   auto v_arr = [&](auto par) __attribute__((always_inline)) -> char* {
     if constexpr (decltype(par)::value == 0) return v_lds0; else return v_lds1;
@@ -1309,23 +1277,29 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
   const int lane = tid % kWave;
   const int l32 = lane & 31;
   const int hsel = lane >> 5;
-  const int hs = wave / 4;  // head of the pair
-  const int wq = wave % 4;  // 32-position query block
+  const int hs = wave / (kWaves / 2);  // head of the pair
+  const int wq = wave % (kWaves / 2);  // 32-position query block
 
-  // ---- the work item: (sequence, column, query tile) and the key tiles [tb, te) of
-  // it this workgroup walks. Item grid: sequence blockIdx.y, column blockIdx.x, query
-  // tiles dispatched longest first, every item whole. Split grid: the piece of rank
-  // blockIdx.x / columns (split_piece), column blockIdx.x % columns, so one XCD keeps
-  // the same columns (and their K/V) as in the item grid.
   const int group = p.hq / p.hk;
-  const int chunks = group / HW;
+  const int chunks = group / 2;
+  // ---- the work item: (sequence, column, query tile) and its key tiles [tb, te). Item
+  // grid: sequence blockIdx.y, column blockIdx.x, query tiles dispatched longest first.
+  // Split: the piece at position blockIdx.x / columns, column blockIdx.x % columns. Either
+  // way one XCD keeps the same kv heads (their K/V in its L2).
   int s, qt, c, tb, te;
-  SplitPiece piece{};
+  PairPiece piece{};
   if constexpr (kSplit) {
+    static_assert(kWaves * 16 == kPairQueryTile, "the split schedule's query tile");
     const int cols = p.hk * chunks;
     c = static_cast<int>(blockIdx.x) % cols;
-    __shared__ SplitLds split_lds;
-    if (!split_piece(p, cols, static_cast<int>(blockIdx.x) / cols, split_lds, piece)) return;
+    const int rank = static_cast<int>(blockIdx.x) / cols;
+    const bool got = pair_piece(p, cols, rank, piece);
+    if (c == 0 && tid == 0) {  // what the merge needs to know of this position
+      p.pf_rec[2 * rank] = got ? make_int4(piece.s, piece.q, piece.piece, piece.pieces)
+                               : make_int4(0, 0, 0, 0);
+      p.pf_rec[2 * rank + 1] = make_int4(piece.slot0, 0, 0, 0);
+    }
+    if (!got) return;
     s = uniform(piece.s);
     qt = uniform(piece.q);
     tb = uniform(piece.tb);
@@ -1339,10 +1313,9 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
   const int context = sload(p.context_lens + s);
   if constexpr (!kSplit) {
     if (len <= 1) return;  // a decode row: the decode kernel has it
-    const int qtiles = (len + kPrefillQueryTile - 1) / kPrefillQueryTile;
-    if (qt >= qtiles) return;
+    if (qt * QT >= len) return;
     tb = 0;
-    te = prefill_item_tiles(context, len, qt);
+    te = pair_item_tiles(context, len, qt, QT);
   }
   const int kvh = c / chunks;
 
@@ -1356,7 +1329,7 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
 
   // ---- this wave's rows: one head, 32 query positions.
   const int offset = context - len;
-  const int w_first = qt * kPrefillQueryTile + 32 * wq;
+  const int w_first = qt * QT + 32 * wq;
   const bool w_active = w_first < len;
   const int w_kv_end = offset + min(w_first + 32, len);  // keys its last query sees
   const int w_kv_full = offset + w_first + 1;            // keys all its queries see
@@ -1365,126 +1338,112 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
   const bool my_valid = my_local < len;
   const int my_visible = offset + my_local + 1;
   const int row_base = sload(p.cu_seqlens_q + s);
-  const int head0 = (c / chunks) * group + (c % chunks) * HW + hs;
+  const int head0 = kvh * group + (c % chunks) * 2 + hs;
 
-  // ---- per-lane constants of the staging and fragment maps (as paged_prefill_lds_kernel).
-  // Copy j of a wave's keys: lane -> key kRowLanes-lane row (64 / kRowLanes) j + lane /
-  // kRowLanes, 16-byte chunk lane % kRowLanes.
-  constexpr int kKeysPerCopy = kWave / kRowLanes;
-  uint32_t k_src_off[kCopies], v_src_off[kCopies], k_src_chunk[kCopies];
+  // ---- staging map: copy j of a wave's keys: lane -> key kKeysPerCopy j + lane /
+  // kRowLanes, 16-byte chunk lane % kRowLanes. 16-bit rows are swizzled through the source
+  // address: chunk c of K row r at chunk c ^ (r & 15), of V row r at chunk c ^ 4 (r & 3).
+  uint32_t k_src_off[kCopies], v_src_off[kCopies];
+  uint32_t k_src_chunk[kCopies], v_src_chunk;
 #pragma unroll
   for (int j = 0; j < kCopies; ++j) {
-    const int key = kKeysPerCopy * j + lane / kRowLanes;  // wave-local
-    if constexpr (kFp8) {
-      // raw rows as they are; the conversion places the chunks
-      k_src_chunk[j] = (lane % kRowLanes) * 16;
-    } else {
-      // K rows: chunk c of key r at chunk c ^ (r & 15), so the 16 lanes of a fragment
-      // read that one LDS cycle serves (16 keys, one chunk) fall in distinct banks.
-      k_src_chunk[j] = (((lane & 15) ^ ((KW * wave + key) & 15)) * 16);
-    }
-    k_src_off[j] = static_cast<uint32_t>(key) * row_bytes + k_src_chunk[j];
-    v_src_off[j] = static_cast<uint32_t>(key) * row_bytes + (lane % kRowLanes) * 16;
+    const int key = KW * wave + kKeysPerCopy * j + lane / kRowLanes;  // of the tile
+    const int chunk = lane % kRowLanes;
+    k_src_chunk[j] = static_cast<uint32_t>(kFp8 ? chunk : chunk ^ (key & 15)) * 16;
+    v_src_chunk = static_cast<uint32_t>(kFp8 ? chunk : chunk ^ (4 * (key & 3))) * 16;
+    k_src_off[j] = static_cast<uint32_t>(key - KW * wave) * row_bytes + k_src_chunk[j];
+    v_src_off[j] = static_cast<uint32_t>(key - KW * wave) * row_bytes + v_src_chunk;
   }
-  const int v_chunk = lane & 15;
-  const int v_key = KW * wave + KV * (lane >> 4);
-  const int vt_chunk = (2 * (v_key >> 4) + ((v_key >> 2) & 1)) ^ (v_chunk & 7);
-  const uint32_t vt_dst = static_cast<uint32_t>(8 * v_chunk * kVRow + (4 * ((v_key >> 3) & 1) + (v_key & 3)) * 2);
+  // ---- fragment maps. K: lane l32 reads key l32 (+ 32), chunk 2 ks + hsel. V: a 16-lane
+  // group reads four keys x 16 dims with ds_read_b64_tr_b16 (lane L of it the four dims 4
+  // (L % 4) of key L / 4) and gets, in lane L, dim L of the four keys: two such reads are
+  // the MFMA's A operand (dim l32, eight keys in the P^T operand's order).
   uint32_t k_rd[kKSteps];
 #pragma unroll
   for (int ks = 0; ks < kKSteps; ++ks) k_rd[ks] = l32 * kRow + (((2 * ks + hsel) ^ (l32 & 15)) * 16);
-  uint32_t v_rd[2][4];
-  {
-    const int f0 = (l32 ^ (l32 >> 3)) & 7;
+  // (32 lanes, four keys x 64 bytes, are read together: the swizzle gives the keys
+  // different 64-byte quarters of the banks.)
+  uint32_t v_rd[kDBlocks];
 #pragma unroll
-    for (int par = 0; par < 2; ++par) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) v_rd[par][ks] = l32 * kVRow + ((((2 * ks + hsel) ^ f0 ^ (4 * par)) & 7) * 16);
-    }
+  for (int db = 0; db < kDBlocks; ++db) {
+    const int L = lane & 15, dhalf = (lane >> 4) & 1;
+    v_rd[db] = (4 * hsel + L / 4) * kRow + ((4 * (db ^ (L / 4)) + 2 * dhalf + (L & 3) / 2) * 16) +
+               (L & 1) * 8;
   }
 
-  // Page id of this wave's keys of tile t (past the last tile: the last tile again).
-  auto page_of = [&](int t) __attribute__((always_inline)) -> int {
-    const int key0 = min(min(t, te - 1) * kTileKeys + KW * wave, context - 1);
-    return sload(table + (key0 >> p.block_shift));
+  // Page ids of this wave's keys, a block of 64 tiles at a time: lane l holds tile
+  // 64 block + l's (past the last tile: the last tile's), and for fp8 pools that page's
+  // scales. One load and its latency (about 1 us) per 64 tiles; a scalar load per tile
+  // instead would be waited for with the first K fragments of every tile (it may return out
+  // of order with LDS reads, so the counter they share has to reach zero).
+  int pages = 0;
+  float ks_lane = 0.0f, vs_lane = 0.0f;
+  auto take_pages = [&](int t) __attribute__((always_inline)) {  // of the block holding tile t
+    const int tile = min((t & -kWave) + lane, te - 1);
+    pages = load_dword_now(table + (min(tile * kTileKeys + KW * wave, context - 1) >> p.block_shift));
+    if constexpr (kFp8) {
+      const int64_t si = static_cast<int64_t>(pages) * p.hk + kvh;
+      ks_lane = __int_as_float(load_dword_now(p.k_scales + si));
+      vs_lane = __int_as_float(load_dword_now(p.v_scales + si));
+    }
   };
-  // fp8 pools: the page's K and V scales of each staged slot (the wave's keys share a
-  // page), loaded with the page id.
-  float ks[3] = {0.0f, 0.0f, 0.0f}, vs[3] = {0.0f, 0.0f, 0.0f};
-  auto stage = [&](int t, int page, auto slot) __attribute__((always_inline)) {
-    constexpr int X = decltype(slot)::value;
+  auto page_of = [&](int t) __attribute__((always_inline)) -> int {
+    return __builtin_amdgcn_readlane(pages, t & (kWave - 1));
+  };
+  auto lane_scale = [&](float scales, int t) __attribute__((always_inline)) -> float {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(scales), t & (kWave - 1)));
+  };
+  auto stage = [&](int t, int page, const char* pool, char* dst_arr, const uint32_t (&src_off)[kCopies],
+                   auto chunk_of) __attribute__((always_inline)) {
     t = min(t, te - 1);
-    const uint32_t kdst = lds_address(k_arr(slot) + KW * wave * kRawRow);
-    const uint32_t rdst = lds_address(r_arr(slot) + KW * wave * kRawRow);
+    const uint32_t dst = lds_address(dst_arr + KW * wave * kRawRow);
     const int key0 = t * kTileKeys + KW * wave;
     const int last = context - 1;
     const uint64_t head = static_cast<uint64_t>(static_cast<uint32_t>(page)) * page_bytes + head_off;
-    if constexpr (kFp8) {
-      const int64_t si = static_cast<int64_t>(page) * p.hk + kvh;
-      ks[X] = __int_as_float(sload(reinterpret_cast<const int32_t*>(p.k_scales + si)));
-      vs[X] = __int_as_float(sload(reinterpret_cast<const int32_t*>(p.v_scales + si)));
-    }
     if (key0 + KW - 1 <= last) {
       const uint64_t base = head + static_cast<uint32_t>(key0 & p.block_mask) * row_bytes;
 #pragma unroll
-      for (int j = 0; j < kCopies; ++j) {
-        copy_to_lds(kpool + base, k_src_off[j], kdst + kKeysPerCopy * j * kRawRow);
-        copy_to_lds(vpool + base, v_src_off[j], rdst + kKeysPerCopy * j * kRawRow);
-      }
+      for (int j = 0; j < kCopies; ++j) copy_to_lds(pool + base, src_off[j], dst + 1024 * j);
     } else {
 #pragma unroll
       for (int j = 0; j < kCopies; ++j) {
         const uint32_t row = static_cast<uint32_t>(min(key0 + kKeysPerCopy * j + lane / kRowLanes, last) &
                                                    p.block_mask) * row_bytes;
-        copy_to_lds(kpool + head, row + k_src_chunk[j], kdst + kKeysPerCopy * j * kRawRow);
-        copy_to_lds(vpool + head, row + (lane % kRowLanes) * 16, rdst + kKeysPerCopy * j * kRawRow);
+        copy_to_lds(pool + head, row + chunk_of(j), dst + 1024 * j);
       }
     }
   };
-  // fp8 pools: eight codes of a raw row -> eight 16-bit elements times the page scale.
-  auto dequant8 = [&](const u32x2& w, float scale) __attribute__((always_inline)) -> u32x4 {
-    u32x4 out;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[i]), false);
-      const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[i]), true);
-      out[2 * i] = Mma<TQ>::pack2(lo[0] * scale, lo[1] * scale);
-      out[2 * i + 1] = Mma<TQ>::pack2(hi[0] * scale, hi[1] * scale);
-    }
-    return out;
+  auto stage_k = [&](int t, int page, auto par) __attribute__((always_inline)) {
+    stage(t, page, kpool, kFp8 ? k_raw : k_arr(par), k_src_off,
+          [&](int j) __attribute__((always_inline)) { return k_src_chunk[j]; });
   };
-  // fp8 pools: this wave's staged K rows of slot `slot` (tile-local keys KW * wave ..
-  // +7, each lane 16 codes of one row) -> converted K buffer `par`, in the swizzled
-  // layout the fragment reads use (logical chunk c of key r at chunk c ^ (r & 15)).
+  auto stage_v = [&](int t, int page, auto par) __attribute__((always_inline)) {
+    stage(t, page, vpool, kFp8 ? v_raw : v_arr(par), v_src_off,
+          [&](int) __attribute__((always_inline)) { return v_src_chunk; });
+  };
+  // fp8 pools: this wave's staged rows (each lane 16 codes of a row, two rows) times the
+  // page's scale, rounded to TQ, into the buffer the MFMAs read, swizzled as above.
   typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-  auto convert_k = [&](auto slot, auto par) __attribute__((always_inline)) {
-    constexpr int X = decltype(slot)::value;
-    const int key = KW * wave + lane / kRowLanes;
-    const int c = 2 * (lane % kRowLanes);
-    const u32x4 w = *reinterpret_cast<const u32x4*>(k_arr(slot) + key * kRawRow + (lane % kRowLanes) * 16);
-    const uint32_t dst = lds_address(kmma_arr(slot, par) + key * kRow);
-    *reinterpret_cast<lds_u32x4*>(dst + ((c ^ (key & 15)) * 16)) = dequant8(u32x2{w[0], w[1]}, ks[X]);
-    *reinterpret_cast<lds_u32x4*>(dst + (((c + 1) ^ (key & 15)) * 16)) = dequant8(u32x2{w[2], w[3]}, ks[X]);
-  };
-  typedef __attribute__((address_space(3))) uint32_t lds_u32;
-  auto store_v = [&](auto slot, auto par) __attribute__((always_inline)) {
-    constexpr int X = decltype(slot)::value;
-    u32x4 vr[KV];
-    if constexpr (kFp8) {
-      const char* raw = r_arr(slot) + v_key * kRawRow + v_chunk * 8;
+  auto convert = [&](const char* raw, char* dst_arr, float scale, bool is_k) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < KV; ++j) vr[j] = dequant8(*reinterpret_cast<const u32x2*>(raw + j * kRawRow), vs[X]);
-    } else {
-      const char* raw = r_arr(slot) + v_key * kRow + v_chunk * 16;
+    for (int j = 0; j < kCopies; ++j) {
+      const int key = KW * wave + kKeysPerCopy * j + lane / kRowLanes;
+      const int ch = 2 * (lane % kRowLanes);
+      const u32x4 w = *reinterpret_cast<const u32x4*>(raw + key * kRawRow + (lane % kRowLanes) * 16);
+      const uint32_t dst = lds_address(dst_arr + key * kRow);
+      const int f = is_k ? key & 15 : 4 * (key & 3);
 #pragma unroll
-      for (int j = 0; j < KV; ++j) vr[j] = *reinterpret_cast<const u32x4*>(raw + j * kRow);
-    }
-    const uint32_t row0 = lds_address(v_arr(par)) + vt_dst + (vt_chunk & 7) * 16;
+      for (int h = 0; h < 2; ++h) {
+        u32x4 out;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t sel = (e & 1) == 0 ? 0x05040100u : 0x07060302u;
-      const uint32_t addr = (row0 ^ (e * 16)) + e * kVRow;
-      *reinterpret_cast<lds_u32*>(addr) = __builtin_amdgcn_perm(vr[1][e >> 1], vr[0][e >> 1], sel);
+        for (int i = 0; i < 2; ++i) {
+          const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[2 * h + i]), false);
+          const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[2 * h + i]), true);
+          out[2 * i] = Mma<TQ>::pack2(lo[0] * scale, lo[1] * scale);
+          out[2 * i + 1] = Mma<TQ>::pack2(hi[0] * scale, hi[1] * scale);
+        }
+        *reinterpret_cast<lds_u32x4*>(dst + ((ch + h) ^ f) * 16) = out;
+      }
     }
   };
 
@@ -1503,26 +1462,26 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
   float m_run = -INFINITY, l_run = 0.0f;
   f32x16 sc0[2], sc1[2];  // scores of even / odd tiles
 
-  // S(t) = K(t) Q^T from K slot `slot`, fragments read four MFMAs ahead.
-  auto qk = [&](auto slot, auto kpar, f32x16 (&sc)[2]) __attribute__((always_inline)) {
-    constexpr int kLook = 4;
-    const char* kt = kmma_arr(slot, kpar);
-    auto k_frag = [&](int i) __attribute__((always_inline)) {
-      return *reinterpret_cast<const u32x4*>(kt + (i & 1) * 32 * kRow + k_rd[i >> 1]);
-    };
+  // Fragment i of the K in buffer `par`: keys 32 (i % 2) .., dims 16 (i / 2) ..; fragments are
+  // read kLook MFMAs ahead of their own.
+  constexpr int kLook = 4;
+  auto k_frag = [&](auto par, int i) __attribute__((always_inline)) {
+    return *reinterpret_cast<const u32x4*>(k_arr(par) + (i & 1) * 32 * kRow + k_rd[i >> 1]);
+  };
+  // S(t) = K(t) Q^T.
+  auto qk = [&](auto par, f32x16 (&sc)[2]) __attribute__((always_inline)) {
     sc[0] = f32x16{};
     sc[1] = f32x16{};
     u32x4 fa[kLook];
 #pragma unroll
-    for (int i = 0; i < kLook; ++i) fa[i] = k_frag(i);
+    for (int i = 0; i < kLook; ++i) fa[i] = k_frag(par, i);
 #pragma unroll
     for (int i = 0; i < 2 * kKSteps; ++i) {
       const u32x4 a = fa[i % kLook];
-      if (i + kLook < 2 * kKSteps) fa[i % kLook] = k_frag(i + kLook);
+      if (i + kLook < 2 * kKSteps) fa[i % kLook] = k_frag(par, i + kLook);
       sc[i & 1] = Mma<TQ>::run(a, qop[i >> 1], sc[i & 1]);
     }
   };
-  // Causal mask of tile t's scores (tiles crossing this wave's diagonal only).
   auto mask = [&](int t, f32x16 (&sc)[2]) __attribute__((always_inline)) {
     const int key0 = t * kTileKeys;
     if (key0 + kTileKeys > w_kv_full) {
@@ -1536,7 +1495,6 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
       }
     }
   };
-  // This lane's largest score of a tile (its 32 keys of the query's 64).
   auto lane_max = [&](const f32x16 (&sc)[2]) __attribute__((always_inline)) -> float {
     float tmax = -INFINITY;
 #pragma unroll
@@ -1546,8 +1504,6 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
     }
     return tmax;
   };
-  // Running max of the scores (raised to a tile's max only past the slack, O and l rescaled
-  // with it); returns -max in log2 units, the exponent's offset.
   auto raise_max = [&](float raw) __attribute__((always_inline)) -> float {
     const float tmax = raw * score_c;
     if (__builtin_amdgcn_ballot_w64(tmax > m_run + kRescaleSlack) != 0) {
@@ -1560,8 +1516,6 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
     }
     return m_run == -INFINITY ? 0.0f : -m_run;
   };
-  // Score element r of key block kb -> probability: exp2(s * c - max), summed into
-  // ps[r % 4] and packed in pairs into the P^T operand pop[2 kb + r / 8].
   auto prob = [&](const f32x16 (&sc)[2], int kb, int r, float neg_mu, float (&pf)[2][16],
                   float (&ps)[4]) __attribute__((always_inline)) {
     pf[kb][r] = __builtin_amdgcn_exp2f(fmaf(sc[kb][r], score_c, neg_mu));
@@ -1573,30 +1527,20 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
                                Mma<TQ>::pack2(v[4], v[5]), Mma<TQ>::pack2(v[6], v[7])};
   };
   constexpr int kMfma = 0x008, kDsRead = 0x100, kVec = 0x002 | 0x400;  // VALU and TRANS
-  // Phase A of tile t: S(t + 1) = K(t + 1) Q^T from K slot `slot`, each MFMA paired with
-  // one K fragment read (four ahead) and one probability of key block 0 of tile t.
-  auto phase_a = [&](auto slot, auto kpar, f32x16 (&nxt)[2], const f32x16 (&cur)[2], float neg_mu,
-                     float (&pf)[2][16], float (&ps)[4], u32x4 (&pop)[4]) __attribute__((always_inline)) {
-    constexpr int kLook = 4;
-    const char* kt = kmma_arr(slot, kpar);
-    auto k_frag = [&](int i) __attribute__((always_inline)) {
-      return *reinterpret_cast<const u32x4*>(kt + (i & 1) * 32 * kRow + k_rd[i >> 1]);
-    };
+  auto phase_a = [&](auto par, u32x4 (&fa)[kLook], f32x16 (&nxt)[2], const f32x16 (&cur)[2],
+                     float neg_mu, float (&pf)[2][16], float (&ps)[4],
+                     u32x4 (&pop)[4]) __attribute__((always_inline)) {
     nxt[0] = f32x16{};
     nxt[1] = f32x16{};
-    u32x4 fa[kLook];
-#pragma unroll
-    for (int i = 0; i < kLook; ++i) fa[i] = k_frag(i);
 #pragma unroll
     for (int i = 0; i < 2 * kKSteps; ++i) {
       const u32x4 a = fa[i % kLook];
-      if (i + kLook < 2 * kKSteps) fa[i % kLook] = k_frag(i + kLook);
+      if (i + kLook < 2 * kKSteps) fa[i % kLook] = k_frag(par, i + kLook);
       nxt[i & 1] = Mma<TQ>::run(a, qop[i >> 1], nxt[i & 1]);
       prob(cur, 0, i, neg_mu, pf, ps);
       if (i == 7) pack(pf, 0, 0, pop);
       if (i == 15) pack(pf, 0, 1, pop);
     }
-    __builtin_amdgcn_sched_group_barrier(kDsRead, kLook, 0);
 #pragma unroll
     for (int i = 0; i < 2 * kKSteps; ++i) {
       __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
@@ -1608,18 +1552,20 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
       }
     }
   };
-  // Phase B of tile t: O^T += V^T(t) P^T(t) from V^T buffer `par`; the first eight MFMAs
-  // (keys 0-31) each paired with two probabilities of key block 1, which the last
-  // eight consume, themselves paired with the running maximum of the next tile's scores.
-  // Returns that tile's row maxima.
   auto phase_b = [&](auto par, const f32x16 (&cur)[2], const f32x16 (&nxt)[2], float neg_mu,
                      float (&pf)[2][16], float (&ps)[4],
                      u32x4 (&pop)[4]) __attribute__((always_inline)) -> float {
-    constexpr int kLook = 4;
-    const char* vt = v_arr(par);
+    typedef short v4i16 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
+    const uint32_t vt = lds_address(v_arr(par));
     auto v_frag = [&](int i) __attribute__((always_inline)) {
       const int db = i & 3, ks = i >> 2;
-      return *reinterpret_cast<const u32x4*>(vt + db * 32 * kVRow + v_rd[db & 1][ks]);
+      const uint32_t at = vt + v_rd[db] + ks * 16 * kRow;
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          reinterpret_cast<lds_v4i16*>(at)));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          reinterpret_cast<lds_v4i16*>(at + 8 * kRow)));
+      return u32x4{lo[0], lo[1], hi[0], hi[1]};
     };
     u32x4 fa[kLook];
 #pragma unroll
@@ -1637,11 +1583,11 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
       if (i == 7) pack(pf, 1, 1, pop);
     }
     const float mx = lane_max(nxt);
-    __builtin_amdgcn_sched_group_barrier(kDsRead, kLook, 0);
+    __builtin_amdgcn_sched_group_barrier(kDsRead, 2 * kLook, 0);
 #pragma unroll
     for (int i = 0; i < kDBlocks * 4; ++i) {
       __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-      if (i + kLook < kDBlocks * 4) __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      if (i + kLook < kDBlocks * 4) __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
       if (i == 3 || i == 7) {
         __builtin_amdgcn_sched_group_barrier(kVec, 10, 0);
       } else if (i < 8) {
@@ -1655,180 +1601,114 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
 
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
 
-  // ---- prologue: tiles tb .. tb + 2 staged, page ids of the next three fetched; tile
-  // tb's V^T built and its scores computed. Slots and buffers go by t - tb.
-  stage(tb, page_of(tb), I0{});
-  stage(tb + 1, page_of(tb + 1), I1{});
-  stage(tb + 2, page_of(tb + 2), I2{});
-  int pg[3] = {page_of(tb + 3), page_of(tb + 4), page_of(tb + 5)};  // pg[x]: next tile staged into slot x
-  // The queries (the oldest loads) and tile tb have landed. The wait names the query
-  // registers: their loads are untracked, and a wait the compiler placed itself would
-  // sit in the tile loop (the first scores are conditional), draining every step's
-  // fresh copies.
-  asm volatile("s_waitcnt vmcnt(%8)"
-               : "+v"(qop[0]), "+v"(qop[1]), "+v"(qop[2]), "+v"(qop[3]), "+v"(qop[4]),
-                 "+v"(qop[5]), "+v"(qop[6]), "+v"(qop[7])
-               : "n"(2 * kStageOps)
-               : "memory");
-  if constexpr (kFp8) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // tile 0's scales
-    convert_k(I0{}, I0{});
+  // ---- prologue: K of tiles tb and tb + 1 and V of tile tb staged; tile tb's scores.
+  // (A block of page ids is taken up at the step that stages its first K; V of the tile
+  // before, staged with it, has its page from the step before.)
+  int pg1 = 0;            // page of tile t + 1
+  float vs1 = 0.0f;       // fp8: its V scale
+  float ks_raw = 0.0f, vs_raw = 0.0f;  // fp8: the scales of the staged raw rows
+  {
+    take_pages(tb);
+    const int pg0 = page_of(tb);
+    const float ks0 = lane_scale(ks_lane, tb);
+    vs_raw = lane_scale(vs_lane, tb);
+    stage_k(tb, pg0, I0{});
+    if constexpr (!kFp8) stage_v(tb, pg0, I0{});
+    if (((tb + 1) & (kWave - 1)) == 0) take_pages(tb + 1);
+    pg1 = page_of(tb + 1);
+    vs1 = lane_scale(vs_lane, tb + 1);
+    ks_raw = lane_scale(ks_lane, tb + 1);
+    if constexpr (!kFp8) stage_k(tb + 1, pg1, I1{});
+    // The queries (the oldest loads) and the first K have landed. The wait names the query
+    // registers: their loads are untracked, and a wait the compiler placed itself would
+    // sit in the tile loop (the first scores are conditional), draining its fresh copies.
+    asm volatile("s_waitcnt vmcnt(%8)"
+                 : "+v"(qop[0]), "+v"(qop[1]), "+v"(qop[2]), "+v"(qop[3]), "+v"(qop[4]),
+                   "+v"(qop[5]), "+v"(qop[6]), "+v"(qop[7])
+                 : "n"(kFp8 ? 0 : 2 * kCopies)
+                 : "memory");
+    if constexpr (kFp8) {
+      convert(k_raw, k_lds0, ks0, true);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      stage_k(tb + 1, pg1, I1{});
+      stage_v(tb, pg0, I0{});
+    }
   }
-  store_v(I0{}, I0{});
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   float row_max = -INFINITY;  // of the current tile's scores, each query's
   if (tb < w_nt) {
-    qk(I0{}, I0{}, sc0);
+    qk(I0{}, sc0);
     mask(tb, sc0);
     row_max = max_across32(lane_max(sc0));
   }
 
-  // Step for tile t: X = (t - tb) % 3 (the slots tile t used, restaged with tile t + 3),
-  // Y = (t - tb + 1) % 3 (tile t + 1's slots), P = (t - tb) & 1 (tile t's score and V^T
-  // buffers).
-  auto step = [&](int t, auto xs, auto par) __attribute__((always_inline)) {
-    constexpr int X = decltype(xs)::value;
-    constexpr int Y = (X + 1) % 3;
+  // Step for tile t, P = (t - tb) & 1: K(t) was read by the previous step, K(t + 1) and
+  // V(t) have landed.
+  auto step = [&](int t, auto par) __attribute__((always_inline)) {
     constexpr int P = decltype(par)::value;
-    using IY = std::integral_constant<int, Y>;
-    using IQ = std::integral_constant<int, 1 - P>;
+    using IN = std::integral_constant<int, 1 - P>;
     f32x16(&cur)[2] = P == 0 ? sc0 : sc1;
     f32x16(&nxt)[2] = P == 0 ? sc1 : sc0;
-    // Tile t + 1 has landed for this wave (tiles t + 2 may still be in flight); the
-    // barrier publishes it and tile t's V^T, and retires tile t - 1.
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStageOps) : "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (kFp8) {
-      // This wave's K rows of tile t + 1, converted before the barrier publishes them
-      // (the buffer's last readers, tile t - 1's scores, finished before the previous
-      // barrier). Tile t + 1's scales were loaded three steps ago.
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      convert_k(IY{}, IQ{});
+      // (the buffers' last readers, S(t - 1) and PV(t - 2), are a barrier behind)
+      convert(k_raw, k_arr(IN{}), ks_raw, true);
+      convert(v_raw, v_arr(par), vs_raw, false);
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    store_v(IY{}, IQ{});
-    stage(t + 3, pg[X], xs);
-    pg[X] = page_of(t + 6);
+    u32x4 fk[kLook];  // the first K fragments, on their way while the copies are issued
+#pragma unroll
+    for (int i = 0; i < kLook; ++i) fk[i] = k_frag(IN{}, i);
+    if (((t + 2) & (kWave - 1)) == 0) take_pages(t + 2);
+    stage_v(t + 1, pg1, IN{});
+    vs_raw = vs1;
+    pg1 = page_of(t + 2);
+    vs1 = lane_scale(vs_lane, t + 2);
+    ks_raw = lane_scale(ks_lane, t + 2);
+    stage_k(t + 2, pg1, par);
     __builtin_amdgcn_sched_barrier(0);
     if (t < w_nt) {
       const float neg_mu = raise_max(row_max);
       float pf[2][16];
       float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       u32x4 pop[4];
-      // Scores of tile t + 1 even past this wave's last tile (the slot then holds a
-      // staged copy of a valid tile; the result goes unused): no branch, so the
-      // probabilities stay interleaved with these MFMAs.
-      phase_a(IY{}, IQ{}, nxt, cur, neg_mu, pf, ps, pop);
-      // (keeps phase A's probabilities ahead of the mask's branch: left alone the compiler
-      // sinks them past it, out of those MFMAs' shadow)
+      phase_a(IN{}, fk, nxt, cur, neg_mu, pf, ps, pop);
       asm volatile("" : "+v"(pop[0]), "+v"(pop[1]), "+v"(ps[0]), "+v"(ps[1]), "+v"(ps[2]), "+v"(ps[3]));
       mask(t + 1, nxt);
       row_max = phase_b(par, cur, nxt, neg_mu, pf, ps, pop);
       l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);
     }
   };
-  for (int t = tb; t < te; t += 6) {
-    step(t, I0{}, I0{});
-    if (t + 1 < te) step(t + 1, I1{}, I1{});
-    if (t + 2 < te) step(t + 2, I2{}, I0{});
-    if (t + 3 < te) step(t + 3, I0{}, I1{});
-    if (t + 4 < te) step(t + 4, I1{}, I0{});
-    if (t + 5 < te) step(t + 5, I2{}, I1{});
+  for (int t = tb; t < te; t += 2) {
+    step(t, I0{});
+    if (t + 1 < te) step(t + 1, I1{});
   }
   // No copy may still be writing LDS when the workgroup ends.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if constexpr (kSplit) {
-    // A cut item: every piece stores its (m, l, O) partial (each lane its own, in the
-    // lane order every piece shares), then counts itself in; the last to arrive
-    // resets the counter for the next launch and merges the other pieces' partials
-    // into its own accumulators before the usual normalise and store.
-    //
-    // The partials are written and read with relaxed atomic stores and loads at agent
-    // (device) scope, which the hardware keeps coherent per location across the XCDs'
-    // L2s (scope bits on each access) rather than with a fence: an agent-scope fence
-    // writes back and invalidates the whole L2 of the XCD, dropping the K/V lines
-    // every other workgroup there is reading (measured: cut pieces ran at 5.6 us per
-    // tile against 3.5). Order: a piece's stores complete (vmcnt(0), every wave, then
-    // the barrier) before its counter increment is issued; the last piece issues its
-    // loads only after the increment has returned, through the barrier that
-    // publishes the result.
-    if (piece.pieces > 1) {
-      __shared__ int split_last;
-      const int cols = p.hk * chunks;
-      auto slot_of = [&](int j) __attribute__((always_inline)) -> float* {
-        return p.pf_part + (static_cast<int64_t>(piece.slot0 + j) * cols + c) * kSplitSlotFloats;
-      };
-      auto o_at = [&](float* slot, int k) __attribute__((always_inline)) -> float* {
-        return slot + ((wave * 16 + k) * kWave + lane) * 4;
-      };
-      auto ml_at = [&](float* slot) __attribute__((always_inline)) -> float* {
-        return slot + kWaves * kWave * 64 + (wave * kWave + lane) * 2;
-      };
-      auto put = [&](float* at, float v) __attribute__((always_inline)) {
-        __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      };
-      auto get = [&](float* at) __attribute__((always_inline)) -> float {
-        return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      };
-      {
-        float* mine = slot_of(piece.piece);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          const f32x16& a = o[k >> 2];
-          const int r = 4 * (k & 3);
-          float* at = o_at(mine, k);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) put(at + e, a[r + e]);
-        }
-        put(ml_at(mine), m_run);
-        put(ml_at(mine) + 1, l_run);
-      }
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (tid == 0) {
-        int* count = p.pf_count + piece.item * cols + c;
-        const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int last = before == piece.pieces - 1 ? 1 : 0;
-        if (last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        split_last = last;
-      }
-      __syncthreads();
-      if (split_last == 0) return;
-      // All pieces folded in piece order from an empty state (this piece's own from
-      // registers), so the result is the same whichever piece finishes last.
-      float m_acc = -INFINITY, l_acc = 0.0f;
-      f32x16 o_acc[kDBlocks];
-#pragma unroll
-      for (int db = 0; db < kDBlocks; ++db) o_acc[db] = f32x16{};
-      for (int j = 0; j < piece.pieces; ++j) {
-        float* other = slot_of(j);
-        const bool own = j == piece.piece;
-        const float m_o = own ? m_run : get(ml_at(other));
-        const float l_o = own ? l_run : get(ml_at(other) + 1);
-        const float m_new = fmaxf(m_acc, m_o);
-        const float fa = m_acc == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_acc - m_new);
-        const float fb = m_o == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_o - m_new);
-        l_acc = l_acc * fa + l_o * fb;
-        m_acc = m_new;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          f32x16& a = o_acc[k >> 2];
-          const f32x16& mine = o[k >> 2];
-          const int r = 4 * (k & 3);
-          float* at = o_at(other, k);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a[r + e] = a[r + e] * fa + (own ? mine[r + e] : get(at + e)) * fb;
-        }
-      }
-      m_run = m_acc;
-      l_run = l_acc;
-#pragma unroll
-      for (int db = 0; db < kDBlocks; ++db) o[db] = o_acc[db];
-    }
-  }
   if (!w_active || !my_valid) return;
   const float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
+  if constexpr (kSplit) {
+    if (piece.pieces > 1) {
+      // A cut item: the unnormalised O, the running max and the sum, fp32, to the piece's
+      // slot ([2 heads][64 rows][D], then [2 heads][64 rows] of (max, sum)).
+      const int cols = p.hk * chunks;
+      float* slot = p.pf_part + (static_cast<int64_t>(piece.slot0 + piece.piece) * cols + c) * kPairSlotFloats;
+      const int row = hs * kPairQueryTile + 32 * wq + l32;
+#pragma unroll
+      for (int db = 0; db < kDBlocks; ++db) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          *reinterpret_cast<f32x4*>(slot + row * D + db * 32 + 8 * j + 4 * hsel) =
+              f32x4{o[db][4 * j], o[db][4 * j + 1], o[db][4 * j + 2], o[db][4 * j + 3]};
+        }
+      }
+      if (hsel == 0) {
+        *reinterpret_cast<float2*>(slot + 2 * kPairQueryTile * D + 2 * row) = make_float2(m_run, l_tot);
+      }
+      return;
+    }
+  }
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   const int64_t orow = (static_cast<int64_t>(row_base + my_local) * p.hq + head0) * D;
 #pragma unroll
@@ -1842,6 +1722,68 @@ __global__ __launch_bounds__(512) void paged_prefill_pipe_kernel(const PagedPara
       *reinterpret_cast<u32x2*>(static_cast<char*>(p.out) + (orow + d) * 2) =
           u32x2{Mma<TQ>::pack2(r[0], r[1]), Mma<TQ>::pack2(r[2], r[3])};
     }
+  }
+}
+
+// Combine the pieces of the pair kernel's cut items: the workgroup at position (rank,
+// column) takes its own piece's share of the item's 128 x D outputs (its two heads' rows),
+// so a long item's merge is spread over as many workgroups as computed it; positions
+// without a cut item end at once. Each thread owns float4 columns of rows and folds the
+// pieces in piece order (the result does not depend on timing), kMergeBatch pieces'
+// loads in flight at a time.
+constexpr int kPairMergeThreads = 256;
+
+template <typename TQ>
+__global__ __launch_bounds__(kPairMergeThreads) void paged_prefill_pair_merge_kernel(const PagedParams p) {
+  constexpr int D = 128;
+  constexpr int kMergeBatch = 8;
+  const int group = p.hq / p.hk;
+  const int cols = p.hq / 2;
+  const int c = static_cast<int>(blockIdx.x) % cols;
+  const int rank = static_cast<int>(blockIdx.x) / cols;
+  const int4 rec = p.pf_rec[2 * rank];
+  const int slot0 = p.pf_rec[2 * rank + 1].x;
+  const int s = rec.x, q = rec.y, piece = rec.z, pieces = rec.w;
+  if (pieces <= 1) return;
+  const int rows = min(kPairQueryTile, p.seq_lens[s] - q * kPairQueryTile);
+  const int row0 = p.cu_seqlens_q[s] + q * kPairQueryTile;
+  const int head0 = (c / (group / 2)) * group + (c % (group / 2)) * 2;
+  const int n4 = 2 * rows * (D / 4);
+  const int lo = piece * n4 / pieces, hi = (piece + 1) * n4 / pieces;
+  const int64_t stride = static_cast<int64_t>(cols) * kPairSlotFloats;
+  const float* base = p.pf_part + (static_cast<int64_t>(slot0) * cols + c) * kPairSlotFloats;
+  for (int j = lo + static_cast<int>(threadIdx.x); j < hi; j += kPairMergeThreads) {
+    const int hw = j / (rows * (D / 4));
+    const int rem = j - hw * rows * (D / 4);
+    const int local = rem / (D / 4), d = (rem % (D / 4)) * 4;
+    const int row = hw * kPairQueryTile + local;
+    float m = -INFINITY, l = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < pieces; i0 += kMergeBatch) {
+      float2 ml[kMergeBatch];
+      f32x4 oi[kMergeBatch];
+#pragma unroll
+      for (int u = 0; u < kMergeBatch; ++u) {
+        const float* slot = base + min(i0 + u, pieces - 1) * stride;
+        ml[u] = *reinterpret_cast<const float2*>(slot + 2 * kPairQueryTile * D + 2 * row);
+        oi[u] = *reinterpret_cast<const f32x4*>(slot + row * D + d);
+      }
+#pragma unroll
+      for (int u = 0; u < kMergeBatch; ++u) {
+        if (i0 + u >= pieces) continue;
+        const float mn = fmaxf(m, ml[u].x);
+        const float mu = mn == -INFINITY ? 0.0f : mn;
+        const float a = __builtin_amdgcn_exp2f(m - mu);
+        const float b = __builtin_amdgcn_exp2f(ml[u].x - mu);
+        l = l * a + ml[u].y * b;
+        acc = acc * a + oi[u] * b;
+        m = mn;
+      }
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int64_t obase = (static_cast<int64_t>(row0 + local) * p.hq + head0 + hw) * D + d;
+    *reinterpret_cast<u32x2*>(static_cast<char*>(p.out) + obase * 2) =
+        u32x2{Mma<TQ>::pack2(acc[0] * inv, acc[1] * inv), Mma<TQ>::pack2(acc[2] * inv, acc[3] * inv)};
   }
 }
 
@@ -2008,59 +1950,56 @@ void launch_prefill_cfg(const PagedParams& p, int max_query_len, hipStream_t str
   }
 }
 
-// The pipelined kernel on the item grid, or on the split grid when the plan cuts items
-// (pf_pieces > 1, with the counters and partial slots it names).
+// The pair kernel: the split schedule when the launch has pieces to make (pf_pieces > 1),
+// the item grid otherwise. Workgroups of 64 query positions, but of 128 for fp8 pools when
+// those still fill the CUs: staging a tile there means converting it, work that the
+// larger workgroup halves (8 x 512 tokens after up to 1536: 67 us against 69; 5 chunks of
+// up to 512 tokens, 134 such workgroups: 73 against 63).
 template <typename TQ, typename TKV>
-void launch_prefill_pipe(const PagedParams& p, int max_query_len, hipStream_t stream) {
-  const int cols = p.hk * (p.hq / p.hk / 2);
-  if (p.pf_pieces > 1 && p.pf_count != nullptr && p.pf_part != nullptr) {
-    paged_prefill_pipe_kernel<TQ, TKV, true><<<cols * p.pf_ranks, 512, 0, stream>>>(p);
+void launch_prefill_pair(const PagedParams& p, int max_query_len, hipStream_t stream) {
+  const int cols = p.hq / 2;
+  if (p.pf_pieces > 1) {
+    paged_prefill_pair_kernel<TQ, TKV, 4, true><<<cols * p.pf_ranks, 256, 0, stream>>>(p);
+    paged_prefill_pair_merge_kernel<TQ><<<cols * p.pf_ranks, kPairMergeThreads, 0, stream>>>(p);
     return;
   }
-  const int qtiles = (max_query_len + kPrefillQueryTile - 1) / kPrefillQueryTile;
-  paged_prefill_pipe_kernel<TQ, TKV, false><<<dim3(cols, p.num_seqs, qtiles), 512, 0, stream>>>(p);
+  if constexpr (std::is_same_v<TKV, fp8_t>) {
+    const int wide = (max_query_len + 127) / 128;
+    if ((p.num_tokens + 127) / 128 * cols >= p.pf_cus) {
+      paged_prefill_pair_kernel<TQ, TKV, 8, false><<<dim3(cols, p.num_seqs, wide), 512, 0, stream>>>(p);
+      return;
+    }
+  }
+  const int qtiles = (max_query_len + kPairQueryTile - 1) / kPairQueryTile;
+  paged_prefill_pair_kernel<TQ, TKV, 4, false><<<dim3(cols, p.num_seqs, qtiles), 256, 0, stream>>>(p);
 }
 
-template <typename TQ, int HS>
+template <typename TQ>
 void launch_prefill_lds(const PagedParams& p, int max_query_len, hipStream_t stream) {
   if (p.pf_wgs > 0) {
-    paged_prefill_lds_kernel<TQ, HS, true><<<p.pf_wgs, 256 * HS, 0, stream>>>(p);
-    paged_prefill_merge_kernel<TQ, 128, HS><<<kMergeSub * p.pf_wgs, kMergeThreads, 0, stream>>>(p);
+    paged_prefill_lds_kernel<TQ, 1, true><<<p.pf_wgs, 256, 0, stream>>>(p);
+    paged_prefill_merge_kernel<TQ, 128, 1><<<kMergeSub * p.pf_wgs, kMergeThreads, 0, stream>>>(p);
   } else {
-    const int cols = p.hk * (p.hq / p.hk / HS);
     const int qtiles = (max_query_len + kPrefillQueryTile - 1) / kPrefillQueryTile;
-    const dim3 grid(cols, p.num_seqs, qtiles);
-    if constexpr (HS == 2) {
-      if (!p.pf_register_staging) {
-        launch_prefill_pipe<TQ, TQ>(p, max_query_len, stream);
-        return;
-      }
-    }
-    paged_prefill_lds_kernel<TQ, HS, false><<<grid, 256 * HS, 0, stream>>>(p);
+    paged_prefill_lds_kernel<TQ, 1, false><<<dim3(p.hq, p.num_seqs, qtiles), 256, 0, stream>>>(p);
   }
 }
 
 template <typename TQ, typename TKV, int D>
 hipError_t launch_prefill_d(const PagedParams& p, int max_query_len, hipStream_t stream) {
-  // 16-bit pools at D = 128 with pages of >= 16 keys and a positive scale: K copied
-  // straight into LDS.
-  if constexpr (std::is_same_v<TQ, TKV> && D == 128) {
+  // D = 128, pages of >= 16 keys and a positive scale: K/V copied straight into LDS.
+  // GQA pairs take the pair kernel (16-bit and fp8 pools), odd groups over a 16-bit pool
+  // the one-head kernel.
+  if constexpr (D == 128) {
     if (p.block_shift >= 4 && p.scale > 0.0f && !p.pf_register_staging) {
-      if (prefill_item_heads(p.hq / p.hk) == 1) {
-        launch_prefill_lds<TQ, 1>(p, max_query_len, stream);
-      } else {
-        launch_prefill_lds<TQ, 2>(p, max_query_len, stream);
+      if (prefill_item_heads(p.hq / p.hk) == 2) {
+        launch_prefill_pair<TQ, TKV>(p, max_query_len, stream);
+        return hipGetLastError();
       }
-      return hipGetLastError();
-    }
-  }
-  // fp8 pools at D = 128, GQA pairs, pages of >= 16 keys, the grid schedule: the
-  // pipelined kernel, codes copied straight into LDS and dequantised there.
-  if constexpr (std::is_same_v<TKV, fp8_t> && D == 128) {
-    if (p.block_shift >= 4 && p.scale > 0.0f && !p.pf_register_staging && p.pf_wgs == 0 &&
-        prefill_item_heads(p.hq / p.hk) == 2) {
-      launch_prefill_pipe<TQ, fp8_t>(p, max_query_len, stream);
-      return hipGetLastError();
+      if constexpr (std::is_same_v<TQ, TKV>) {
+        launch_prefill_lds<TQ>(p, max_query_len, stream);
+        return hipGetLastError();
+      }
     }
   }
   // Both heads of an even GQA group in one wave (HCW = 2) would share K/V fragments,

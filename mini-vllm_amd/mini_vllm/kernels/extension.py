@@ -900,8 +900,9 @@ class HipExtension:
             sink.data_ptr(), sink.numel() * sink.element_size() // 4, _stream(base.device)))
 
     def split_stats(self) -> dict[str, int]:
-        """The split prefill grid's counter regions in use on the current device, and the
-        split launches that ran every item whole (no region left; stream capturing)."""
+        """Prefill launches whose items the grid would have cut but that ran whole because
+        their stream was being captured (``mvllm_split_stats``; the other two counts
+        described arrival counters that the kernels no longer have: 0)."""
         used, no_region, capturing = ctypes.c_int32(0), ctypes.c_int64(0), ctypes.c_int64(0)
         self.lib.mvllm_split_stats(ctypes.byref(used), ctypes.byref(no_region),
                                    ctypes.byref(capturing))

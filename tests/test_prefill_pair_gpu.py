@@ -1,0 +1,74 @@
+"""The pair prefill kernel (GQA pairs, D = 128) at the edges of its tiles, its blocks of page
+ids and its split schedule, on the MI355X (``-m gpu``), against the fp32 oracle at the
+repository's tolerances (tests/conftest.py)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from mini_vllm.workloads import build_batch
+from oracle.paged_attention import paged_attention as oracle
+from conftest import ATTN_ATOL, assert_max_abs
+
+pytestmark = pytest.mark.gpu
+
+F8 = torch.float8_e4m3fn
+WHOLE = {"prefill_schedule": "grid", "prefill_pieces": 1}
+CUT = {"prefill_schedule": "stream", "prefill_share_tiles": 1}
+
+
+def check(extension, contexts, lens, dtype, kv_dtype, options, hq=16):
+    b = build_batch(contexts, lens, dtype=dtype, kv_dtype=kv_dtype, num_q_heads=hq,
+                    num_kv_heads=8, head_dim=128, seed=len(contexts), device="cuda")
+    got = extension.paged_attention(*b.args(), k_scale=b.k_scale, v_scale=b.v_scale,
+                                    plan_options=options)
+    want = oracle(b.q, b.key_pool, b.value_pool, b.block_tables, b.cu_seqlens_q, b.context_lens,
+                  b.scale, **({"k_scale": b.k_scale, "v_scale": b.v_scale} if kv_dtype else {}))
+    assert_max_abs(got.float(), want, ATTN_ATOL[kv_dtype or dtype], f"{contexts} {lens}")
+
+
+@pytest.mark.parametrize("options", [WHOLE, CUT], ids=["whole", "cut"])
+@pytest.mark.parametrize("dtype,kv_dtype", [(torch.bfloat16, None), (torch.float16, None),
+                                            (torch.bfloat16, F8)])
+def test_tile_edges(extension, device, dtype, kv_dtype, options):
+    """Query and key counts one below, at and one past the 64-row tiles, one to three key
+    tiles, a wave with no rows, rows that see a tile's first key only."""
+    lens = [2, 31, 32, 33, 63, 64, 65, 127, 129]
+    contexts = [2, 64, 65, 33, 128, 127, 192, 193, 129]
+    check(extension, contexts, lens, dtype, kv_dtype, options)
+
+
+@pytest.mark.parametrize("options", [WHOLE, CUT], ids=["whole", "cut"])
+@pytest.mark.parametrize("kv_dtype", [None, F8], ids=["bf16", "fp8"])
+def test_page_id_blocks(extension, device, kv_dtype, options):
+    """A wave holds its page ids 64 tiles at a time: contexts ending around tiles 63-66 and
+    127-129, where the next block is taken up a step or two before it is used."""
+    contexts = [64 * n + d for n, d in ((63, 0), (63, 1), (64, 0), (64, 1), (65, 1), (66, 0), (128, 5))]
+    check(extension, contexts, [5] * 7, torch.bfloat16, kv_dtype, options)
+
+
+@pytest.mark.parametrize("tokens", [64 * 31, 64 * 32 + 1])
+def test_fp8_workgroups_of_either_size(extension, device, tokens):
+    """Around the token count where fp8 pools take 128-position workgroups (256 of them)."""
+    lens = [tokens - 3 * 500, 500, 500, 500]
+    check(extension, [n + 77 for n in lens], lens, torch.bfloat16, F8, WHOLE, hq=32)
+
+
+def test_cut_items_of_many_sequences(extension, device):
+    """More than 64 sequences (the schedule's lanes hold 64 at a time), chunks among decode
+    rows, one far longer than the rest and cut into many pieces; three calls, the same bits."""
+    contexts = [40 + 7 * i for i in range(150)]
+    lens = [1 if i % 3 else 1 + i % 90 for i in range(150)]
+    contexts[99], lens[99] = 5000, 66
+    lens = [min(n, c) for n, c in zip(lens, contexts)]
+    check(extension, contexts, lens, torch.bfloat16, None, CUT)
+    b = build_batch([3000, 64], [70, 64], dtype=torch.bfloat16, num_q_heads=16, num_kv_heads=8,
+                    head_dim=128, seed=2, device="cuda")
+    outs = [extension.paged_attention(*b.args(), plan_options=CUT) for _ in range(3)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+def test_the_default_cuts_a_lone_long_chunk(extension, device):
+    """No options: 63 tokens after 6393 keys (8 items on 256 CUs)."""
+    check(extension, [6456], [63], torch.bfloat16, None, None)

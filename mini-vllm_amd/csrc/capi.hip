@@ -43,6 +43,8 @@ int hip_status(hipError_t err, const char* what) {
               hipGetErrorString(err));
 }
 
+int element_bytes(int dtype) { return dtype == mvllm::kF32 ? 4 : (dtype == mvllm::kFP8E4M3 ? 1 : 2); }
+
 bool is_pow2(int64_t v) { return v > 0 && (v & (v - 1)) == 0; }
 
 // Compute units of the current device, cached per device id.
@@ -318,10 +320,12 @@ void plan_decode(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, i
 
   if (plan.pub.decode_mode == MVLLM_DECODE_STREAM) {
     // A few workgroups per CU, each streaming an equal share of all decode keys; no
-    // more workgroups than there are ~64-key shares in the largest possible batch.
+    // more workgroups than there are smallest shares in the largest possible batch.
     int64_t wgs = static_cast<int64_t>(o.decode_wgs_per_cu) * device_cus();
-    const int64_t by_size = (static_cast<int64_t>(num_seqs) * max_ctx + 63) / 64;
+    const int64_t least = mvllm::decode_min_share_keys(element_bytes(kv_dtype), d);
+    const int64_t by_size = (static_cast<int64_t>(num_seqs) * max_ctx + least - 1) / least;
     if (wgs > by_size) wgs = by_size;
+    if (wgs > mvllm::kMaxDecodeShares) wgs = mvllm::kMaxDecodeShares;
     if (wgs < 1) wgs = 1;
     plan.pub.decode_workgroups = static_cast<int32_t>(wgs);
     // [prefix: num_seqs + 1 int32][O partials][(m, l) partials]
@@ -365,6 +369,7 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
                    int32_t kv_dtype, int32_t head_dim, int32_t max_query_len, hipStream_t s,
                    const char* name) {
   p.stream_wgs = plan.pub.decode_mode == MVLLM_DECODE_STREAM ? plan.pub.decode_workgroups : 0;
+  p.stream_min_keys = mvllm::decode_min_share_keys(element_bytes(kv_dtype), head_dim);
   p.split_tokens = plan.pub.split_tokens > 0 ? plan.pub.split_tokens : mvllm::kMaxSplitTokens;
   p.max_splits = plan.max_splits;
   p.by_row = plan.pub.decode_mode == MVLLM_DECODE_BY_ROW ? 1 : 0;
@@ -878,6 +883,7 @@ int mvllm_paged_decode_qk_norm_rope(
   p.kv_row_bytes = p.kv_head_bytes * num_kv_heads;
   p.scale = scale;
   p.stream_wgs = plan.pub.decode_workgroups;
+  p.stream_min_keys = mvllm::decode_min_share_keys(2, head_dim);
   char* ws = static_cast<char*>(workspace);
   p.seq_prefix = reinterpret_cast<int*>(ws);
   p.part_o = reinterpret_cast<float*>(ws + plan.off_o);
@@ -945,8 +951,13 @@ int mvllm_dense_attention(const mvllm_dense_args* args, void* workspace, uint64_
   meta.query_len = args->query_len;
   meta.kv_len = args->kv_len;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  rc = hip_status(mvllm::launch_dense_meta(meta, s), name);
-  if (rc != MVLLM_OK) return rc;
+  // The stream decode works the metadata out for itself (4.2 us of a 56 us call); the grid
+  // decode and the prefill kernels read it.
+  const bool direct = d.plan.pub.decode_mode == MVLLM_DECODE_STREAM && !d.plan.pub.prefill_mfma;
+  if (!direct) {
+    rc = hip_status(mvllm::launch_dense_meta(meta, s), name);
+    if (rc != MVLLM_OK) return rc;
+  }
 
   const int esize = args->dtype == mvllm::kF32 ? 4 : 2;
   mvllm::PagedParams p{};
@@ -966,6 +977,10 @@ int mvllm_dense_attention(const mvllm_dense_args* args, void* workspace, uint64_
   p.block_shift = 4;
   p.block_mask = 15;
   p.table_shift = 0;
+  if (direct) {
+    p.dense_keys = args->kv_len;
+    p.dense_slots = static_cast<int>(d.slots_per_batch);
+  }
   p.kv_row_bytes = args->k_stride_pos * esize;
   p.kv_head_bytes = args->k_stride_head * esize;
   p.scale = args->scale;

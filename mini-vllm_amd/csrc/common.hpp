@@ -301,6 +301,19 @@ __device__ __forceinline__ float group_max(float v) {
 __device__ __forceinline__ float wave_sum(float v) { return group_sum<64>(v); }
 __device__ __forceinline__ float wave_max(float v) { return group_max<64>(v); }
 
+// Inclusive prefix sum over the wave's 64 lanes: DPP row shifts 1, 2, 4, 8 (within
+// each 16-lane row; a lane whose source lies outside its row adds 0), then lane 15's
+// row total broadcast into rows 1 and 3 and lane 31's into rows 2 and 3.
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
 // Pack N floats (N = 16 / sizeof(T)) back into one 16-byte chunk of T.
 template <typename T>
 __device__ __forceinline__ u32x4 pack_chunk(const float* v) {

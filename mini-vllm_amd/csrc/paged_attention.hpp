@@ -76,19 +76,49 @@ __host__ __device__ inline int prefill_item_tiles(int context, int len, int q) {
   return (context - len + last + kPrefillKeyTile - 1) / kPrefillKeyTile;
 }
 
-// Stream decode: the workgroups that take a share. Shares of at least
-// kMinDecodeShareKeys keys: with few decode keys (a prefill step carrying a handful of
-// decode rows) equal shares over every CU would cut each sequence into dozens of
-// pieces, whose merge then costs more than the keys. (64 since the merge folds a
-// sequence's pieces in several workgroups and thread groups at once; measured
-// graph-replayed: one 8192-key sequence 23.8 -> 21.0 us, 16 x 1024 keys 25.4 -> 20.6 us
-// against 128, 32 no better; full batches, whose shares are larger, unchanged.) Shared
-// by the decode kernel and its merge.
-constexpr int64_t kMinDecodeShareKeys = 64;
-__host__ __device__ inline int64_t decode_stream_shares(int64_t total_keys, int64_t wgs) {
-  const int64_t cap = (total_keys + kMinDecodeShareKeys - 1) / kMinDecodeShareKeys;
-  return cap < 1 ? 1 : (cap < wgs ? cap : wgs);
+// Stream decode: the fewest keys of a share while there are several, the tokens one step of
+// a wave covers (4 per row group of D / (16 / element bytes) lanes): 16 for 16-bit pools
+// at D = 128, 8 for fp32, 32 for fp8. With few keys the launch is a chain of memory round trips
+// per step, and a share of several steps leaves CUs idle meanwhile. (Shares of 64 keys
+// whatever the type before: four fp32 sequences of 37-1000 keys 22.0 us a call, 15.7 with 16;
+// one bf16 sequence of 1500 keys 14.8 -> 11.7, of 200 13.1 -> 9.9, of 8192 17.4 -> 16.9;
+// batches of more than 64 keys per CU do not change.)
+__host__ __device__ inline int decode_min_share_keys(int elem_bytes, int head_dim) {
+  const int keys = 256 * (16 / elem_bytes) / head_dim;
+  return keys < 8 ? 8 : keys;
 }
+constexpr int kMaxDecodeShares = 65535;  // DecodeShares' 32-bit products
+
+// The stream decode's shares: share w owns keys [begin(w), begin(w + 1)) of the `total` laid
+// end to end, begin(w) = floor(w total / count). Never empty: count <= max(1, ceil(total /
+// min_keys)) <= max(1, total). Formed as w floor(total / count) + floor(w (total mod count) /
+// count), in 32 bits: a 64-bit division is ~150 dependent instructions, and each launch made
+// three. (count <= kMaxDecodeShares.)
+struct DecodeShares {
+  uint32_t total, count_u, whole, rest;
+  int count;
+  __host__ __device__ DecodeShares(int total_keys, int wgs, int min_keys)
+      : total(static_cast<uint32_t>(total_keys)) {
+    const uint32_t cap = (total + static_cast<uint32_t>(min_keys) - 1) / static_cast<uint32_t>(min_keys);
+    count_u = cap < 1 ? 1 : (cap < static_cast<uint32_t>(wgs) ? cap : static_cast<uint32_t>(wgs));
+    count = static_cast<int>(count_u);
+    whole = total / count_u;
+    rest = total - whole * count_u;
+  }
+  __host__ __device__ int begin(int w) const {
+    const uint32_t u = static_cast<uint32_t>(w);
+    return static_cast<int>(u * whole + u * rest / count_u);
+  }
+  // The share holding key x (0 <= x < total): an estimate within one, corrected.
+  __host__ __device__ int owner(int x) const {
+    int w = static_cast<int>((static_cast<float>(x) + 0.5f) * static_cast<float>(count_u) /
+                             static_cast<float>(total));
+    w = w < 0 ? 0 : (w >= count ? count - 1 : w);
+    while (w > 0 && begin(w) > x) --w;
+    while (w + 1 < count && begin(w + 1) <= x) ++w;
+    return w;
+  }
+};
 
 // Equal shares of `total` work units over `wgs` workgroups: workgroup w owns
 // [floor(w * total / wgs), floor((w + 1) * total / wgs)).
@@ -131,6 +161,8 @@ struct PagedParams {
                           // are slot ids themselves)
   int64_t kv_row_bytes;   // pool bytes between consecutive slots (a paged pool: H_k D elements)
   int64_t kv_head_bytes;  // pool bytes between kv heads of one slot (a paged pool: D elements)
+  int dense_keys;     // stream decode of a dense cache: keys of every sequence (0: paged);
+  int dense_slots;    // position i of sequence s at slot s * dense_slots + i, row s of q
   int stream_wgs;     // decode: > 0 selects the stream schedule with this many workgroups
   int split_tokens;   // grid decode: nominal keys per split
   int max_splits;     // grid decode: grid extent along the split axis
@@ -138,6 +170,7 @@ struct PagedParams {
   float scale;
   float* part_o;      // split partials, D fp32 each
   float* part_ml;     // split partials' (running max in log2 units, sum)
+  int stream_min_keys;  // stream decode: fewest keys of a share while there are several
   int* seq_prefix;    // stream decode: [num_seqs + 1] decode keys before each sequence
   int pf_wgs;         // prefill: > 0 selects the stream schedule with this many workgroups
   int* pf_prefix;     // stream prefill: [num_seqs + 1] work units before each sequence

@@ -96,6 +96,87 @@ __device__ __forceinline__ bool resolve_row(const PagedParams& p, int index, int
   return visible > 0;
 }
 
+// One lane's E elements of a query head, and their dot product with a 16-byte chunk of a K
+// row in fp32. 16-bit queries stay packed and use the two-element dot instruction (exact
+// products, one rounding per pair: against 64 bits 1.27e-8 where the multiply-adds of widened
+// values give 1.32e-8 for bfloat16, 3.94e-8 and 3.94e-8 for float16) over K as it is, or
+// over fp8 codes widened exactly to the query's type: per key and head 4 instructions
+// instead of 8, and no widening of a 16-bit K.
+template <typename TQ, typename TKV> struct Query {
+  static constexpr int E = Chunk<TKV>::kN;
+  float f[E];
+  __device__ void load(const void* q, int64_t base) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) f[e] = Elem<TQ>::load(q, base + e);
+  }
+  __device__ static void widen(const u32x4& k, float (&kf)[E]) { Chunk<TKV>::unpack(k, kf); }
+  using Key = float[E];
+  __device__ float dot(const float (&kf)[E]) const {
+    float d = 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) d = fmaf(f[e], kf[e], d);
+    return d;
+  }
+};
+
+template <typename TQ> __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
+  if constexpr (__is_same(TQ, bf16_t)) {
+    typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b), c,
+                                           false);
+  } else {
+    typedef _Float16 v2 __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b), c, false);
+  }
+}
+
+template <typename TQ, typename TKV> struct PackedQuery {
+  static constexpr int E = Chunk<TKV>::kN;
+  uint32_t w[E / 2];
+  __device__ void load(const void* q, int64_t base) {
+    if (reinterpret_cast<uintptr_t>(q) % 16 == 0) {
+#pragma unroll
+      for (int i = 0; i < E / 8; ++i) set(i, load16(static_cast<const char*>(q) + (base + 8 * i) * 2));
+    } else {  // (the rows start at any element: nothing requires more of q)
+      const uint16_t* e = static_cast<const uint16_t*>(q) + base;
+#pragma unroll
+      for (int i = 0; i < E / 2; ++i) w[i] = e[2 * i] | (static_cast<uint32_t>(e[2 * i + 1]) << 16);
+    }
+  }
+  __device__ void set(int i, const u32x4& v) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[4 * i + j] = v[j];
+  }
+  using Key = uint32_t[E / 2];
+  __device__ static void widen(const u32x4& k, uint32_t (&kw)[E / 2]) {
+    if constexpr (Elem<TKV>::kBytes == 2) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) kw[j] = k[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (__is_same(TQ, bf16_t)) {
+          kw[2 * j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(k[j], 1.0f, false));
+          kw[2 * j + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(k[j], 1.0f, true));
+        } else {
+          kw[2 * j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(k[j], 1.0f, false));
+          kw[2 * j + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(k[j], 1.0f, true));
+        }
+      }
+    }
+  }
+  __device__ float dot(const uint32_t (&kw)[E / 2]) const {
+    float d = 0.0f;
+#pragma unroll
+    for (int j = 0; j < E / 2; ++j) d = dot2<TQ>(w[j], kw[j], d);
+    return d;
+  }
+};
+template <> struct Query<bf16_t, bf16_t> : PackedQuery<bf16_t, bf16_t> {};
+template <> struct Query<f16_t, f16_t> : PackedQuery<f16_t, f16_t> {};
+template <> struct Query<bf16_t, fp8_t> : PackedQuery<bf16_t, fp8_t> {};
+template <> struct Query<f16_t, fp8_t> : PackedQuery<f16_t, fp8_t> {};
+
 // Per-wave online-softmax state over a run of keys, for GC query heads.
 template <int GC, int E>
 struct WaveState {
@@ -104,7 +185,7 @@ struct WaveState {
   float acc[GC][E];
 };
 
-template <typename TKV, int D, int GC>
+template <typename TQ, typename TKV, int D, int GC>
 struct Decode {
   static constexpr int E = Chunk<TKV>::kN;   // elements per 16-byte chunk
   static constexpr int R = D / E;            // lanes per token row
@@ -113,14 +194,12 @@ struct Decode {
   static_assert(R >= 1 && R <= kWave && (kWave % R) == 0, "head dim / dtype mismatch");
   using State = WaveState<GC, E>;
 
-  template <typename TQ>
-  __device__ static void load_queries(const PagedParams& p, int row, int h0, int r,
-                                      float (&qf)[GC][E]) {
+  using Q = Query<TQ, TKV>;
+
+  __device__ static void load_queries(const PagedParams& p, int row, int h0, int r, Q (&qf)[GC]) {
 #pragma unroll
     for (int h = 0; h < GC; ++h) {
-      const int64_t base = (static_cast<int64_t>(row) * p.hq + h0 + h) * D + r * E;
-#pragma unroll
-      for (int e = 0; e < E; ++e) qf[h][e] = Elem<TQ>::load(p.q, base + e);
+      qf[h].load(p.q, (static_cast<int64_t>(row) * p.hq + h0 + h) * D + r * E);
     }
   }
 
@@ -136,15 +215,16 @@ struct Decode {
 
   // Stream keys [sb, se) of one sequence for kv head `kvh` into `st`. Page ids come
   // from `lds_pages` (page i of the run at lds_pages[i - first_page]) when given,
-  // otherwise from the sequence's block table; the next step's page ids are requested
+  // otherwise from the sequence's block table, or with none (a dense cache, table_shift 0)
+  // are the slots of positions 16 i from dense_base on; the next step's ids are requested
   // before this step is computed. (Requesting the next step's K/V rows early as well
   // measured slower: on shuffled pages more requests in flight per CU cost DRAM
   // efficiency.)
-  __device__ static void stream(const PagedParams& p, const int32_t* table, const int* lds_pages,
-                                int first_page, int kvh, int sb, int se, int g, int r,
-                                const float (&qf)[GC][E], float score_scale, State& st) {
+  __device__ static void stream(const PagedParams& p, const int32_t* table, int dense_base,
+                                const int* lds_pages, int first_page, int kvh, int sb, int se, int g, int r,
+                                const Q (&qf)[GC], float score_scale, State& st) {
     const Fresh none{-1, {}, {}};
-    stream_with<false>(p, table, lds_pages, first_page, kvh, sb, se, g, r, qf, score_scale, st,
+    stream_with<false>(p, table, dense_base, lds_pages, first_page, kvh, sb, se, g, r, qf, score_scale, st,
                        [] {}, none);
   }
 
@@ -162,8 +242,8 @@ struct Decode {
   // first step's K/V requests instead measured the same, with 60% more registers.)
   template <bool kFresh, typename Prep>
   __device__ static void stream_with(const PagedParams& p, const int32_t* table,
-                                     const int* lds_pages, int first_page, int kvh, int sb, int se,
-                                     int g, int r, const float (&qf)[GC][E], float score_scale,
+                                     int dense_base, const int* lds_pages, int first_page, int kvh, int sb, int se,
+                                     int g, int r, const Q (&qf)[GC], float score_scale,
                                      State& st, Prep&& prep, const Fresh& fresh) {
     static_assert(!(kFresh && kFp8), "the fresh-token stream serves 16-bit pools");
     const char* kbase = static_cast<const char*>(p.k_pool);
@@ -172,6 +252,7 @@ struct Decode {
     constexpr int kStep = RG * kUnroll;
 
     auto page_of = [&](int tok) -> int {
+      if (table == nullptr) return dense_base + (tok & ~p.block_mask);
       const int pi = tok >> p.block_shift;
       return lds_pages != nullptr ? lds_pages[pi - first_page] : table[pi];
     };
@@ -223,14 +304,11 @@ struct Decode {
       float s[kUnroll][GC];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        float kf[E];
-        Chunk<TKV>::unpack(kw[u], kf);
+        typename Q::Key kf;
+        Q::widen(kw[u], kf);
 #pragma unroll
         for (int h = 0; h < GC; ++h) {
-          float dot = 0.0f;
-#pragma unroll
-          for (int e = 0; e < E; ++e) dot = fmaf(qf[h][e], kf[e], dot);
-          dot = group_sum<R>(dot);
+          const float dot = group_sum<R>(qf[h].dot(kf));
           // The reference scales after the reduction (paged_attention.cu:181-183).
           float sc = dot * score_scale;
           if constexpr (kFp8) sc *= ks[u];
@@ -300,7 +378,6 @@ struct Decode {
     }
   }
 
-  template <typename TQ>
   __device__ static void write_output(const PagedParams& p, int row, int h0, int r, const State& st) {
 #pragma unroll
     for (int h = 0; h < GC; ++h) {
@@ -350,43 +427,61 @@ __device__ __forceinline__ bool wave_unit(const PagedParams& p, int unit, int& k
 template <typename TQ, typename TKV, int D, int GC, bool kFresh>
 __global__ __launch_bounds__(512) void paged_decode_stream_kernel(const PagedParams p,
                                                                   const FreshParams f) {
-  using K = Decode<TKV, D, GC>;
+  using K = Decode<TQ, TKV, D, GC>;
   __shared__ int s_prefix[kMaxStreamSeqs + 1];  // decode keys before sequence s
 
   const int n = p.num_seqs;
   const int tid = threadIdx.x;
-  // Prefix scan of the decode sequences' context lengths (0 for prefill chunks), by
-  // wave 0: each lane sums a contiguous run, then a 64-lane inclusive scan.
-  if (tid < kWave) {
-    const int per = (n + kWave - 1) / kWave;
-    const int begin = min(tid * per, n);
-    const int end = min(begin + per, n);
-    int run = 0;
-    for (int s = begin; s < end; ++s) run += p.seq_lens[s] == 1 ? max(p.context_lens[s], 0) : 0;
-    int incl = run;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int other = __shfl_up(incl, off, kWave);
-      if (tid >= off) incl += other;
+  // Prefix sums of the decode sequences' context lengths (0 for prefill chunks). Up to 64
+  // sequences: every wave for itself, lane s holding the keys up to and with sequence s's,
+  // no barrier and no LDS. More: by wave 0, each lane summing a contiguous run, through
+  // s_prefix.
+  // A dense cache: every sequence holds dense_keys, nothing is read.
+  const bool dense = !kFresh && p.dense_keys > 0;
+  const bool by_lane = n <= kWave;
+  int upto = 0;
+  if (dense) {
+  } else if (by_lane) {
+    const int s = tid % kWave;
+    upto = wave_inclusive_scan(s < n && p.seq_lens[s] == 1 ? max(p.context_lens[s], 0) : 0);
+  } else {
+    if (tid < kWave) {
+      const int per = (n + kWave - 1) / kWave;
+      const int begin = min(tid * per, n);
+      const int end = min(begin + per, n);
+      int run = 0;
+      for (int s = begin; s < end; ++s) run += p.seq_lens[s] == 1 ? max(p.context_lens[s], 0) : 0;
+      const int incl = wave_inclusive_scan(run);
+      int acc = incl - run;
+      for (int s = begin; s < end; ++s) {
+        s_prefix[s] = acc;
+        acc += p.seq_lens[s] == 1 ? max(p.context_lens[s], 0) : 0;
+      }
+      if (tid == kWave - 1) s_prefix[n] = incl;
     }
-    int acc = incl - run;
-    for (int s = begin; s < end; ++s) {
-      s_prefix[s] = acc;
-      acc += p.seq_lens[s] == 1 ? max(p.context_lens[s], 0) : 0;
-    }
-    if (tid == kWave - 1) s_prefix[n] = incl;
+    __syncthreads();
   }
-  __syncthreads();
+  // Decode keys before sequence i (i uniform, 0 .. n).
+  auto prefix = [&](int i) __attribute__((always_inline)) -> int {
+    if (dense) return i * p.dense_keys;
+    if (!by_lane) return __builtin_amdgcn_readfirstlane(s_prefix[i]);
+    return i == 0 ? 0 : __builtin_amdgcn_readlane(upto, i - 1);
+  };
 
-  const int64_t total = s_prefix[n];
-  const int64_t wgs = decode_stream_shares(total, gridDim.x);
-  if (blockIdx.x == 0) {
-    for (int s = tid; s <= n; s += blockDim.x) p.seq_prefix[s] = s_prefix[s];
+  const int total = prefix(n);
+  const DecodeShares shares(total, gridDim.x, p.stream_min_keys);
+  if (blockIdx.x == 0 && !dense) {
+    if (by_lane) {
+      if (tid < n) p.seq_prefix[tid + 1] = upto;
+      if (tid == 0) p.seq_prefix[0] = 0;
+    } else {
+      for (int s = tid; s <= n; s += blockDim.x) p.seq_prefix[s] = s_prefix[s];
+    }
   }
-  if (blockIdx.x >= wgs) return;  // whole workgroup: no barrier follows for it
-  const int64_t lo = static_cast<int64_t>(blockIdx.x) * total / wgs;
-  const int64_t hi = (static_cast<int64_t>(blockIdx.x) + 1) * total / wgs;
-  if (lo >= hi) return;  // whole workgroup: no barrier follows for it
+  if (static_cast<int>(blockIdx.x) >= shares.count) return;
+  const int lo = shares.begin(blockIdx.x);
+  const int hi = shares.begin(blockIdx.x + 1);
+  if (lo >= hi) return;
 
   const int wave = tid / kWave;
   const int lane = tid % kWave;
@@ -396,27 +491,33 @@ __global__ __launch_bounds__(512) void paged_decode_stream_kernel(const PagedPar
   const bool active = wave_unit<GC>(p, wave, kvh, h0);
   const float score_scale = p.scale * kLog2e;
 
-  // First sequence whose keys include `lo`: the last s with prefix[s] <= lo.
-  int a = 0, b = n;  // invariant: prefix[a] <= lo < prefix[b]
-  while (b - a > 1) {
-    const int mid = (a + b) >> 1;
-    if (s_prefix[mid] <= lo) a = mid; else b = mid;
+  // First sequence whose keys include `lo`: the last s with prefix[s] <= lo < prefix[s + 1].
+  int seq = 0;
+  if (dense) {
+    seq = static_cast<int>(static_cast<uint32_t>(lo) / static_cast<uint32_t>(p.dense_keys));
+  } else if (by_lane) {
+    seq = __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto > lo));
+  } else {
+    int b = n;  // invariant: prefix[seq] <= lo < prefix[b]
+    while (b - seq > 1) {
+      const int mid = (seq + b) >> 1;
+      if (prefix(mid) <= lo) seq = mid; else b = mid;
+    }
   }
-  int seq = a;
-  int64_t pos = lo;
+  int pos = lo;
   while (pos < hi) {
-    while (s_prefix[seq + 1] == s_prefix[seq]) ++seq;  // skip prefill / empty sequences
-    const int base = s_prefix[seq];
-    const int ctx = s_prefix[seq + 1] - base;
-    const int sb = static_cast<int>(pos - base);
-    const int se = static_cast<int>(min(hi, static_cast<int64_t>(s_prefix[seq + 1])) - base);
+    while (prefix(seq + 1) == prefix(seq)) ++seq;  // skip prefill / empty sequences
+    const int base = prefix(seq);
+    const int ctx = prefix(seq + 1) - base;
+    const int sb = pos - base;
+    const int se = min(hi, base + ctx) - base;
     // A decode-only batch (the fresh-token stream) has row s for sequence s: no load
     // ahead of the raw q/k/v reads that address by row.
-    const int row = kFresh ? seq : p.cu_seqlens_q[seq];
+    const int row = kFresh || dense ? seq : p.cu_seqlens_q[seq];
     const bool whole = sb == 0 && se == ctx;
     typename K::State st;
     if (active) {
-      float qf[GC][K::E];
+      typename K::Q qf[GC];
       K::init(st);
       const int32_t* table = p.block_tables + static_cast<int64_t>(seq) * p.max_blocks;
       if constexpr (kFresh) {
@@ -482,8 +583,8 @@ __global__ __launch_bounds__(512) void paged_decode_stream_kernel(const PagedPar
           };
 #pragma unroll
           for (int h = 0; h < GC; ++h) {
-            // rounded to TQ as the unfused kernel stores q, widened as the attention loads it
-            Chunk<TQ>::unpack(row_of(h), qf[h]);
+            // rounded to TQ as the unfused kernel stores q
+            qf[h].set(0, row_of(h));
           }
           fresh.k = row_of(GC);
           fresh.v = vraw;
@@ -500,16 +601,17 @@ __global__ __launch_bounds__(512) void paged_decode_stream_kernel(const PagedPar
             }
           }
         };
-        K::template stream_with<true>(p, table, nullptr, 0, kvh, sb, se, g, r, qf, score_scale,
+        K::template stream_with<true>(p, table, 0, nullptr, 0, kvh, sb, se, g, r, qf, score_scale,
                                       st, prep, fresh);
       } else {
-        K::template load_queries<TQ>(p, row, h0, r, qf);
-        K::stream(p, table, nullptr, 0, kvh, sb, se, g, r, qf, score_scale, st);
+        K::load_queries(p, row, h0, r, qf);
+        K::stream(p, dense ? nullptr : table, seq * p.dense_slots, nullptr, 0, kvh, sb, se, g, r, qf,
+                  score_scale, st);
       }
       K::merge_row_groups(st);
       if (g == 0) {
         if (whole) {
-          K::template write_output<TQ>(p, row, h0, r, st);
+          K::write_output(p, row, h0, r, st);
         } else {
           K::write_partial(p, (static_cast<int64_t>(blockIdx.x) + seq) * p.hq + h0, 1, r, st);
         }
@@ -523,7 +625,7 @@ __global__ __launch_bounds__(512) void paged_decode_stream_kernel(const PagedPar
 // Combine the pieces of every decode sequence cut between stream workgroups. Piece i
 // of sequence s lives in slot (first + i + s), first/last being the workgroups owning
 // the sequence's first and last key. Grid (sequence, block of kMergeCols float4
-// columns of its H_q x D output); in a workgroup, kMergeGroups groups of threads take
+// columns of its H_q x D output, 512 / kMergeGroups); in a workgroup, kMergeGroups groups of threads take
 // the pieces round robin (group g: pieces g, g + G, ...), each thread folding its
 // pieces for one float4 column online (running max, rescaled sums) with kMergeBatch
 // pieces' loads in flight at once; the groups' states then meet in LDS and are folded
@@ -531,27 +633,27 @@ __global__ __launch_bounds__(512) void paged_decode_stream_kernel(const PagedPar
 // instead of one per eight pieces, and a batch's sequences spread over H_q D / 4 /
 // kMergeCols workgroups each instead of one. The fold order depends on the piece count
 // alone, so a call's result does not depend on timing.
-constexpr int kMergeCols = 128;
-constexpr int kMergeGroups = 4;
+constexpr int kMergeThreads = 512;
 constexpr int kMergeBatch = 8;
 
-template <typename TQ, int D>
-__global__ __launch_bounds__(kMergeCols * kMergeGroups) void paged_decode_stream_merge_kernel(
+template <typename TQ, int D, int kMergeGroups>
+__global__ __launch_bounds__(kMergeThreads) void paged_decode_stream_merge_kernel(
     const PagedParams p, int wgs_i) {
+  constexpr int kMergeCols = kMergeThreads / kMergeGroups;
   __shared__ float s_m[kMergeGroups][kMergeCols];
   __shared__ float s_l[kMergeGroups][kMergeCols];
   __shared__ f32x4 s_o[kMergeGroups][kMergeCols];
   const int seq = blockIdx.x;
-  const int64_t total = p.seq_prefix[p.num_seqs];
-  const int64_t wgs = decode_stream_shares(total, wgs_i);
-  const int64_t begin = p.seq_prefix[seq];
-  const int64_t end = p.seq_prefix[seq + 1];
-  if (end == begin || total == 0) return;  // whole workgroup: no barrier follows for it
-  const int64_t first = share_owner(begin, total, wgs);
-  const int64_t last = share_owner(end - 1, total, wgs);
+  const bool dense = p.dense_keys > 0;
+  const int total = dense ? p.num_seqs * p.dense_keys : p.seq_prefix[p.num_seqs];
+  const int begin = dense ? seq * p.dense_keys : p.seq_prefix[seq];
+  const int end = dense ? begin + p.dense_keys : p.seq_prefix[seq + 1];
+  if (end == begin) return;  // whole workgroup: no barrier follows for it
+  const DecodeShares shares(total, wgs_i, p.stream_min_keys);
+  const int first = shares.owner(begin);
+  const int last = shares.owner(end - 1);
   if (first == last) return;  // one piece: the decode kernel stored the output
-  const bool all_live = total >= wgs;
-  const int pieces = static_cast<int>(last - first + 1);
+  const int pieces = last - first + 1;
   const int n4 = p.hq * D / 4;
   const int local = threadIdx.x % kMergeCols;
   const int grp = threadIdx.x / kMergeCols;
@@ -569,7 +671,7 @@ __global__ __launch_bounds__(kMergeCols * kMergeGroups) void paged_decode_stream
 #pragma unroll
       for (int u = 0; u < kMergeBatch; ++u) {
         const int i = min(i0 + u * kMergeGroups, pieces - 1);
-        const int64_t pidx = (first + i + seq) * p.hq + head;
+        const int64_t pidx = static_cast<int64_t>(first + i + seq) * p.hq + head;
         mi[u] = p.part_ml[pidx * 2];
         li[u] = p.part_ml[pidx * 2 + 1];
         oi[u] = *reinterpret_cast<const f32x4*>(p.part_o + pidx * D + d);
@@ -577,9 +679,7 @@ __global__ __launch_bounds__(kMergeCols * kMergeGroups) void paged_decode_stream
 #pragma unroll
       for (int u = 0; u < kMergeBatch; ++u) {
         const int i = i0 + u * kMergeGroups;
-        // Beyond the last piece, or a workgroup whose share was empty (fewer keys
-        // than workgroups): it wrote nothing and contributes nothing.
-        if (i >= pieces || !(all_live || share_nonempty(first + i, total, wgs))) continue;
+        if (i >= pieces) continue;  // (a share is never empty: see DecodeShares)
         const float mn = fmaxf(m, mi[u]);
         const float mu = mn == -INFINITY ? 0.0f : mn;
         const float a = fast_exp2(m - mu);
@@ -610,7 +710,7 @@ __global__ __launch_bounds__(kMergeCols * kMergeGroups) void paged_decode_stream
     m = mn;
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  const int row = p.cu_seqlens_q[seq];
+  const int row = dense ? seq : p.cu_seqlens_q[seq];
   const int64_t obase = (static_cast<int64_t>(row) * p.hq + head) * D + d;
 #pragma unroll
   for (int k = 0; k < 4; ++k) Elem<TQ>::store(p.out, obase + k, o[k] * inv);
@@ -620,7 +720,7 @@ __global__ __launch_bounds__(kMergeCols * kMergeGroups) void paged_decode_stream
 
 template <typename TQ, typename TKV, int D, int GC>
 __global__ __launch_bounds__(512) void paged_decode_grid_kernel(const PagedParams p) {
-  using K = Decode<TKV, D, GC>;
+  using K = Decode<TQ, TKV, D, GC>;
   __shared__ int s_pages[kMaxSplitPages];
 
   int seq, row, visible;
@@ -651,16 +751,16 @@ __global__ __launch_bounds__(512) void paged_decode_grid_kernel(const PagedParam
   int kvh, h0;
   if (!wave_unit<GC>(p, blockIdx.z * (blockDim.x / kWave) + wave, kvh, h0)) return;
 
-  float qf[GC][K::E];
-  K::template load_queries<TQ>(p, row, h0, r, qf);
+  typename K::Q qf[GC];
+  K::load_queries(p, row, h0, r, qf);
   typename K::State st;
   K::init(st);
-  K::stream(p, table, pages_in_lds ? s_pages : nullptr, first_page, kvh, sb, se, g, r, qf,
+  K::stream(p, table, 0, pages_in_lds ? s_pages : nullptr, first_page, kvh, sb, se, g, r, qf,
             p.scale * kLog2e, st);
   K::merge_row_groups(st);
   if (g != 0) return;
   if (nsplit == 1) {
-    K::template write_output<TQ>(p, row, h0, r, st);
+    K::write_output(p, row, h0, r, st);
   } else {
     K::write_partial(p, (static_cast<int64_t>(partial_row) * p.hq + h0) * p.max_splits + split,
                      p.max_splits, r, st);
@@ -729,12 +829,23 @@ int decode_waves(const PagedParams& p, int gc) {
   return units < 8 ? units : 8;
 }
 
+// From this many workgroups per sequence on (so about as many pieces) 16 thread groups of
+// 32 columns share a sequence's pieces instead of four of 128: one 8192-key sequence 20.4 ->
+// 17.4 us a call, 8 of 300-2300 keys level, 16 of 1024 (16 pieces) 19.1 -> 20.0.
+constexpr int kWideMergePieces = 32;
+
 template <typename TQ, int D>
 hipError_t launch_stream_merge(const PagedParams& p, hipStream_t stream) {
   const int n4 = p.hq * D / 4;
-  const dim3 mgrid(p.num_seqs, (n4 + kMergeCols - 1) / kMergeCols);
-  paged_decode_stream_merge_kernel<TQ, D>
-      <<<mgrid, kMergeCols * kMergeGroups, 0, stream>>>(p, p.stream_wgs);
+  auto grid = [&](int groups) {
+    const int cols = kMergeThreads / groups;
+    return dim3(p.num_seqs, (n4 + cols - 1) / cols);
+  };
+  if (p.stream_wgs >= kWideMergePieces * p.num_seqs) {
+    paged_decode_stream_merge_kernel<TQ, D, 16><<<grid(16), kMergeThreads, 0, stream>>>(p, p.stream_wgs);
+  } else {
+    paged_decode_stream_merge_kernel<TQ, D, 4><<<grid(4), kMergeThreads, 0, stream>>>(p, p.stream_wgs);
+  }
   return hipGetLastError();
 }
 

@@ -285,19 +285,6 @@ __device__ __forceinline__ bool prefill_work(const PagedParams& p, int cols, int
   return true;
 }
 
-// Inclusive prefix sum over the wave's 64 lanes: DPP row shifts 1, 2, 4, 8 (within
-// each 16-lane row; a lane whose source lies outside its row adds 0), then lane 15's
-// row total broadcast into rows 1 and 3 and lane 31's into rows 2 and 3.
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-  return v;
-}
-
 // A piece of the pair kernel's work: key tiles [tb, te) of query tile q (of kPairQueryTile
 // positions) of sequence s, the `piece`th of the item's `pieces`, its partial in slot
 // slot0 + piece when there are several.

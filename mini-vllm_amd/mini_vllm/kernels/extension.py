@@ -20,11 +20,14 @@ from __future__ import annotations
 
 import ctypes
 import hashlib
+import importlib.machinery
+import importlib.util
 import math
 import os
 import struct
 import subprocess
 import sys
+import sysconfig
 import threading
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -39,6 +42,8 @@ LIB_DIR = PACKAGE_ROOT / "lib"
 # MVLLM_LIBRARY points the loader at another build of the same library (variant builds
 # for measurements); the default is the in-tree build.
 LIB_PATH = Path(os.environ.get("MVLLM_LIBRARY") or LIB_DIR / "libminivllm_hip.so")
+HOST_SOURCE = CSRC_DIR / "host" / "host.cpp"
+HOST_PATH = LIB_DIR / "mvllm_host.so"
 REPO_ROOT = PACKAGE_ROOT.parent
 INCLUDE_DIR = REPO_ROOT / "include"
 
@@ -68,6 +73,11 @@ EXTRA_FLAGS = {"elementwise.hip": ["-ffp-contract=off"], "linear.hip": ["-ffp-co
 # hipBLASLt (csrc/blas.hip). Its soname is the one torch's bundled copy carries, so in a
 # process that has imported torch the library binds to that copy.
 LINK_LIBS = ["-L/opt/rocm/lib", "-lhipblaslt"]
+
+# The host module: plain C++ against torch's headers (hipified, so its stream header wants
+# the platform named).
+CXX = os.environ.get("CXX", "g++")
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
 
 ABI_VERSION = 16
 
@@ -111,8 +121,53 @@ def source_hash() -> str | None:
     return h.hexdigest()[:16]
 
 
+def host_hash() -> str | None:
+    """The identity of the host module's source (:data:`HOST_SOURCE`), the C headers it
+    calls by and the torch it is built against; None where the sources are not there."""
+    if not HOST_SOURCE.exists():
+        return None
+    h = hashlib.sha256(repr((HOST_FLAGS, torch.__version__, sys.version_info[:2])).encode())
+    for f in [HOST_SOURCE, *sorted(INCLUDE_DIR.glob("*.h"))]:
+        h.update(f.name.encode() + b"\0" + f.read_bytes() + b"\0")
+    return h.hexdigest()[:16]
+
+
+def build_host() -> Path:
+    """Compile ``csrc/host/host.cpp`` (no device code) against torch into ``lib/``."""
+    include = Path(torch.__file__).resolve().parent / "include"
+    lib = include.parent / "lib"
+    tmp = HOST_PATH.with_suffix(f".so.tmp{os.getpid()}")
+    cmd = [CXX, *HOST_FLAGS, f'-DMVLLM_SOURCE_HASH="{host_hash()}"',
+           f"-I{INCLUDE_DIR}", f"-I{include}", f"-I{include}/torch/csrc/api/include",
+           "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", str(HOST_SOURCE),
+           "-o", str(tmp), f"-L{lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-ltorch_python"]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise ToolchainError(f"{CXX} failed on {HOST_SOURCE.name}:\n{result.stderr}{result.stdout}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
+def open_host():
+    """The host module (``csrc/host/host.cpp``), or None where it is not built: the ops'
+    Python bodies then do its work. One built from other sources is refused."""
+    if not HOST_PATH.exists():
+        return None
+    loader = importlib.machinery.ExtensionFileLoader("mvllm_host", str(HOST_PATH))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mvllm_host", loader))
+    loader.exec_module(module)
+    current = host_hash()
+    if current is not None and module.source_hash != current:
+        raise ToolchainError(f"{HOST_PATH} was built from other sources or for another torch "
+                             f"(build id {module.source_hash}, sources {current}); rebuild it: "
+                             "__graft_entry__.build()")
+    return module
+
+
 def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
-    """Compile every ``csrc/*.hip`` for gfx950 and link ``lib/libminivllm_hip.so``.
+    """Compile every ``csrc/*.hip`` for gfx950 and link ``lib/libminivllm_hip.so``, and
+    build the host module beside it.
 
     Always compiles (this is the "does it build" check); objects go to ``_build/``
     and the library is replaced atomically so a running process never maps a
@@ -140,7 +195,10 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
 
     workers = jobs or min(8, os.cpu_count() or 4)
     with ThreadPoolExecutor(max_workers=workers) as pool:
+        host = pool.submit(build_host) if HOST_SOURCE.exists() else None
         objects = list(pool.map(compile_one, sources()))
+        if host is not None:
+            host.result()
 
     tmp = LIB_PATH.with_suffix(f".so.tmp{os.getpid()}")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), *LINK_LIBS,
@@ -427,6 +485,36 @@ class HipExtension:
         self.path = LIB_PATH
         self._workspaces: dict[tuple[int, int], torch.Tensor] = {}
         self._recording: list[torch.Tensor] | None = None
+        self._host = open_host()
+        self._entries = None if self._host is None else self._host.entries(*(
+            ctypes.cast(f, ctypes.c_void_p).value for f in (
+                lib.mvllm_paged_attention_plan, lib.mvllm_paged_attention,
+                lib.mvllm_paged_decode_qk_norm_rope, lib.mvllm_linear_workspace_bytes,
+                lib.mvllm_linear_swiglu, lib.mvllm_linear_residual_rmsnorm,
+                lib.mvllm_last_error)))
+
+    # The ops below in native code (csrc/host/host.cpp): the result, or None where the call
+    # is not one that it serves as it stands and the Python body has to look at it. Their
+    # launches' workspaces are only recorded by the Python bodies (:meth:`workspace`), which
+    # therefore serve every call under :meth:`recording_workspaces`.
+    def paged_served(self, *args) -> bool:
+        """Whether ``paged_attention(*args)`` would pass every check (False: unknown)."""
+        return self._host is not None and self._host.paged_served(*args)
+
+    def try_linear_swiglu(self, x: torch.Tensor, w_packed: torch.Tensor, n: int):
+        if self._host is None or self._recording is not None:
+            return None
+        return self._host.linear_swiglu(self._entries, self._workspaces, x, w_packed, n)
+
+    def try_linear_residual_rmsnorm(self, *args):
+        if self._host is None or self._recording is not None:
+            return None
+        return self._host.linear_residual_rmsnorm(self._entries, self._workspaces, *args)
+
+    def try_paged_decode_qk_norm_rope(self, *args):
+        if self._host is None or self._recording is not None:
+            return None
+        return self._host.paged_decode_qk_norm_rope(self._entries, self._workspaces, *args)
 
     def workspace(self, device: torch.device, nbytes: int) -> torch.Tensor:
         """The kernels' workspace of (device, current stream), grown on demand (paged and
@@ -1396,6 +1484,14 @@ class HipExtension:
         ``out`` to write into a caller-owned ``T x H_q x D`` tensor, and ``plan_options``
         (``mvllm_plan_options`` fields by name) to force a schedule.
         """
+        if (self._host is not None and self._recording is None and out is None
+                and plan_options is None):
+            served = self._host.paged_attention(
+                self._entries, self._workspaces, q, key_pool, value_pool, block_tables,
+                cu_seqlens_q, context_lens, seq_lens, max_query_len, max_context_len, scale,
+                k_scale, v_scale)
+            if served is not None:
+                return served
         cu_seqlens_q, context_lens, seq_lens = self._paged_checks(
             q, key_pool, value_pool, block_tables, cu_seqlens_q, context_lens, seq_lens,
             max_query_len, max_context_len, k_scale, v_scale)

@@ -321,6 +321,11 @@ def paged_decode_qk_norm_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if not _use_kernel("paged_attention", use_cuda, q):
         return None
     ext = load_extension()
+    served = ext.try_paged_decode_qk_norm_rope(
+        q, k, v, q_weight, k_weight, cos, sin, eps, key_pool, value_pool, block_tables,
+        cu_seqlens_q, context_lens, seq_lens, max_context_len, scale)
+    if served is not None:
+        return served
     if (q.dim() != 3 or k.dtype != q.dtype or v.dtype != q.dtype or q_weight.dtype != q.dtype
             or k_weight.dtype != q.dtype or value_pool.dtype != q.dtype
             or _rope_reason(q, cos, sin) is not None or not key_pool.is_contiguous()
@@ -496,6 +501,11 @@ def linear_residual_rmsnorm(x: torch.Tensor, w: PackedWeight, residual: torch.Te
     reduction that adds the residual and normalises). None where the kernel does not
     serve the shape (K <= 1024, N not a multiple of 512, ...): the caller runs the two
     ops. Not dispatched on the PyTorch path either (None)."""
+    if x.is_cuda and _use_kernel("linear", use_cuda, x) and isinstance(w, PackedWeight):
+        served = load_extension().try_linear_residual_rmsnorm(
+            x, w.packed, w.shape[0], residual, norm_weight, eps)
+        if served is not None:
+            return served
     ext = _skinny_ext(x, w, w.shape[0], use_cuda)
     if (ext is None or not ext.linear_residual_rmsnorm_supported(x, w.shape[0])
             or not residual.is_contiguous() or residual.dtype != x.dtype
@@ -508,6 +518,10 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: PackedWeight, use_cuda: bool = Fal
     """``swiglu(x @ gate.T, x @ up.T)`` over ``torch_path.interleave_gate_up(gate, up)``.
     Kernel: ``csrc/linear.hip``."""
     n = w_gate_up.shape[0]
+    if x.is_cuda and _use_kernel("linear", use_cuda, x) and isinstance(w_gate_up, PackedWeight):
+        served = load_extension().try_linear_swiglu(x, w_gate_up.packed, n)
+        if served is not None:
+            return served
     ext = _skinny_ext(x, w_gate_up, n, use_cuda)
     if ext is not None and n % 32 == 0:
         return ext.linear_swiglu(x, w_gate_up.packed, n // 2)
@@ -606,9 +620,11 @@ def paged_attention(
     """
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
-    if _use_kernel("paged_attention", use_cuda, q) and _served(
+    if _use_kernel("paged_attention", use_cuda, q) and (load_extension().paged_served(
+            q, key_pool, value_pool, block_tables, cu_seqlens_q, context_lens, seq_lens,
+            max_query_len, max_context_len, scale, k_scale, v_scale) or _served(
             "paged_attention", _kernel_can_page(q, key_pool, value_pool, block_tables,
-                                                (cu_seqlens_q, context_lens, seq_lens))):
+                                                (cu_seqlens_q, context_lens, seq_lens)))):
         return load_extension().paged_attention(
             q, key_pool, value_pool, block_tables, cu_seqlens_q, context_lens, seq_lens,
             int(max_query_len), int(max_context_len), scale, k_scale, v_scale,

@@ -9,8 +9,8 @@
 // from the row's maximum finds the bin it lies in, and an exact selection among that
 // bin's few tokens finds the token.
 //
-// Four launches, a workgroup per (row, segment of 16384 logits) in each, so a single row
-// already runs on ten CUs of a 151936-entry vocabulary:
+// Four launches, a workgroup per (row, segment of 4096 to 16384 logits, see segment_of) in
+// each, so a single row already runs on nineteen CUs of a 151936-entry vocabulary:
 //   max      the segment's largest logit and its index (argmax_key order: NaN highest)
 //   mass     exp(x - max) of every token summed into 512 bins of 1/32 nat (LDS atomics)
 //            with, for top-k rows, the bins' token counts; rows that do not truncate
@@ -46,7 +46,7 @@ namespace {
 
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / kWave;
-constexpr int64_t kSegment = 16384;
+constexpr int kLongestSegment = 16384;
 constexpr int kMaxSegments = 64;
 constexpr int kBins = kThreads;      // one per thread in the scans
 constexpr float kBinsPerNat = 32.0f;
@@ -130,10 +130,10 @@ __device__ __forceinline__ uint64_t block_exclusive_scan64(uint64_t v, uint64_t*
 }
 
 // f(index, logit) over this thread's elements of the segment [lo, hi) of a row. kVec: 16-byte
-// chunks (rows 16-byte aligned; kSegment is a whole number of chunks), a thread's loads
+// chunks (rows 16-byte aligned; a segment is a whole number of chunks), a thread's loads
 // issued together; the elements past the last whole chunk, and every element otherwise,
 // one by one.
-template <typename T, bool kVec, typename F>
+template <typename T, bool kVec, int kSegment, typename F>
 __device__ __forceinline__ void for_each(const T* row, int64_t lo, int64_t hi, F f) {
   constexpr int kPer = 16 / sizeof(T);
   int64_t done = lo;
@@ -211,14 +211,14 @@ __device__ __forceinline__ bool keeps(uint64_t count_before, uint64_t mass_befor
   return count_before < static_cast<uint64_t>(k) && static_cast<double>(mass_before) < limit;
 }
 
-template <typename T, bool kVec>
+template <typename T, bool kVec, int kSegment>
 __global__ __launch_bounds__(kThreads) void sampling_max_kernel(const Work w, const T* logits,
                                                                int64_t v, int64_t row_stride) {
   __shared__ uint64_t lds[kWaves];
   const T* row = logits + static_cast<int64_t>(blockIdx.x) * row_stride;
-  const int64_t lo = blockIdx.y * kSegment, hi = min(v, lo + kSegment);
+  const int64_t lo = static_cast<int64_t>(blockIdx.y) * kSegment, hi = min(v, lo + kSegment);
   uint64_t best = 0;
-  for_each<T, kVec>(row, lo, hi, [&](int64_t i, float x) __attribute__((always_inline)) {
+  for_each<T, kVec, kSegment>(row, lo, hi, [&](int64_t i, float x) __attribute__((always_inline)) {
     const uint64_t key = x != x ? 0xffffffffu : order_key(x);
     const uint64_t mine = (key << 32) | (0xffffffffu - static_cast<uint32_t>(i));
     best = best > mine ? best : mine;
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void sampling_max_kernel(const Work w, co
   if (threadIdx.x == 0) w.keys[blockIdx.x * gridDim.y + blockIdx.y] = best;
 }
 
-template <typename T, bool kVec>
+template <typename T, bool kVec, int kSegment>
 __global__ __launch_bounds__(kThreads) void sampling_mass_kernel(const Rows rows, const Work w,
                                                                 const T* logits, int64_t v,
                                                                 int64_t row_stride, float unit) {
@@ -243,11 +243,11 @@ __global__ __launch_bounds__(kThreads) void sampling_mass_kernel(const Rows rows
   const RowState s = row_state(rows.row[r], w, r, segments, v, lds);  // (has barriers)
   if (s.mode == kGreedy || !s.finite) return;
   const T* row = logits + static_cast<int64_t>(r) * row_stride;
-  const int64_t lo = seg * kSegment, hi = min(v, lo + kSegment);
+  const int64_t lo = static_cast<int64_t>(seg) * kSegment, hi = min(v, lo + kSegment);
   const int64_t cell = static_cast<int64_t>(r) * segments + seg;
   if (s.mode == kSoftmax) {
     uint64_t sum = 0;
-    for_each<T, kVec>(row, lo, hi, [&](int64_t, float l) __attribute__((always_inline)) {
+    for_each<T, kVec, kSegment>(row, lo, hi, [&](int64_t, float l) __attribute__((always_inline)) {
       sum += mass_of(expf(l / s.t - s.max), unit);
     });
     sum = block_sum64(sum, lds);
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kThreads) void sampling_mass_kernel(const Rows rows
   const bool counted = s.k != INT32_MAX;
   const int copy = threadIdx.x % kCopies;
   uint64_t tail = 0, tail_count = 0;
-  for_each<T, kVec>(row, lo, hi, [&](int64_t, float l) __attribute__((always_inline)) {
+  for_each<T, kVec, kSegment>(row, lo, hi, [&](int64_t, float l) __attribute__((always_inline)) {
     const float x = l / s.t;
     const int bin = bin_of(s.max, x);
     const uint64_t m = mass_of(expf(x - s.max), unit);
@@ -325,7 +325,7 @@ __device__ __forceinline__ Boundary find_boundary(const RowState& s, const Work&
   return b;
 }
 
-template <typename T, bool kVec>
+template <typename T, bool kVec, int kSegment>
 __global__ __launch_bounds__(kThreads) void sampling_gather_kernel(const Rows rows, const Work w,
                                                                   const T* logits, int64_t v,
                                                                   int64_t row_stride) {
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kThreads) void sampling_gather_kernel(const Rows ro
   if (s.mode != kTruncate || !s.finite) return;
   const Boundary b = find_boundary(s, w, r, segments, lds);
   const T* row = logits + static_cast<int64_t>(r) * row_stride;
-  const int64_t lo = seg * kSegment, hi = min(v, lo + kSegment);
+  const int64_t lo = static_cast<int64_t>(seg) * kSegment, hi = min(v, lo + kSegment);
   const int64_t cell = static_cast<int64_t>(r) * segments + seg;
   uint16_t* list = w.list + cell * kSegment;
   // The approximate distance d' = max - l * inv_t is within slack + d' * 1e-6 of the exact
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kThreads) void sampling_gather_kernel(const Rows ro
   const float near = static_cast<float>(b.bin) / kBinsPerNat * (1.0f - 1e-5f) - slack;
   const float far = b.bin == kBins - 1 ? INFINITY
                                        : static_cast<float>(b.bin + 1) / kBinsPerNat * (1.0f + 1e-5f) + slack;
-  for_each<T, kVec>(row, lo, hi, [&](int64_t i, float l) __attribute__((always_inline)) {
+  for_each<T, kVec, kSegment>(row, lo, hi, [&](int64_t i, float l) __attribute__((always_inline)) {
     const float d = s.max - l * s.inv_t;
     if (s.approx && !(d >= near && d <= far)) return;
     if (bin_of(s.max, l / s.t) == b.bin) {
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kThreads) void sampling_gather_kernel(const Rows ro
 // the boundary bin's listed tokens. While more than kThreads remain, a pass of eight
 // bits of the rank narrows them (the same rule over 256 bins); then each thread takes
 // one and compares it with all. Ranks are unique, so eight passes leave one token.
-template <typename T>
+template <typename T, int kSegment>
 __device__ __forceinline__ uint64_t select_last(const RowState& s, const Boundary& b,
                                                 const Work& w, const T* row, int r, int segments,
                                                 float unit, uint64_t* lds, uint64_t& kept_mass) {
@@ -469,7 +469,7 @@ __device__ __forceinline__ uint64_t select_last(const RowState& s, const Boundar
   return kept;
 }
 
-template <typename T, bool kVec>
+template <typename T, bool kVec, int kSegment>
 __global__ __launch_bounds__(kThreads) void sampling_write_kernel(const Rows rows, const Work w,
                                                                  float* __restrict__ probs,
                                                                  const T* logits, int64_t v,
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(kThreads) void sampling_write_kernel(const Rows row
   const RowState s = row_state(rows.row[r], w, r, segments, v, lds);
   const T* row = logits + static_cast<int64_t>(r) * row_stride;
   float* out = probs + static_cast<int64_t>(r) * v;
-  const int64_t lo = seg * kSegment, hi = min(v, lo + kSegment);
+  const int64_t lo = static_cast<int64_t>(seg) * kSegment, hi = min(v, lo + kSegment);
   uint64_t last = ~uint64_t{0};  // rank of the last kept token
   float sum = 1.0f;
   if (s.mode == kGreedy) {
@@ -496,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void sampling_write_kernel(const Rows row
   } else {
     const Boundary b = find_boundary(s, w, r, segments, lds);
     uint64_t kept_mass = 0;
-    last = select_last<T>(s, b, w, row, r, segments, unit, lds, kept_mass);
+    last = select_last<T, kSegment>(s, b, w, row, r, segments, unit, lds, kept_mass);
     sum = static_cast<float>(kept_mass) * inv_unit;
   }
   // Tokens whose approximate quotient is below the last kept value by more than the two can
@@ -552,12 +552,25 @@ __global__ __launch_bounds__(kThreads) void sampling_write_kernel(const Rows row
   }
 }
 
-int segments_of(int64_t v) { return static_cast<int>((v + kSegment - 1) / kSegment); }
+int segments_of(int64_t v, int segment) { return static_cast<int>((v + segment - 1) / segment); }
+
+// A row's segment length: shorter ones spread few rows over more CUs, but every workgroup
+// of a truncated row adds up the histograms of all its segments, so they pay only while all
+// workgroups run at once (256 CUs), and the shortest only for rows of up to eight of them.
+// Graph-replayed calls with 16384, 8192 and 4096: 8 rows of 151936 34.1, 31.4 and 43.7 us,
+// 16 rows 34.6, 39.7 and 53.2; 32 rows of 32000 32.0, 27.1 and 25.0, 64 rows 32.9, 28.1 and
+// 31.8, 128 rows 34.7, 35.3 and 50.5.
+int segment_of(int64_t rows, int64_t v) {
+  if (segments_of(v, 4096) <= 8 && rows * segments_of(v, 4096) <= 256) return 4096;
+  if (segments_of(v, 8192) <= kMaxSegments && rows * segments_of(v, 8192) <= 256) return 8192;
+  return kLongestSegment;
+}
+
 uint64_t align256(uint64_t n) { return (n + 255) / 256 * 256; }
 
 // The workspace's parts for `rows` rows; returns its size.
-uint64_t layout(int64_t rows, int64_t v, char* base, Work& w) {
-  const uint64_t cells = static_cast<uint64_t>(rows) * segments_of(v);
+uint64_t layout(int64_t rows, int64_t v, int segment, char* base, Work& w) {
+  const uint64_t cells = static_cast<uint64_t>(rows) * segments_of(v, segment);
   uint64_t at = 0;
   auto part = [&](uint64_t bytes) {
     char* p = base == nullptr ? nullptr : base + at;
@@ -569,37 +582,37 @@ uint64_t layout(int64_t rows, int64_t v, char* base, Work& w) {
   w.masses = reinterpret_cast<uint64_t*>(part(cells * kBins * 8));
   w.counts = reinterpret_cast<uint32_t*>(part(cells * kBins * 4));
   w.listed = reinterpret_cast<uint32_t*>(part(cells * 4));
-  w.list = reinterpret_cast<uint16_t*>(part(cells * kSegment * 2));
+  w.list = reinterpret_cast<uint16_t*>(part(cells * segment * 2));
   return at;
 }
 
-template <typename T, bool kVec>
+template <typename T, bool kVec, int kSegment>
 hipError_t launch(float* probs, const void* logits, int64_t v, int64_t row_stride,
                   const Rows& rows, int n, const Work& w, bool truncates, bool softmax,
                   hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(n), segments_of(v));
+  const dim3 grid(static_cast<unsigned>(n), segments_of(v, kSegment));
   const T* l = static_cast<const T*>(logits);
   int bits = 0;  // the least with 2^bits >= v: v maximal masses of 2^(62 - bits) sum to at most 2^62
   while ((int64_t{1} << bits) < v) ++bits;
   const float unit = static_cast<float>(uint64_t{1} << (62 - bits));
-  sampling_max_kernel<T, kVec><<<grid, kThreads, 0, stream>>>(w, l, v, row_stride);
+  sampling_max_kernel<T, kVec, kSegment><<<grid, kThreads, 0, stream>>>(w, l, v, row_stride);
   if (truncates || softmax) {
-    sampling_mass_kernel<T, kVec><<<grid, kThreads, 0, stream>>>(rows, w, l, v, row_stride, unit);
+    sampling_mass_kernel<T, kVec, kSegment><<<grid, kThreads, 0, stream>>>(rows, w, l, v, row_stride, unit);
   }
   if (truncates) {
-    sampling_gather_kernel<T, kVec><<<grid, kThreads, 0, stream>>>(rows, w, l, v, row_stride);
+    sampling_gather_kernel<T, kVec, kSegment><<<grid, kThreads, 0, stream>>>(rows, w, l, v, row_stride);
   }
-  sampling_write_kernel<T, kVec><<<grid, kThreads, 0, stream>>>(rows, w, probs, l, v, row_stride,
+  sampling_write_kernel<T, kVec, kSegment><<<grid, kThreads, 0, stream>>>(rows, w, probs, l, v, row_stride,
                                                                unit, 1.0f / unit);
   return hipGetLastError();
 }
 
-template <typename T>
+template <typename T, int kSegment>
 hipError_t launch_rows(float* probs, const void* logits, int64_t rows, int64_t v,
                        int64_t row_stride, const SamplingRow* params, void* workspace,
                        hipStream_t stream) {
   Work w;
-  layout(std::min<int64_t>(rows, kSamplingRows), v, static_cast<char*>(workspace), w);
+  layout(std::min<int64_t>(rows, kSamplingRows), v, kSegment, static_cast<char*>(workspace), w);
   const bool vec = reinterpret_cast<uintptr_t>(logits) % 16 == 0 &&
                    (row_stride * static_cast<int64_t>(sizeof(T))) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(probs) % 16 == 0 && v % 4 == 0;
@@ -618,21 +631,36 @@ hipError_t launch_rows(float* probs, const void* logits, int64_t rows, int64_t v
     const T* l = static_cast<const T*>(logits) + r0 * row_stride;
     float* out = probs + r0 * v;
     const hipError_t e =
-        vec ? launch<T, true>(out, l, v, row_stride, part, n, w, truncates, softmax, stream)
-            : launch<T, false>(out, l, v, row_stride, part, n, w, truncates, softmax, stream);
+        vec ? launch<T, true, kSegment>(out, l, v, row_stride, part, n, w, truncates, softmax, stream)
+            : launch<T, false, kSegment>(out, l, v, row_stride, part, n, w, truncates, softmax, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+template <typename T>
+hipError_t launch_segments(float* probs, const void* logits, int64_t rows, int64_t v,
+                           int64_t row_stride, const SamplingRow* params, void* workspace,
+                           hipStream_t stream) {
+  switch (segment_of(rows, v)) {
+    case 4096:
+      return launch_rows<T, 4096>(probs, logits, rows, v, row_stride, params, workspace, stream);
+    case 8192:
+      return launch_rows<T, 8192>(probs, logits, rows, v, row_stride, params, workspace, stream);
+    default:
+      return launch_rows<T, kLongestSegment>(probs, logits, rows, v, row_stride, params, workspace,
+                                             stream);
+  }
 }
 
 }  // namespace
 
 uint64_t sampling_workspace_bytes(int64_t rows, int64_t v) {
   Work w;
-  return layout(std::min<int64_t>(rows, kSamplingRows), v, nullptr, w);
+  return layout(std::min<int64_t>(rows, kSamplingRows), v, segment_of(rows, v), nullptr, w);
 }
 
-int64_t sampling_max_vocab() { return kSegment * kMaxSegments; }
+int64_t sampling_max_vocab() { return int64_t{kLongestSegment} * kMaxSegments; }
 
 hipError_t launch_sampling_probabilities(float* probs, const void* logits, int64_t rows,
                                          int64_t v, int64_t row_stride, int dtype,
@@ -640,11 +668,11 @@ hipError_t launch_sampling_probabilities(float* probs, const void* logits, int64
                                          hipStream_t stream) {
   switch (dtype) {
     case kF32:
-      return launch_rows<float>(probs, logits, rows, v, row_stride, params, workspace, stream);
+      return launch_segments<float>(probs, logits, rows, v, row_stride, params, workspace, stream);
     case kF16:
-      return launch_rows<f16_t>(probs, logits, rows, v, row_stride, params, workspace, stream);
+      return launch_segments<f16_t>(probs, logits, rows, v, row_stride, params, workspace, stream);
     case kBF16:
-      return launch_rows<bf16_t>(probs, logits, rows, v, row_stride, params, workspace, stream);
+      return launch_segments<bf16_t>(probs, logits, rows, v, row_stride, params, workspace, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -45,6 +45,16 @@ def test_matches_the_oracle(device, vocab, dtype):
     check(logits, PARAMS)
 
 
+@pytest.mark.parametrize("rows,vocab", [
+    (256, 4096), (257, 4096), (128, 4097), (7, 32768), (32, 32769), (51, 40960), (52, 40960),
+    (3, 524288), (4, 524289), (14, 151936)])
+def test_segment_lengths(device, rows, vocab):
+    """Both sides of each line where the segments' length changes, and of a segment's end."""
+    gen = torch.Generator(device=device).manual_seed(rows)
+    logits = torch.randn(rows, vocab, generator=gen, device=device) * 2.5
+    check(logits.to(torch.bfloat16), [PARAMS[i % len(PARAMS)] for i in range(rows)])
+
+
 @pytest.mark.parametrize("vocab", [700, 151936])
 def test_many_tokens_at_the_boundary(device, vocab):
     """Flat rows: every token in one bin, all equal (kept by index) or apart by less than

@@ -87,6 +87,10 @@ __host__ __device__ inline int decode_min_share_keys(int elem_bytes, int head_di
   const int keys = 256 * (16 / elem_bytes) / head_dim;
   return keys < 8 ? 8 : keys;
 }
+// MFMA prefill: log2 units a row's scores may pass its running max by before O is rescaled
+// (exponentials stay <= 2^8).
+constexpr float kRescaleSlack = 8.0f;
+
 constexpr int kMaxDecodeShares = 65535;  // DecodeShares' 32-bit products
 
 // The stream decode's shares: share w owns keys [begin(w), begin(w + 1)) of the `total` laid
@@ -181,6 +185,7 @@ struct PagedParams {
                             // fewest key tiles per piece
   int pf_register_staging;  // 1: the register-staged prefill kernel even where the
                             // direct-to-LDS one serves (a plan option, for measurement)
+  float pf_slack;     // pair prefill: log2 units a score may pass the running max by
   int pf_pieces;      // pair prefill: > 1 cuts long items into at most this many pieces (a
                       // 1-D grid of pf_ranks x columns); otherwise the (column,
                       // sequence, query tile) grid with every item whole

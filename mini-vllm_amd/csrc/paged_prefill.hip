@@ -60,7 +60,6 @@ namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kTileKeys = kPrefillKeyTile;
-constexpr float kRescaleSlack = 8.0f;  // log2 units: exponentials stay <= 2^8
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -1493,7 +1492,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
   };
   auto raise_max = [&](float raw) __attribute__((always_inline)) -> float {
     const float tmax = raw * score_c;
-    if (__builtin_amdgcn_ballot_w64(tmax > m_run + kRescaleSlack) != 0) {
+    if (__builtin_amdgcn_ballot_w64(tmax > m_run + p.pf_slack) != 0) {
       const float m_new = fmaxf(m_run, tmax);
       const float alpha = m_new == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;

@@ -501,7 +501,8 @@ def linear_residual_rmsnorm(x: torch.Tensor, w: PackedWeight, residual: torch.Te
     reduction that adds the residual and normalises). None where the kernel does not
     serve the shape (K <= 1024, N not a multiple of 512, ...): the caller runs the two
     ops. Not dispatched on the PyTorch path either (None)."""
-    if x.is_cuda and _use_kernel("linear", use_cuda, x) and isinstance(w, PackedWeight):
+    if (x.is_cuda and x.shape[0] <= 64  # (more rows are never the skinny kernels')
+            and _use_kernel("linear", use_cuda, x) and isinstance(w, PackedWeight)):
         served = load_extension().try_linear_residual_rmsnorm(
             x, w.packed, w.shape[0], residual, norm_weight, eps)
         if served is not None:
@@ -518,7 +519,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: PackedWeight, use_cuda: bool = Fal
     """``swiglu(x @ gate.T, x @ up.T)`` over ``torch_path.interleave_gate_up(gate, up)``.
     Kernel: ``csrc/linear.hip``."""
     n = w_gate_up.shape[0]
-    if x.is_cuda and _use_kernel("linear", use_cuda, x) and isinstance(w_gate_up, PackedWeight):
+    if (x.is_cuda and x.shape[0] <= 64
+            and _use_kernel("linear", use_cuda, x) and isinstance(w_gate_up, PackedWeight)):
         served = load_extension().try_linear_swiglu(x, w_gate_up.packed, n)
         if served is not None:
             return served

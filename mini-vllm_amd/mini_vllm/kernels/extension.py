@@ -75,9 +75,14 @@ EXTRA_FLAGS = {"elementwise.hip": ["-ffp-contract=off"], "linear.hip": ["-ffp-co
 LINK_LIBS = ["-L/opt/rocm/lib", "-lhipblaslt"]
 
 # The host module: plain C++ against torch's headers (hipified, so its stream header wants
-# the platform named).
+# the platform named). NDEBUG keeps out the headers' debug counter, a thread_local: a module
+# with thread-local storage, loaded late, sends every other library's accesses to theirs
+# through glibc's slow path (before 2.39) for good. With it a prefill's MLP of 81 to 600 rows, four
+# calls none of them the module's, took 55 us of host time, without it 49, as without the
+# module.
 CXX = os.environ.get("CXX", "g++")
-HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-DNDEBUG", "-D__HIP_PLATFORM_AMD__=1",
+              "-DUSE_ROCM=1"]
 
 ABI_VERSION = 16
 

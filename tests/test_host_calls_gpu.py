@@ -3,6 +3,7 @@ where both serve a call, and the Python body's answer or refusal everywhere else
 
 from __future__ import annotations
 
+import struct
 from contextlib import contextmanager
 
 import pytest
@@ -65,6 +66,18 @@ def test_the_built_module_matches_its_source():
     assert host.paged_served(*[x] * 12) is False
     with pytest.raises(ValueError):
         host.linear_swiglu(x, {}, x, x, 32)  # not the library's entries
+
+
+def test_the_module_has_no_thread_local_storage():
+    """A late-loaded module with a TLS segment slows every other library's thread-local
+    accesses (glibc before 2.39), and so every op that is not the module's."""
+    if not ext_module.HOST_PATH.exists():
+        pytest.skip("the host module is not built")
+    elf = ext_module.HOST_PATH.read_bytes()
+    at, = struct.unpack_from("<Q", elf, 32)  # the ELF64 header's e_phoff, e_phentsize, e_phnum
+    size, count = struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
 
 
 @gpu

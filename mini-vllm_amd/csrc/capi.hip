@@ -376,7 +376,6 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
   p.pf_register_staging = plan.register_staging;
   p.pf_share_tiles = plan.prefill_share_tiles;
   p.pf_cus = device_cus();
-  p.pf_slack = mvllm::kRescaleSlack;
   if (plan.pub.workspace_bytes > 0) {
     char* ws = static_cast<char*>(workspace);
     if (plan.pub.decode_mode == MVLLM_DECODE_STREAM) p.seq_prefix = reinterpret_cast<int*>(ws);
@@ -399,11 +398,6 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
         p.pf_pieces = 0;
       }
     }
-    // Whole items of a small launch follow the maximum exactly: its own weight, the largest,
-    // is then 1 and not rounded to 16 bits (float16, 100 tokens after 300 keys: 2.7e-4 and
-    // not 2.9e-4 against 64 bits); cut items get the same from their pieces, and on the grid
-    // the rescales would cost every tile.
-    if (plan.pub.prefill_workgroups > 0 && p.pf_pieces <= 1) p.pf_slack = 0.0f;
     if (p.pf_pieces > 1) {
       p.pf_ranks = plan.split_ranks;
       p.pf_slots = plan.split_slots;

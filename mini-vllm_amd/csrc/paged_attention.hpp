@@ -90,6 +90,19 @@ __host__ __device__ inline int decode_min_share_keys(int elem_bytes, int head_di
 // MFMA prefill: log2 units a row's scores may pass its running max by before O is rescaled
 // (exponentials stay <= 2^8).
 constexpr float kRescaleSlack = 8.0f;
+// Pair prefill: the tiles whose probabilities are taken against the tile's own maxima, so that
+// each query's largest one is 1 and not rounded to 16 bits: all of an item (or piece) of at
+// most kExactTiles, every kExactEvery'th of a longer one, half as often where the items fill
+// the chip. Each costs a rescale of O, 64 multiplies of a tile's ~400 vector cycles per wave:
+// 7% of a chip-filling launch (8 x 512 tokens after up to 1536 keys 57.3 -> 61.7 us, 2048 after
+// 14336 526 -> 563), hidden in a small one (100 tokens after 300 keys 13.3 -> 14.2, 512 after
+// 4000 42.6 -> 44.5). Errors against 64 bits without, with all, and as chosen, float16: 100
+// tokens after 300 keys 2.88e-4, 2.62e-4 and 2.62e-4; three of 300 after 700 2.91e-4,
+// 2.61e-4 and 2.79e-4; 512 after 4000 2.90e-4, 2.60e-4 and 2.83e-4 (cut
+// in one- to nine-tile pieces, as the launch before the pair kernel had them, 2.62e-4,
+// 2.84e-4 and 2.88e-4).
+constexpr int kExactTiles = 12;
+constexpr int kExactEvery = 4;
 
 constexpr int kMaxDecodeShares = 65535;  // DecodeShares' 32-bit products
 
@@ -185,7 +198,6 @@ struct PagedParams {
                             // fewest key tiles per piece
   int pf_register_staging;  // 1: the register-staged prefill kernel even where the
                             // direct-to-LDS one serves (a plan option, for measurement)
-  float pf_slack;     // pair prefill: log2 units a score may pass the running max by
   int pf_pieces;      // pair prefill: > 1 cuts long items into at most this many pieces (a
                       // 1-D grid of pf_ranks x columns); otherwise the (column,
                       // sequence, query tile) grid with every item whole

@@ -1446,6 +1446,9 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
 #pragma unroll
   for (int db = 0; db < kDBlocks; ++db) o[db] = f32x16{};
   float m_run = -INFINITY, l_run = 0.0f;
+  float m_top = -INFINITY;  // the largest score so far
+  const int exact_mask =    // tiles t & exact_mask == 0 are taken against their own maxima
+      te - tb <= kExactTiles ? 0 : p.pf_wgs > 0 ? kExactEvery - 1 : 2 * kExactEvery - 1;
   f32x16 sc0[2], sc1[2];  // scores of even / odd tiles
 
   // Fragment i of the K in buffer `par`: keys 32 (i % 2) .., dims 16 (i / 2) ..; fragments are
@@ -1490,10 +1493,16 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
     }
     return tmax;
   };
-  auto raise_max = [&](float raw) __attribute__((always_inline)) -> float {
+  auto raise_max = [&](int t, float raw) __attribute__((always_inline)) -> float {
     const float tmax = raw * score_c;
-    if (__builtin_amdgcn_ballot_w64(tmax > m_run + p.pf_slack) != 0) {
-      const float m_new = fmaxf(m_run, tmax);
+    float m_new = fmaxf(m_run, tmax);
+    bool change = tmax > m_run + kRescaleSlack;
+    m_top = fmaxf(m_top, tmax);
+    if ((t & exact_mask) == 0) {  // (but O is never kept more than 2^slack above its scale)
+      m_new = fmaxf(tmax, m_top - kRescaleSlack);
+      change = m_new != m_run;
+    }
+    if (__builtin_amdgcn_ballot_w64(change) != 0) {
       const float alpha = m_new == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
       l_run *= alpha;
@@ -1655,7 +1664,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
     stage_k(t + 2, pg1, par);
     __builtin_amdgcn_sched_barrier(0);
     if (t < w_nt) {
-      const float neg_mu = raise_max(row_max);
+      const float neg_mu = raise_max(t, row_max);
       float pf[2][16];
       float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       u32x4 pop[4];

@@ -72,3 +72,24 @@ def test_cut_items_of_many_sequences(extension, device):
 def test_the_default_cuts_a_lone_long_chunk(extension, device):
     """No options: 63 tokens after 6393 keys (8 items on 256 CUs)."""
     check(extension, [6456], [63], torch.bfloat16, None, None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("context,tokens", [(128, 64), (400, 100), (600, 61)])
+def test_whole_short_items_err_no_more_than_single_tiles(extension, device, dtype, context, tokens):
+    """An item of a few tiles run whole against one cut into single tiles, whose probabilities
+    are all taken against their tile's own maximum (the largest is 1 and not rounded): the
+    same products are rounded, so the error against 64 bits is the same but for which way
+    single outputs round (their share of the error's square is about 1 / sqrt(outputs), below
+    1%). Against one maximum per item it is 1.4% to 4% larger."""
+    b = build_batch([context], [tokens], dtype=dtype, num_q_heads=16, num_kv_heads=8,
+                    head_dim=128, seed=11, device="cuda")
+    ids = b.block_tables[0, : -(-context // 16)].long()
+    k, v = (p[ids].double().reshape(-1, 8, 128)[:context].repeat_interleave(2, dim=1).transpose(0, 1)
+            for p in (b.key_pool, b.value_pool))
+    scores = b.q.double().transpose(0, 1) @ k.transpose(1, 2).contiguous() * b.scale
+    hidden = torch.ones(tokens, context, dtype=torch.bool, device="cuda").triu(context - tokens + 1)
+    want = (scores.masked_fill(hidden, -torch.inf).softmax(dim=-1) @ v).transpose(0, 1)
+    whole, single = ((extension.paged_attention(*b.args(), plan_options=o).double() - want).norm()
+                     for o in (WHOLE, CUT))
+    assert whole <= 1.01 * single

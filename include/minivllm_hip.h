@@ -64,14 +64,20 @@ typedef struct mvllm_paged_plan {
   int32_t split_tokens;      /* grid modes: keys per split */
   int32_t prefill_mfma;      /* 1: prefill rows go to the MFMA prefill kernel */
   uint64_t workspace_bytes;  /* split partials and their index; 0 when none are needed */
-  int32_t prefill_workgroups; /* MFMA prefill: > 0 the stream schedule, balanced shares of
-                                 all key tiles for this many workgroups (cut items merged
-                                 after); 0 the grid, a workgroup per (sequence, heads,
-                                 query tile) */
-  int32_t prefill_pieces;     /* MFMA prefill on the grid: > 1 items longer than
-                                 prefill_piece_pct of the mean work per CU may be cut into
-                                 at most this many key ranges (merged after); 0 every item
-                                 whole */
+  int32_t prefill_workgroups; /* MFMA prefill: > 0 the stream schedule, work balanced over
+                                 this many workgroups; 0 the grid, a workgroup per
+                                 (sequence, heads, query tile). The GQA-pair kernel
+                                 (prefill_item > 0) runs either as the last two fields
+                                 say */
+  int32_t prefill_pieces;     /* MFMA prefill on the grid: > 1 the caller's or the default
+                                 limit to which items may be cut, with workspace for it;
+                                 whether they are is prefill_listed */
+  int32_t prefill_item;       /* GQA-pair prefill kernel (it takes positive scales): query
+                                 positions of a work item, 64 or 128; 0: another kernel */
+  int32_t prefill_listed;     /* GQA-pair prefill kernel: 0 the item grid; 1 whole items from
+                                 a list without the grid's holes; > 1 the list's items cut
+                                 into at most this many key ranges each, as their lengths
+                                 ask for, and merged after */
 } mvllm_paged_plan;
 
 /* Explicit overrides of the planner's schedule choices, for measurement and for tests
@@ -89,9 +95,10 @@ typedef struct mvllm_plan_options {
   int32_t prefill_staging;     /* 0 auto (direct-to-LDS copies where served); 1 forces the
                                   register-staged prefill kernel */
   int32_t prefill_share_tiles; /* stream prefill: fewest 64-key tiles per workgroup share
-                                  while a quarter of the workgroups stay busy; grid
-                                  prefill: fewest tiles per piece of a cut item
-                                  (default 4): small work uses fewer workgroups */
+                                  while a quarter of the workgroups stay busy; GQA-pair
+                                  kernel: fewest tiles per piece of a cut item (default
+                                  4; 2 over fp8 on the stream schedule): small work
+                                  uses fewer workgroups */
   int32_t prefill_pieces;      /* grid prefill: most key-range pieces per item (default
                                   8); 1 keeps every item whole */
   int32_t prefill_piece_pct;   /* grid prefill: an item is cut into pieces of at least this
@@ -100,11 +107,9 @@ typedef struct mvllm_plan_options {
 } mvllm_plan_options;
 
 /* Prefills whose plan cut items on the grid but that ran every item whole because their
- * stream was being captured into a graph (so a graph's result does not depend on how the
- * lengths at capture would have been cut). The merge of cut items is a launch of its own
- * over the caller's workspace: there are no arrival counters, so `regions_used` and
- * `whole_no_region`, which described them, are 0. No counterpart in the reference. Any
- * pointer may be NULL. */
+ * stream was being captured into a graph. `regions_used` and `whole_no_region` described
+ * arrival counters that the kernels no longer have: 0. No counterpart in the reference.
+ * Any pointer may be NULL. */
 void mvllm_split_stats(int32_t* regions_used, int64_t* whole_no_region,
                        int64_t* whole_capturing);
 

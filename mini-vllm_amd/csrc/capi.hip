@@ -74,6 +74,7 @@ struct Options {
   int prefill_share_tiles = mvllm::kPrefillShareTiles;
   int prefill_staging = 0;
   int prefill_pieces = mvllm::kSplitDefaultPieces;
+  bool share_tiles_given = false;
   bool pieces_given = false;  // prefill_pieces is the caller's, not the default
   int prefill_piece_pct = mvllm::kSplitDefaultPct;
 };
@@ -98,6 +99,7 @@ int read_options(const mvllm_plan_options* o, Options& out) {
   if (o->prefill_share_tiles > 0) out.prefill_share_tiles = o->prefill_share_tiles;
   out.prefill_staging = o->prefill_staging;
   if (o->prefill_pieces > 0) out.prefill_pieces = o->prefill_pieces;
+  out.share_tiles_given = o->prefill_share_tiles > 0;
   out.pieces_given = o->prefill_pieces > 0;
   if (o->prefill_piece_pct > 0) out.prefill_piece_pct = o->prefill_piece_pct;
   return MVLLM_OK;
@@ -161,14 +163,18 @@ struct Plan {
   uint64_t off_pf = 0;      // stream prefill: [prefix][O partials][(m, l) partials]
   uint64_t off_pf_o = 0;
   uint64_t off_pf_ml = 0;
-  // The pair prefill kernel's split schedule (paged_prefill.hip): pieces per item (<= 1:
-  // every item whole), rank extent, partial slots per column, piece length (percent of the
-  // mean tiles per workgroup of `split_wgs`); its slots and its ranks' records.
+  // The pair prefill kernel's launch (paged_prefill.hip): query positions of an item; 0 the
+  // item grid, else its schedule with at most that many pieces per item; rank extent, partial
+  // slots per column, piece length (percent of the mean tiles per workgroup of `split_wgs`);
+  // the slots and the ranks' records.
+  int split_tile = 64;
   int split_pieces = 0;
   int split_ranks = 0;
   int split_slots = 0;
   int split_pct = 0;
   int split_wgs = 0;
+  bool split_by_seq = false;  // whole items: a sequence's after another's
+  bool split_weigh = false;   // cut: the device may still leave the items whole
   uint64_t off_split = 0;
   uint64_t off_rec = 0;
 };
@@ -189,53 +195,126 @@ bool pair_prefill(int32_t hq, int32_t hk, int32_t d, int32_t block_size, int32_t
          (kv_dtype == q_dtype || kv_dtype == mvllm::kFP8E4M3);
 }
 
-// Whether the pair kernel should cut its items. With few items the longest, of n = max_ctx /
-// 64 tiles at 0.93 us each, sets the time while CUs idle; cut, the tiles spread over all CUs
-// at 1.25 us each (every CU then streams its own keys), for 13 us more of schedule, partials
-// and merge. Whole against cut: one 512-token chunk (64 items) fresh 15 and 24 us, after
-// 1000 keys 28.3 and 27.4, after 8000 126 and 57; 63 tokens after 6393 (8 items) 97 and 23;
-// 1024 tokens after 4000 (128 items) 77 and 70; two 512-token chunks after 1000 (128 items) 29
-// and 36. With more items than half the CUs an even batch is best whole; only a sequence
-// far longer than the others gains, which the host cannot see, so several sequences with
-// contexts past 96 tiles are cut where an item exceeds the piece length (a 2048-token chunk
-// after 6000 keys, where none does: 131 us whole, 144 through the schedule and the empty merge).
-bool pair_wants_split(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max_ctx, int cus) {
-  const int64_t wgs = static_cast<int64_t>((num_tokens + mvllm::kPairQueryTile - 1) /
-                                           mvllm::kPairQueryTile) * (hq / 2);
-  const int64_t n = (static_cast<int64_t>(max_ctx) + mvllm::kPrefillKeyTile - 1) / mvllm::kPrefillKeyTile;
-  if (2 * wgs > cus) return num_seqs > 1 && n > 96;
-  return n * (93 * cus - 125 * wgs) > 1300 * static_cast<int64_t>(cus);
+// Items of one column, at most: a sequence of L queries has ceil(L / tile).
+int64_t pair_items(int32_t num_tokens, int32_t num_seqs, int32_t max_q, int tile) {
+  const int64_t by_seqs = static_cast<int64_t>(num_seqs) * ((max_q + tile - 1) / tile);
+  const int64_t by_tokens = (static_cast<int64_t>(num_tokens) + tile - 1) / tile + num_seqs;
+  return by_seqs < by_tokens ? by_seqs : by_tokens;
 }
 
-// The split's extents over `wgs` workgroups' shares: ranks are the items' bound (a
-// sequence of L queries has ceil(L / 64) items) plus the extra pieces'. Left whole past
-// kSplitMaxRanks: each position is a workgroup, and one without a piece still costs ~4 ns.
-void plan_split(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max_q,
-                int wgs, int pct, int pieces) {
-  const int64_t q_tiles = (max_q + mvllm::kPairQueryTile - 1) / mvllm::kPairQueryTile;
-  const int64_t by_seqs = static_cast<int64_t>(num_seqs) * q_tiles;
-  const int64_t by_tokens =
-      (static_cast<int64_t>(num_tokens) + mvllm::kPairQueryTile - 1) / mvllm::kPairQueryTile + num_seqs;
-  const int64_t items = by_seqs < by_tokens ? by_seqs : by_tokens;
+// The schedule of items of `tile` positions in at most `pieces` pieces (1: whole), cut for
+// `wgs` workgroups' shares: ranks are the items' bound plus the extra pieces'. Left on the item
+// grid past kSplitMaxRanks: each position is a workgroup.
+void plan_ranked(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max_q, int tile,
+                 int wgs, int pct, int pieces) {
   const int cols = hq / 2;
-  const int64_t ranks = items + mvllm::split_extra_ranks(wgs, cols, pct);
+  int64_t ranks = pair_items(num_tokens, num_seqs, max_q, tile);
+  if (pieces > 1) ranks += mvllm::split_extra_ranks(wgs, cols, pct);
   if (ranks > mvllm::kSplitMaxRanks) return;
+  plan.split_tile = tile;
   plan.split_pieces = pieces;
   plan.split_ranks = static_cast<int>(ranks);
   plan.split_slots = mvllm::split_slots(wgs, cols, pct);
   plan.split_pct = pct;
   plan.split_wgs = wgs;
-  plan.off_split = align256(plan.pub.workspace_bytes);
-  plan.off_rec = align256(plan.off_split + static_cast<uint64_t>(plan.split_slots) * cols *
-                                               mvllm::kPairSlotFloats * sizeof(float));
-  plan.pub.workspace_bytes = plan.off_rec + align256(static_cast<uint64_t>(ranks) * 32);
+  plan.off_split = plan.off_rec = align256(plan.pub.workspace_bytes);
+  if (pieces > 1) {
+    plan.off_rec = align256(plan.off_split + static_cast<uint64_t>(plan.split_slots) * cols *
+                                                 mvllm::pair_slot_floats(tile) * sizeof(float));
+  }
+  if (pieces > 1) {
+    plan.pub.workspace_bytes = plan.off_rec + align256(static_cast<uint64_t>(ranks) * 32);
+  }
+}
+
+// A prefill's 64-query work items as far as host sizes tell: with T tokens in N sequences of at
+// most max_q, at least (T - N) / (max_q - 1) of them are chunks, the rest decode rows.
+struct PairWork {
+  int64_t chunks, tokens;
+  int64_t wgs;    // items of all columns
+  int64_t n;      // key tiles of the longest item, at most (a decode row's context may be longer)
+  int64_t tiles;  // of all items, with the longest's context
+};
+PairWork pair_work(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max_q, int32_t max_ctx) {
+  PairWork w{};
+  const int64_t beyond = static_cast<int64_t>(num_tokens) - num_seqs;
+  w.chunks = max_q > 1 && beyond > 0 ? (beyond + max_q - 2) / (max_q - 1) : 0;
+  w.tokens = w.chunks > 0 ? beyond + w.chunks : 0;
+  w.wgs = (w.tokens + 63) / 64 * (hq / 2);
+  w.n = (static_cast<int64_t>(max_ctx) + mvllm::kPrefillKeyTile - 1) / mvllm::kPrefillKeyTile;
+  w.tiles = w.wgs * (2 * w.n - max_q / 64) / 2;
+  return w;
+}
+
+// The pair kernel's query positions per item, and whether to cut the items.
+//
+// Half the CUs' worth of items and fewer: the longest, n tiles, sets the time while CUs idle;
+// cut, the tiles spread over all CUs (pair_costs: whole 0.93 us a tile and 1.55 over fp8,
+// cut 1.25 and 1.85 of the mean per CU, each CU then streaming its own keys, and 13 us for
+// partials and merge). Whole against cut: bf16, one 512-token chunk (64 items) fresh 17 and 27
+// us, after 1000 keys 32 and 30, after 12000 201 and 79; 64 tokens after 8000 (8) 132 and
+// 26; 1024 after 4000 (128) 85 and 72; fp8, 512 after 1000 46 and 35, 1024 after 4000 133 and 98.
+//   Cut items of 128 positions read K and V half as often and need half the merging, but
+// are half as many: with 20 tiles a CU on the mean (9 over fp8, whose conversion they halve as
+// well) they are ahead. 64 against 128: bf16, 512 after 4000 (17) 43 and 43, after 12000
+// (48) 79 and 72, 1024 after 12000 (98) 137 and 123; fp8, 512 after 1000 (5) 35 and 35,
+// after 4000 54 and 47, after 12000 111 and 82.
+// More items, up to one a CU: 128-position items, two or three pieces each, where contexts
+// are long. Whole and cut: bf16, 160 items of 64 up to 50 tiles 62 and 66, 176 up to 64 81 and 79,
+// 160 up to 84 96 and 83, 200 up to 88 95 and 107; fp8, 144 up to 34 68 and 60, 200 up to 25
+// 49 and 59, 232 up to 55 102 and 93, 256 up to 32 60 and 64, up to 126 205 and 167.
+// More still: whole. 128 positions over fp8 from one and a half a CU, but for chunks that
+// are long against their context (their items differ so much that fewer pair badly): 440 items
+// of 8 chunks 73 and 65 us, 400 of one fresh chunk of 1600 tokens 48 and 55.
+struct PairMode {
+  int tile;
+  bool cut;
+};
+PairMode pair_mode(const PairWork& w, int32_t num_seqs, int32_t hq, int32_t max_q, int32_t kv_dtype, int cus) {
+  const bool fp8 = kv_dtype == mvllm::kFP8E4M3;
+  // A grid of very many positions is halved (1500 decodes and 2048 tokens, 384K: 738 -> 700 us).
+  const bool vast = static_cast<int64_t>(num_seqs) * ((max_q + 63) / 64) * (hq / 2) >= 128 * 1024;
+  const PairMode whole{vast || (fp8 && 2 * w.wgs >= 3 * cus && max_q <= 32 * w.n) ? 128 : 64, false};
+  // Past 64 sequences the schedule is a launch of its own, and the list and the merge have a
+  // position per sequence and column: about 6 us and 1.5 ns each.
+  const int64_t n = w.n - (num_seqs > 64 ? 6 + static_cast<int64_t>(num_seqs) * hq / 1333 : 0);
+  if (w.wgs > cus) return whole;
+  if (2 * w.wgs > cus) {
+    const bool cut = fp8 ? n * cus >= 64 * (w.wgs - cus / 10) : 16 * w.wgs <= 11 * cus && n >= 64;
+    return cut ? PairMode{128, true} : whole;
+  }
+  const mvllm::PairCosts c = mvllm::pair_costs(64, fp8);
+  if (n * (c.whole * cus - c.cut * w.wgs) <= c.fixed * static_cast<int64_t>(cus)) return whole;
+  return PairMode{w.tiles >= (fp8 ? 9 : 20) * static_cast<int64_t>(cus) ? 128 : 64, true};
+}
+
+// Whole items: by the schedule where the item grid would be twice the live items or more (decode
+// rows, chunks shorter than the longest). Its empty workgroups leave at once, but the others
+// are then dealt two to a CU beside idle ones: 28 decodes and 1024 tokens after 4000 keys 157
+// us a call by the grid, 124 by the schedule; 28 decodes and 4 chunks of up to 512 after up to 4000
+// 220 and 116. Where the grid has few holes it is level or up to 2 us ahead, having nothing to
+// scan. Past one item a CU a sequence's items run one after another from contexts of 44 tiles
+// on, by the schedule in any case, so that they meet in the L2 (320 items of up to 84 tiles: 119
+// us and 130 with all sequences' last query tiles first, over fp8 156 and 168), before
+// that the longest of all first (440 of up to 27 tiles over fp8: 68 and 73).
+void plan_whole(Plan& plan, const PairWork& w, int32_t num_tokens, int32_t num_seqs, int32_t hq,
+                int32_t max_q, int tile, int cus) {
+  plan.split_tile = tile;
+  plan.split_pieces = 0;
+  const int64_t grid = static_cast<int64_t>(num_seqs) * ((max_q + tile - 1) / tile);
+  const int64_t live = (w.tokens + tile - 1) / tile + w.chunks / 2;
+  plan.split_by_seq = w.n >= 44;
+  if ((grid >= 2 * live || (w.wgs > cus && plan.split_by_seq && num_seqs > 1)) &&
+      num_seqs <= 64) {
+    plan_ranked(plan, num_tokens, num_seqs, hq, max_q, tile, cus, 100, 1);
+  }
 }
 
 // The MFMA prefill's schedule, from host sizes: the grid where its 128-query items, ceil(
 // num_tokens / 128) query tiles per kv column, reach half the CU count, the stream schedule
 // (balanced shares of all key tiles) below; the prefill_schedule option 1 / 2 forces
-// stream / grid. The pair kernel runs both as its item grid or, where pair_wants_split or
-// an option says so, cut into pieces; the other kernels run the stream as one persistent
+// stream / grid. The pair kernel runs either as pair_mode says: on the item grid, or by its own
+// schedule with the items whole or cut. The other kernels run the stream as one persistent
 // workgroup per CU (times the prefill_wgs_per_cu option), whose workspace follows the decode
 // part's (four 512-query chunks beside 28 decodes, 136 items: grid 102 us, stream 110 us;
 // one chunk of a long prompt, 40 items: stream 104 us, grid 109 us; 2.5-3x the grid at
@@ -249,19 +328,21 @@ void plan_prefill(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, 
   const int forced = o.prefill_schedule;
   const int cus = device_cus();
   const bool pair = pair_prefill(hq, hk, d, block_size, q_dtype, kv_dtype, o);
+  const PairWork work = pair_work(num_tokens, num_seqs, hq, max_q, max_ctx);
+  const PairMode m = pair_mode(work, num_seqs, hq, max_q, kv_dtype, cus);
   const int64_t qtiles = (static_cast<int64_t>(num_tokens) + mvllm::kPrefillQueryTile - 1) /
                          mvllm::kPrefillQueryTile;
   const int64_t items = qtiles * (hq / mvllm::prefill_item_heads(hq / hk));
   if (num_seqs > mvllm::kMaxStreamSeqs || forced == 2 || (forced != 1 && 2 * items >= cus)) {
-    // The grid may cut at most kSplitMaxItems 128-query items (bounded as in plan_split).
-    const int64_t q_tiles = (max_q + mvllm::kPrefillQueryTile - 1) / mvllm::kPrefillQueryTile;
-    const int64_t by_seqs = num_seqs * q_tiles, by_tokens = qtiles + num_seqs;
-    if (pair && o.prefill_pieces > 1 && hq / 2 <= mvllm::kSplitMaxCols &&
-        (by_seqs < by_tokens ? by_seqs : by_tokens) <= mvllm::kSplitMaxItems) {
+    if (!pair) return;
+    // The grid may cut at most kSplitMaxItems 128-query items.
+    if (o.prefill_pieces > 1 && hq / 2 <= mvllm::kSplitMaxCols &&
+        pair_items(num_tokens, num_seqs, max_q, mvllm::kPrefillQueryTile) <= mvllm::kSplitMaxItems) {
       plan.pub.prefill_pieces = o.prefill_pieces;
-      plan_split(plan, num_tokens, num_seqs, hq, max_q, cus, o.prefill_piece_pct, o.prefill_pieces);
-      if (!o.pieces_given && !pair_wants_split(num_tokens, num_seqs, hq, max_ctx, cus)) plan.split_pieces = 0;
+      plan_ranked(plan, num_tokens, num_seqs, hq, max_q, m.tile, cus, o.prefill_piece_pct, o.prefill_pieces);
+      if (o.pieces_given || m.cut) return;
     }
+    plan_whole(plan, work, num_tokens, num_seqs, hq, max_q, m.tile, cus);
     return;
   }
   int64_t wgs = static_cast<int64_t>(o.prefill_wgs_per_cu) * cus;
@@ -273,11 +354,19 @@ void plan_prefill(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, 
   plan.off_pf_o = plan.off_pf + align256(static_cast<uint64_t>(num_seqs + 1) * sizeof(int));
   plan.off_pf_ml = plan.off_pf_o + align256(rows * d * sizeof(float));
   plan.pub.workspace_bytes = plan.off_pf_ml + align256(rows * 2 * sizeof(float));
-  if (pair && (forced == 1 || pair_wants_split(num_tokens, num_seqs, hq, max_ctx, cus))) {
+  if (pair) {
     // (the stream's partial rows are not used then: the slots and records take their place)
     const uint64_t end = plan.pub.workspace_bytes;
     plan.pub.workspace_bytes = plan.off_pf_o;
-    plan_split(plan, num_tokens, num_seqs, hq, max_q, static_cast<int>(wgs), 100, kStreamPieces);
+    if (forced == 1 || m.cut) {
+      plan_ranked(plan, num_tokens, num_seqs, hq, max_q, m.tile, static_cast<int>(wgs), 100, kStreamPieces);
+      plan.split_weigh = forced != 1;
+      // (64 tokens after 500 keys over fp8, 8 items of 9 tiles: 24 us with pieces of at least
+      // the default 4 tiles, 20 with 2; over bf16 level)
+      if (kv_dtype == mvllm::kFP8E4M3 && !o.share_tiles_given) plan.prefill_share_tiles = 2;
+    } else {
+      plan_whole(plan, work, num_tokens, num_seqs, hq, max_q, m.tile, cus);
+    }
     if (plan.pub.workspace_bytes < end) plan.pub.workspace_bytes = end;
   }
 }
@@ -290,6 +379,10 @@ Plan make_plan(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t hk, int
               kv_dtype, o);
   plan_prefill(plan, num_tokens, num_seqs, hq, hk, d, block_size, max_q, max_ctx, q_dtype, kv_dtype,
                o);
+  if (plan.pub.prefill_mfma && pair_prefill(hq, hk, d, block_size, q_dtype, kv_dtype, o)) {
+    plan.pub.prefill_item = plan.split_tile;
+    plan.pub.prefill_listed = plan.split_pieces;
+  }
   return plan;
 }
 
@@ -375,7 +468,6 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
   p.by_row = plan.pub.decode_mode == MVLLM_DECODE_BY_ROW ? 1 : 0;
   p.pf_register_staging = plan.register_staging;
   p.pf_share_tiles = plan.prefill_share_tiles;
-  p.pf_cus = device_cus();
   if (plan.pub.workspace_bytes > 0) {
     char* ws = static_cast<char*>(workspace);
     if (plan.pub.decode_mode == MVLLM_DECODE_STREAM) p.seq_prefix = reinterpret_cast<int*>(ws);
@@ -387,25 +479,29 @@ int launch_planned(const Plan& plan, mvllm::PagedParams& p, void* workspace, int
       p.pf_o = reinterpret_cast<float*>(ws + plan.off_pf_o);
       p.pf_ml = reinterpret_cast<float*>(ws + plan.off_pf_ml);
     }
-    p.pf_pieces = plan.split_pieces;
-    if (plan.split_pieces > 1 && plan.pub.prefill_workgroups == 0) {
-      // The grid under graph capture runs its items whole: a graph's result does not depend
-      // on how a batch's lengths would cut them.
-      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing(s, &capture) != hipSuccess ||
-          capture != hipStreamCaptureStatusNone) {
-        g_split_whole_capturing.fetch_add(1, std::memory_order_relaxed);
-        p.pf_pieces = 0;
-      }
+  }
+  p.pf_tile = plan.split_tile;
+  p.pf_pieces = plan.split_pieces;
+  if (plan.split_pieces > 1 && plan.pub.prefill_workgroups == 0) {
+    // The grid's cut items run whole under graph capture, counted: what callers of
+    // mvllm_split_stats were promised when cutting needed counters of a stream's own. (The
+    // cut needs none now, and the stream schedule's is captured as it is.)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess ||
+        capture != hipStreamCaptureStatusNone) {
+      g_split_whole_capturing.fetch_add(1, std::memory_order_relaxed);
+      p.pf_pieces = 0;
     }
-    if (p.pf_pieces > 1) {
-      p.pf_ranks = plan.split_ranks;
-      p.pf_slots = plan.split_slots;
-      p.pf_piece_pct = plan.split_pct;
-      p.pf_cus = plan.split_wgs;
-      p.pf_part = reinterpret_cast<float*>(ws + plan.off_split);
-      p.pf_rec = reinterpret_cast<int4*>(ws + plan.off_rec);
-    }
+  }
+  if (p.pf_pieces >= 1) {
+    p.pf_ranks = plan.split_ranks;
+    p.pf_slots = plan.split_slots;
+    p.pf_piece_pct = plan.split_pct;
+    p.pf_cus = plan.split_wgs;
+    p.pf_weigh = plan.split_weigh ? 1 : 0;
+    p.pf_by_seq = plan.split_by_seq ? 1 : 0;
+    p.pf_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_split);
+    p.pf_rec = reinterpret_cast<int4*>(static_cast<char*>(workspace) + plan.off_rec);
   }
   if (plan.pub.decode_mode != MVLLM_DECODE_NONE) {
     const int rc = hip_status(mvllm::launch_paged_decode(p, q_dtype, kv_dtype, head_dim, s),
@@ -575,7 +671,7 @@ extern "C" {
 
 const char* mvllm_last_error(void) { return g_error; }
 
-int mvllm_abi_version(void) { return 16; }
+int mvllm_abi_version(void) { return 17; }
 
 #ifndef MVLLM_SOURCE_HASH
 #define MVLLM_SOURCE_HASH "unstamped"

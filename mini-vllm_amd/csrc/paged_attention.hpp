@@ -40,14 +40,23 @@ __host__ __device__ inline int64_t prefill_stream_shares(int64_t total_units, in
 constexpr int kXcds = 8;
 constexpr int kPrefillKeyTile = 64;
 
-// The pair prefill kernel's items (64 query positions of two heads of a GQA group) and its
-// split schedule: items longer than a piece length (a percentage of the mean key tiles per
-// workgroup) are cut into key ranges ("pieces") run by workgroups of their own, whose (m, l,
-// O) partials a second kernel merges. Every workgroup derives the same schedule from the
-// sequences' sizes.
-constexpr int kPairQueryTile = 64;
-// Floats of one piece's partial: two heads x 64 rows x (128 of O + (m, l)).
-constexpr int kPairSlotFloats = 2 * kPairQueryTile * 130;
+// The pair prefill kernel's items (64 or 128 query positions of two heads of a GQA group) and
+// its schedule: items in a list without the grid's holes, those longer than a piece length
+// (a percentage of the mean key tiles per workgroup) cut, where the plan says so, into key ranges
+// ("pieces") run by workgroups of their own, whose (m, l, O) partials a second kernel
+// merges. The schedule is formed on the device from the sequences' sizes.
+// Times in units of 10 ns: a key tile of the longest item when items run whole, of the mean per
+// CU when they are cut, and what cutting costs beside, for the host's choice and, where the
+// launch is ready for both, the device's.
+struct PairCosts {
+  int whole, cut, fixed, weigh;
+};
+__host__ __device__ constexpr PairCosts pair_costs(int tile, bool fp8) {
+  return tile == 64 ? (fp8 ? PairCosts{155, 185, 1300, 900} : PairCosts{93, 125, 1300, 900})
+                    : (fp8 ? PairCosts{190, 230, 1800, 1800} : PairCosts{95, 190, 1800, 1800});
+}
+// Floats of one piece's partial: two heads x qt rows x (128 of O + (m, l)).
+__host__ __device__ constexpr int pair_slot_floats(int qt) { return 2 * qt * 130; }
 // The grid plan cuts at most this many 128-query items over at most this many columns.
 constexpr int kSplitMaxItems = 64;
 constexpr int kSplitMaxCols = 64;
@@ -92,8 +101,8 @@ __host__ __device__ inline int decode_min_share_keys(int elem_bytes, int head_di
 constexpr float kRescaleSlack = 8.0f;
 // Pair prefill: the tiles whose probabilities are taken against the tile's own maxima, so that
 // each query's largest one is 1 and not rounded to 16 bits: all of an item (or piece) of at
-// most kExactTiles, every kExactEvery'th of a longer one, half as often where the items fill
-// the chip. Each costs a rescale of O, 64 multiplies of a tile's ~400 vector cycles per wave:
+// most kExactTiles, every kExactEvery'th of a longer one, half as often where the items fill the
+// chip or are of 128 positions, none of a longer one of 128 over fp8. Each costs a rescale of O, 64 multiplies of a tile's ~400 vector cycles per wave:
 // 7% of a chip-filling launch (8 x 512 tokens after up to 1536 keys 57.3 -> 61.7 us, 2048 after
 // 14336 526 -> 563), hidden in a small one (100 tokens after 300 keys 13.3 -> 14.2, 512 after
 // 4000 42.6 -> 44.5). Errors against 64 bits without, with all, and as chosen, float16: 100
@@ -198,15 +207,19 @@ struct PagedParams {
                             // fewest key tiles per piece
   int pf_register_staging;  // 1: the register-staged prefill kernel even where the
                             // direct-to-LDS one serves (a plan option, for measurement)
-  int pf_pieces;      // pair prefill: > 1 cuts long items into at most this many pieces (a
-                      // 1-D grid of pf_ranks x columns); otherwise the (column,
-                      // sequence, query tile) grid with every item whole
-  int pf_ranks;       // split: grid extent in ranks (items + extra pieces bound)
-  int pf_slots;       // split: partial slots per column
-  int pf_cus;         // the device's CUs; split: the workgroups the pieces are sized for
-  int pf_piece_pct;   // split: piece length, percent of the mean tiles per workgroup
-  float* pf_part;     // split: [pf_slots][columns] partials of kPairSlotFloats
-  int4* pf_rec;       // split: [pf_ranks][2], each position's piece for the merge
+  int pf_tile;        // pair prefill: query positions of an item, 64 or 128
+  int pf_pieces;      // pair prefill: 0 the (column, sequence, query tile) grid; else a 1-D grid
+                      // of pf_ranks x columns by the schedule, items in at most this
+                      // many pieces
+  int pf_by_seq;      // schedule of whole items: 1 a sequence's after another's
+  int pf_ranks;       // schedule: grid extent in ranks (items + extra pieces bound)
+  int pf_slots;       // cut: partial slots per column
+  int pf_cus;         // cut: the workgroups the pieces are sized for
+  int pf_piece_pct;   // cut: piece length, percent of the mean tiles per workgroup
+  int pf_weigh;       // cut: 1 leaves all items whole where their sizes make that faster
+  float* pf_part;     // cut: [pf_slots][columns] partials of pair_slot_floats
+  int4* pf_rec;       // [pf_ranks][2], each position's piece: for the merge, and from the
+                      // schedule kernel (more than 64 sequences)
 };
 
 // Splits of one row: as many as its visible context needs at `split_tokens` keys

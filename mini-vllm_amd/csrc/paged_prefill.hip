@@ -284,9 +284,8 @@ __device__ __forceinline__ bool prefill_work(const PagedParams& p, int cols, int
   return true;
 }
 
-// A piece of the pair kernel's work: key tiles [tb, te) of query tile q (of kPairQueryTile
-// positions) of sequence s, the `piece`th of the item's `pieces`, its partial in slot
-// slot0 + piece when there are several.
+// A piece of the pair kernel's work: key tiles [tb, te) of query tile q of sequence s, the
+// `piece`th of the item's `pieces`, its partial in slot slot0 + piece when there are several.
 struct PairPiece {
   int s, q, piece, pieces, slot0, tb, te;
 };
@@ -296,100 +295,235 @@ __device__ __forceinline__ int pair_item_tiles(int context, int len, int q, int 
   return (context - len + min((q + 1) * qt, len) + kTileKeys - 1) / kTileKeys;
 }
 
-// The piece at position `rank` of the split schedule, computed by every wave for itself
-// from the sequences' sizes (no host read of device data, no launch before, no barrier).
-// The piece length is pct% of the mean key tiles per CU, at least pf_share_tiles; an item
-// of nt tiles is cut into P = min(pf_pieces, ceil(nt / length)) equal key ranges. P - 1 <
-// nt / length, so the pieces beyond one an item number fewer than 100 cus / (pct cols) and
-// the cut items' pieces fewer than twice that: the grid's extra ranks and the partial
-// slots. The positions past the last piece end here; they come last, so that the pieces
-// are dealt to empty CUs one each (first, they left some CUs two pieces and others none: a
-// 512-token chunk after 8000 keys 60 us against 57). Lane l holds sequence 64 i + l of the i-th chunk.
-__device__ __forceinline__ bool pair_piece(const PagedParams& p, int cols, int rank,
-                                           PairPiece& out) {
+// Query tiles of a sequence (a decode row has none here).
+__device__ __forceinline__ int pair_query_tiles(int len, int qt) {
+  return len > 1 ? (len + qt - 1) / qt : 0;
+}
+
+// The schedule's piece length in tiles: pct% of the mean tiles per CU of all items, at least
+// pf_share_tiles; an item of nt tiles is cut into P = min(pf_pieces, ceil(nt / length)) equal
+// key ranges. P - 1 < nt / length, so the pieces beyond one an item number fewer than 100 cus /
+// (pct cols) and the cut items' pieces fewer than twice that: the grid's extra ranks and
+// the partial slots.
+__device__ __forceinline__ int pair_piece_tiles(const PagedParams& p, int cols, int total) {
+  const int64_t scaled = static_cast<int64_t>(p.pf_piece_pct) * total * cols;
+  return max(static_cast<int>((scaled + 100 * p.pf_cus - 1) / (100 * p.pf_cus)), max(p.pf_share_tiles, 1));
+}
+template <int QT, bool kFp8>
+__device__ __forceinline__ bool pair_stays_whole(const PagedParams& p, int cols, int total, int longest) {
+  constexpr PairCosts c = pair_costs(QT, kFp8);
+  return p.pf_weigh != 0 && static_cast<int64_t>(longest) * c.whole * p.pf_cus <=
+                                static_cast<int64_t>(total) * cols * c.cut + c.weigh * static_cast<int64_t>(p.pf_cus);
+}
+__device__ __forceinline__ int pair_pieces(const PagedParams& p, int nt, int length) {
+  return min(p.pf_pieces, (nt + length - 1) / length);
+}
+
+// Whether to stop at this length: all pieces run at once, or longer ones change nothing or
+// cannot matter. Rounding each item's pieces up may pass the CUs by a few, whose two
+// workgroups then take twice as long as the others (one 512-token chunk after 8000 keys, 272
+// pieces on 256 CUs: 68 us, 256 60 us), so the length grows until they fit.
+__device__ __forceinline__ bool pair_fits(const PagedParams& p, int cols, int ranks, int items) {
+  return ranks * cols <= p.pf_cus || ranks <= items || 2 * items * cols > p.pf_cus;
+}
+
+// Pieces (low half) and cut items' slots (high half; both below 2^15) of a sequence.
+template <int QT>
+__device__ __forceinline__ int pair_count(const PagedParams& p, int ctx, int len, int length) {
+  const int qts = pair_query_tiles(len, QT);
+  int both = 0;
+  for (int q = 0; q < qts; ++q) {
+    const int pcs = pair_pieces(p, pair_item_tiles(ctx, len, q, QT), length);
+    both += pcs | (pcs > 1 ? pcs << 16 : 0);
+  }
+  return both;
+}
+
+// The `r`th piece of a sequence, whose cut items' slots start at out.slot0.
+template <int QT>
+__device__ __forceinline__ void pair_locate(const PagedParams& p, int ctx, int len, int length, int r,
+                                            PairPiece& out) {
+  for (out.q = 0;; ++out.q) {
+    const int nt = pair_item_tiles(ctx, len, out.q, QT);
+    out.pieces = pair_pieces(p, nt, length);
+    if (r < out.pieces) {
+      out.piece = r;
+      out.tb = r * nt / out.pieces;
+      out.te = (r + 1) * nt / out.pieces;
+      return;
+    }
+    r -= out.pieces;
+    if (out.pieces > 1) out.slot0 += out.pieces;
+  }
+}
+
+// The piece at position `rank` of the schedule of at most 64 sequences, computed by every wave
+// for itself from the sequences' sizes, lane s holding sequence s's (no host read of device
+// data, no launch before, no barrier). The positions past the last piece end here; they come
+// last, so that the pieces are dealt to empty CUs one each (first, they left some CUs two
+// pieces and others none: a 512-token chunk after 8000 keys 60 us against 57).
+template <int QT, bool kFp8>
+__device__ __forceinline__ bool pair_piece(const PagedParams& p, int cols, int rank, PairPiece& out) {
   const int lane = threadIdx.x % kWave;
-  const int n = p.num_seqs;
-  int total = 0, items = 0;
-  int len = 0, ctx = 0, qts = 0;
-  auto load = [&](int base) __attribute__((always_inline)) {  // sequence base + lane
-    len = base + lane < n ? p.seq_lens[base + lane] : 0;
-    ctx = base + lane < n ? p.context_lens[base + lane] : 0;
-    qts = len > 1 ? (len + kPairQueryTile - 1) / kPairQueryTile : 0;
-  };
+  const int len = lane < p.num_seqs ? p.seq_lens[lane] : 0;
+  const int ctx = lane < p.num_seqs ? p.context_lens[lane] : 0;
   auto wave_total = [&](int v) __attribute__((always_inline)) -> int {
     return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1);
   };
-  for (int base = 0; base < n; base += kWave) {
-    load(base);
-    int tiles = 0;
-    for (int q = 0; q < qts; ++q) tiles += pair_item_tiles(ctx, len, q, kPairQueryTile);
-    total += wave_total(tiles);
-    items += wave_total(qts);
-  }
-  const int64_t scaled = static_cast<int64_t>(p.pf_piece_pct) * total * cols;
-  int length = static_cast<int>((scaled + 100 * p.pf_cus - 1) / (100 * p.pf_cus));
-  length = max(length, max(p.pf_share_tiles, 1));
-  auto pieces_of = [&](int nt) __attribute__((always_inline)) -> int {
-    return min(p.pf_pieces, (nt + length - 1) / length);
-  };
-  // Pieces (low half) and cut items' slots (high half; both below 2^15) of a sequence.
-  auto count = [&]() __attribute__((always_inline)) -> int {
-    int both = 0;
-    for (int q = 0; q < qts; ++q) {
-      const int pcs = pieces_of(pair_item_tiles(ctx, len, q, kPairQueryTile));
-      both += pcs | (pcs > 1 ? pcs << 16 : 0);
-    }
-    return both;
-  };
-  // Every piece at once: rounding each item's pieces up may pass the CUs by a few, whose two
-  // workgroups then take twice as long as the others (one 512-token chunk after 8000 keys,
-  // 272 pieces on 256 CUs: 68 us, 256 60 us), so the length grows until they fit.
-  int ranks = 0;
-  for (int i = 0; i < 12; ++i) {
-    ranks = 0;
-    for (int base = 0; base < n; base += kWave) {
-      if (n > kWave) load(base);
-      ranks += wave_total(count() & 0xffff);
-    }
-    if (ranks * cols <= p.pf_cus || ranks <= items || 2 * items * cols > p.pf_cus) break;
-    length += (length + 15) / 16;
-  }
-  if (rank >= ranks) return false;
-  int before = 0, slots = 0;
-  for (int base = 0; base < n; base += kWave) {
-    if (n > kWave) load(base);
-    const int both = count();
-    const int incl = wave_inclusive_scan(both);
-    const int all = __builtin_amdgcn_readlane(incl, kWave - 1);
-    const int first = before + ((incl - both) & 0xffff);
-    const uint64_t mine =
-        __builtin_amdgcn_ballot_w64(rank >= first && rank < first + (both & 0xffff));
-    if (mine != 0) {
-      const int i = __builtin_ctzll(mine);
-      const int len_i = __builtin_amdgcn_readlane(len, i), ctx_i = __builtin_amdgcn_readlane(ctx, i);
-      int r = rank - __builtin_amdgcn_readlane(first, i);
-      out.slot0 = slots + (__builtin_amdgcn_readlane(incl - both, i) >> 16);
-      out.s = base + i;
-      for (out.q = 0;; ++out.q) {
-        const int nt = pair_item_tiles(ctx_i, len_i, out.q, kPairQueryTile);
-        out.pieces = pieces_of(nt);
-        if (r < out.pieces) {
-          out.piece = r;
-          out.tb = r * nt / out.pieces;
-          out.te = (r + 1) * nt / out.pieces;
+  const int qts = pair_query_tiles(len, QT);
+  if (p.pf_pieces == 1) {
+    // Whole items, longest first: by sequence, or every sequence's last query tile, then every
+    // one's before it, and so on.
+    int q_from_last = 0;
+    if (p.pf_by_seq) {
+      const int before = wave_inclusive_scan(qts) - qts;
+      const uint64_t mine = __builtin_amdgcn_ballot_w64(rank >= before && rank < before + qts);
+      if (mine == 0) return false;
+      out.s = __builtin_ctzll(mine);
+      q_from_last = rank - __builtin_amdgcn_readlane(before, out.s);
+    } else {
+      for (int before = 0;; ++q_from_last) {
+        const uint64_t have = __builtin_amdgcn_ballot_w64(qts > q_from_last);
+        if (have == 0) return false;
+        const int count = __builtin_popcountll(have);
+        if (rank < before + count) {
+          const int nth = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+              static_cast<uint32_t>(have >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(have), 0)));
+          out.s = __builtin_ctzll(__builtin_amdgcn_ballot_w64(qts > q_from_last && nth == rank - before));
           break;
         }
-        r -= out.pieces;
-        if (out.pieces > 1) out.slot0 += out.pieces;
+        before += count;
       }
-      // (the bounds above rule this out; a slot is never written past the workspace)
-      if (out.pieces > 1 && out.slot0 + out.pieces > p.pf_slots) return false;
-      return true;
     }
-    before += all & 0xffff;
+    out.q = __builtin_amdgcn_readlane(qts, out.s) - 1 - q_from_last;
+    out.piece = out.tb = out.slot0 = 0;
+    out.pieces = 1;
+    out.te = pair_item_tiles(__builtin_amdgcn_readlane(ctx, out.s), __builtin_amdgcn_readlane(len, out.s),
+                             out.q, QT);
+    return true;
+  }
+  int length = 0;
+  {
+    int tiles = 0;
+    for (int q = 0; q < qts; ++q) tiles += pair_item_tiles(ctx, len, q, QT);
+    const int items = wave_total(qts), total = wave_total(tiles);
+    const int own = qts > 0 ? pair_item_tiles(ctx, len, qts - 1, QT) : 0;
+    const int longest = static_cast<int>(wave_max(static_cast<float>(own)));  // (below 2^24)
+    const bool whole = pair_stays_whole<QT, kFp8>(p, cols, total, longest);
+    length = whole ? max(longest, 1) : pair_piece_tiles(p, cols, total);
+    for (int i = 0; i < 12 && !whole; ++i) {
+      if (pair_fits(p, cols, wave_total(pair_count<QT>(p, ctx, len, length) & 0xffff), items)) break;
+      length += (length + 15) / 16;
+    }
+  }
+  const int both = pair_count<QT>(p, ctx, len, length);
+  const int before = wave_inclusive_scan(both) - both;
+  const int first = before & 0xffff;
+  const uint64_t mine = __builtin_amdgcn_ballot_w64(rank >= first && rank < first + (both & 0xffff));
+  if (mine == 0) return false;
+  out.s = __builtin_ctzll(mine);
+  out.slot0 = __builtin_amdgcn_readlane(before, out.s) >> 16;
+  pair_locate<QT>(p, __builtin_amdgcn_readlane(ctx, out.s), __builtin_amdgcn_readlane(len, out.s), length,
+                  rank - (__builtin_amdgcn_readlane(before, out.s) & 0xffff), out);
+  // (the bounds above rule this out; a slot is never written past the workspace)
+  return out.pieces == 1 || out.slot0 + out.pieces <= p.pf_slots;
+}
+
+__device__ __forceinline__ void pair_store(const PagedParams& p, int rank, const PairPiece& w) {
+  p.pf_rec[2 * rank] = make_int4(w.s, w.q, w.piece, w.pieces);
+  p.pf_rec[2 * rank + 1] = make_int4(w.slot0, w.tb, w.te, 0);
+}
+
+// The same schedule of cut items for more than 64 sequences (up to kMaxStreamSeqs), written to
+// the ranks' records by one wave ahead of the pair kernel: the chunks among the sequences are
+// listed in LDS, then held a lane each, 64 at a time. (Every workgroup scanning all sequences
+// for itself, once per length tried, took longer than the prefill: one 512-token chunk after
+// 7000 keys among 500 decodes 309 us a call, so 275.)
+template <int QT, bool kFp8>
+__global__ __launch_bounds__(kWave) void paged_prefill_schedule_kernel(const PagedParams p) {
+  constexpr int kAhead = 8;
+  __shared__ int s_seq[kMaxStreamSeqs], s_len[kMaxStreamSeqs], s_ctx[kMaxStreamSeqs];
+  const int lane = threadIdx.x, cols = p.hq / 2, n = p.num_seqs;
+  auto wave_total = [&](int v) __attribute__((always_inline)) -> int {
+    return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1);
+  };
+  int chunks = 0;
+  for (int base = 0; base < n; base += kAhead * kWave) {
+    int len[kAhead], ctx[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int s = min(base + i * kWave + lane, n - 1);
+      len[i] = p.seq_lens[s];
+      ctx[i] = p.context_lens[s];
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int s = base + i * kWave + lane;
+      const uint64_t have = __builtin_amdgcn_ballot_w64(s < n && len[i] > 1);
+      const int nth = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+          static_cast<uint32_t>(have >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(have), 0)));
+      if (s < n && len[i] > 1) {
+        s_seq[chunks + nth] = s;
+        s_len[chunks + nth] = len[i];
+        s_ctx[chunks + nth] = ctx[i];
+      }
+      chunks += __builtin_popcountll(have);
+    }
+  }
+  __syncthreads();
+  int len = 0, ctx = 0;
+  auto take = [&](int base) __attribute__((always_inline)) {  // chunk base + lane
+    len = base + lane < chunks ? s_len[base + lane] : 0;
+    ctx = base + lane < chunks ? s_ctx[base + lane] : 0;
+  };
+  int total = 0, items = 0, longest = 0;
+  for (int base = 0; base < chunks; base += kWave) {
+    take(base);
+    const int qts = pair_query_tiles(len, QT);
+    int tiles = 0;
+    for (int q = 0; q < qts; ++q) tiles += pair_item_tiles(ctx, len, q, QT);
+    const int own = qts > 0 ? pair_item_tiles(ctx, len, qts - 1, QT) : 0;
+    total += wave_total(tiles);
+    items += wave_total(qts);
+    longest = max(longest, static_cast<int>(wave_max(static_cast<float>(own))));  // (below 2^24)
+  }
+  const bool whole = pair_stays_whole<QT, kFp8>(p, cols, total, longest);
+  int length = whole ? max(longest, 1) : pair_piece_tiles(p, cols, total);
+  for (int i = 0; i < 12 && !whole; ++i) {
+    int ranks = 0;
+    for (int base = 0; base < chunks; base += kWave) {
+      if (chunks > kWave) take(base);
+      ranks += wave_total(pair_count<QT>(p, ctx, len, length) & 0xffff);
+    }
+    if (pair_fits(p, cols, ranks, items)) break;
+    length += (length + 15) / 16;
+  }
+  int ranks = 0, slots = 0;
+  for (int base = 0; base < chunks; base += kWave) {
+    if (chunks > kWave) take(base);
+    const int both = pair_count<QT>(p, ctx, len, length);
+    const int incl = wave_inclusive_scan(both);
+    const int all = __builtin_amdgcn_readlane(incl, kWave - 1);
+    int rank = ranks + ((incl - both) & 0xffff), slot0 = slots + ((incl - both) >> 16);
+    const int qts = pair_query_tiles(len, QT);
+    PairPiece w{};
+    w.s = base + lane < chunks ? s_seq[base + lane] : 0;
+    for (w.q = 0; w.q < qts; ++w.q) {
+      const int nt = pair_item_tiles(ctx, len, w.q, QT);
+      w.pieces = pair_pieces(p, nt, length);
+      w.slot0 = slot0;
+      if (w.pieces > 1) slot0 += w.pieces;
+      const bool fits = w.pieces == 1 || slot0 <= p.pf_slots;  // (the host's bounds see to both)
+      for (w.piece = 0; w.piece < w.pieces; ++w.piece, ++rank) {
+        w.tb = w.piece * nt / w.pieces;
+        w.te = (w.piece + 1) * nt / w.pieces;
+        if (rank < p.pf_ranks) pair_store(p, rank, fits ? w : PairPiece{});
+      }
+    }
+    ranks += all & 0xffff;
     slots += all >> 16;
   }
-  return false;
+  for (int r = ranks + lane; r < p.pf_ranks; r += kWave) pair_store(p, r, PairPiece{});
 }
 
 }  // namespace
@@ -1275,17 +1409,22 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
   int s, qt, c, tb, te;
   PairPiece piece{};
   if constexpr (kSplit) {
-    static_assert(kWaves * 16 == kPairQueryTile, "the split schedule's query tile");
     const int cols = p.hk * chunks;
     c = static_cast<int>(blockIdx.x) % cols;
     const int rank = static_cast<int>(blockIdx.x) / cols;
-    const bool got = pair_piece(p, cols, rank, piece);
-    if (c == 0 && tid == 0) {  // what the merge needs to know of this position
-      p.pf_rec[2 * rank] = got ? make_int4(piece.s, piece.q, piece.piece, piece.pieces)
-                               : make_int4(0, 0, 0, 0);
-      p.pf_rec[2 * rank + 1] = make_int4(piece.slot0, 0, 0, 0);
+    if (p.num_seqs > kWave) {  // (the schedule kernel's record)
+      const int4 a = p.pf_rec[2 * rank], b = p.pf_rec[2 * rank + 1];
+      if (a.w == 0) return;
+      piece = PairPiece{a.x, a.y, a.z, a.w, b.x, b.y, b.z};
+    } else {
+      const bool got = pair_piece<QT, kFp8>(p, cols, rank, piece);
+      if (p.pf_pieces > 1 && c == 0 && tid == 0) {  // what the merge needs to know
+        pair_store(p, rank, got ? piece : PairPiece{});
+      }
+      if (!got) return;
     }
-    if (!got) return;
+    piece.slot0 = uniform(piece.slot0 + piece.piece);  // (its own from here on)
+    piece.pieces = uniform(piece.pieces);
     s = uniform(piece.s);
     qt = uniform(piece.q);
     tb = uniform(piece.tb);
@@ -1448,7 +1587,9 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
   float m_run = -INFINITY, l_run = 0.0f;
   float m_top = -INFINITY;  // the largest score so far
   const int exact_mask =    // tiles t & exact_mask == 0 are taken against their own maxima
-      te - tb <= kExactTiles ? 0 : p.pf_wgs > 0 ? kExactEvery - 1 : 2 * kExactEvery - 1;
+      te - tb <= kExactTiles ? 0
+      : QT == 64 && p.pf_wgs > 0 ? kExactEvery - 1
+      : QT == 64 || !kFp8 ? 2 * kExactEvery - 1 : INT_MAX;
   f32x16 sc0[2], sc1[2];  // scores of even / odd tiles
 
   // Fragment i of the K in buffer `par`: keys 32 (i % 2) .., dims 16 (i / 2) ..; fragments are
@@ -1686,10 +1827,10 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
   if constexpr (kSplit) {
     if (piece.pieces > 1) {
       // A cut item: the unnormalised O, the running max and the sum, fp32, to the piece's
-      // slot ([2 heads][64 rows][D], then [2 heads][64 rows] of (max, sum)).
+      // slot ([2 heads][QT rows][D], then [2 heads][QT rows] of (max, sum)).
       const int cols = p.hk * chunks;
-      float* slot = p.pf_part + (static_cast<int64_t>(piece.slot0 + piece.piece) * cols + c) * kPairSlotFloats;
-      const int row = hs * kPairQueryTile + 32 * wq + l32;
+      float* slot = p.pf_part + (static_cast<int64_t>(piece.slot0) * cols + c) * pair_slot_floats(QT);
+      const int row = hs * QT + 32 * wq + l32;
 #pragma unroll
       for (int db = 0; db < kDBlocks; ++db) {
 #pragma unroll
@@ -1699,7 +1840,7 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
         }
       }
       if (hsel == 0) {
-        *reinterpret_cast<float2*>(slot + 2 * kPairQueryTile * D + 2 * row) = make_float2(m_run, l_tot);
+        *reinterpret_cast<float2*>(slot + 2 * QT * D + 2 * row) = make_float2(m_run, l_tot);
       }
       return;
     }
@@ -1721,14 +1862,14 @@ __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(c
 }
 
 // Combine the pieces of the pair kernel's cut items: the workgroup at position (rank,
-// column) takes its own piece's share of the item's 128 x D outputs (its two heads' rows),
+// column) takes its own piece's share of the item's 2 QT x D outputs (its two heads' rows),
 // so a long item's merge is spread over as many workgroups as computed it; positions
 // without a cut item end at once. Each thread owns float4 columns of rows and folds the
 // pieces in piece order (the result does not depend on timing), kMergeBatch pieces'
 // loads in flight at a time.
 constexpr int kPairMergeThreads = 256;
 
-template <typename TQ>
+template <typename TQ, int QT>
 __global__ __launch_bounds__(kPairMergeThreads) void paged_prefill_pair_merge_kernel(const PagedParams p) {
   constexpr int D = 128;
   constexpr int kMergeBatch = 8;
@@ -1740,18 +1881,18 @@ __global__ __launch_bounds__(kPairMergeThreads) void paged_prefill_pair_merge_ke
   const int slot0 = p.pf_rec[2 * rank + 1].x;
   const int s = rec.x, q = rec.y, piece = rec.z, pieces = rec.w;
   if (pieces <= 1) return;
-  const int rows = min(kPairQueryTile, p.seq_lens[s] - q * kPairQueryTile);
-  const int row0 = p.cu_seqlens_q[s] + q * kPairQueryTile;
+  const int rows = min(QT, p.seq_lens[s] - q * QT);
+  const int row0 = p.cu_seqlens_q[s] + q * QT;
   const int head0 = (c / (group / 2)) * group + (c % (group / 2)) * 2;
   const int n4 = 2 * rows * (D / 4);
   const int lo = piece * n4 / pieces, hi = (piece + 1) * n4 / pieces;
-  const int64_t stride = static_cast<int64_t>(cols) * kPairSlotFloats;
-  const float* base = p.pf_part + (static_cast<int64_t>(slot0) * cols + c) * kPairSlotFloats;
+  const int64_t stride = static_cast<int64_t>(cols) * pair_slot_floats(QT);
+  const float* base = p.pf_part + (static_cast<int64_t>(slot0) * cols + c) * pair_slot_floats(QT);
   for (int j = lo + static_cast<int>(threadIdx.x); j < hi; j += kPairMergeThreads) {
     const int hw = j / (rows * (D / 4));
     const int rem = j - hw * rows * (D / 4);
     const int local = rem / (D / 4), d = (rem % (D / 4)) * 4;
-    const int row = hw * kPairQueryTile + local;
+    const int row = hw * QT + local;
     float m = -INFINITY, l = 0.0f;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int i0 = 0; i0 < pieces; i0 += kMergeBatch) {
@@ -1760,7 +1901,7 @@ __global__ __launch_bounds__(kPairMergeThreads) void paged_prefill_pair_merge_ke
 #pragma unroll
       for (int u = 0; u < kMergeBatch; ++u) {
         const float* slot = base + min(i0 + u, pieces - 1) * stride;
-        ml[u] = *reinterpret_cast<const float2*>(slot + 2 * kPairQueryTile * D + 2 * row);
+        ml[u] = *reinterpret_cast<const float2*>(slot + 2 * QT * D + 2 * row);
         oi[u] = *reinterpret_cast<const f32x4*>(slot + row * D + d);
       }
 #pragma unroll
@@ -1945,27 +2086,35 @@ void launch_prefill_cfg(const PagedParams& p, int max_query_len, hipStream_t str
   }
 }
 
-// The pair kernel: the split schedule when the launch has pieces to make (pf_pieces > 1),
-// the item grid otherwise. Workgroups of 64 query positions, but of 128 for fp8 pools when
-// those still fill the CUs: staging a tile there means converting it, work that the
-// larger workgroup halves (8 x 512 tokens after up to 1536: 67 us against 69; 5 chunks of
-// up to 512 tokens, 134 such workgroups: 73 against 63).
+// The pair kernel by its schedule (pf_pieces >= 1: a workgroup per position of it; pieces
+// merged after) or on the item grid.
+template <typename TQ, typename TKV, int kWaves>
+void launch_prefill_ranked(const PagedParams& p, hipStream_t stream) {
+  constexpr int QT = kWaves * 16;
+  const int grid = p.hq / 2 * p.pf_ranks;
+  if (p.num_seqs > kWave) {
+    paged_prefill_schedule_kernel<QT, std::is_same_v<TKV, fp8_t>><<<1, kWave, 0, stream>>>(p);
+  }
+  paged_prefill_pair_kernel<TQ, TKV, kWaves, true><<<grid, kWaves * kWave, 0, stream>>>(p);
+  if (p.pf_pieces > 1) {
+    paged_prefill_pair_merge_kernel<TQ, QT><<<grid, kPairMergeThreads, 0, stream>>>(p);
+  }
+}
+
 template <typename TQ, typename TKV>
 void launch_prefill_pair(const PagedParams& p, int max_query_len, hipStream_t stream) {
   const int cols = p.hq / 2;
-  if (p.pf_pieces > 1) {
-    paged_prefill_pair_kernel<TQ, TKV, 4, true><<<cols * p.pf_ranks, 256, 0, stream>>>(p);
-    paged_prefill_pair_merge_kernel<TQ><<<cols * p.pf_ranks, kPairMergeThreads, 0, stream>>>(p);
+  if (p.pf_pieces >= 1) {
+    if (p.pf_tile == 128) launch_prefill_ranked<TQ, TKV, 8>(p, stream);
+    else launch_prefill_ranked<TQ, TKV, 4>(p, stream);
     return;
   }
-  if constexpr (std::is_same_v<TKV, fp8_t>) {
+  if (p.pf_tile == 128) {
     const int wide = (max_query_len + 127) / 128;
-    if ((p.num_tokens + 127) / 128 * cols >= p.pf_cus) {
-      paged_prefill_pair_kernel<TQ, TKV, 8, false><<<dim3(cols, p.num_seqs, wide), 512, 0, stream>>>(p);
-      return;
-    }
+    paged_prefill_pair_kernel<TQ, TKV, 8, false><<<dim3(cols, p.num_seqs, wide), 512, 0, stream>>>(p);
+    return;
   }
-  const int qtiles = (max_query_len + kPairQueryTile - 1) / kPairQueryTile;
+  const int qtiles = (max_query_len + 63) / 64;
   paged_prefill_pair_kernel<TQ, TKV, 4, false><<<dim3(cols, p.num_seqs, qtiles), 256, 0, stream>>>(p);
 }
 

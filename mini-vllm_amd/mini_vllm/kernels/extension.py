@@ -84,7 +84,7 @@ CXX = os.environ.get("CXX", "g++")
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-DNDEBUG", "-D__HIP_PLATFORM_AMD__=1",
               "-DUSE_ROCM=1"]
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 DTYPE_CODES: dict[torch.dtype, int] = {
     torch.float32: 0,
@@ -288,6 +288,8 @@ class _Plan(ctypes.Structure):
         ("workspace_bytes", ctypes.c_uint64),
         ("prefill_workgroups", ctypes.c_int32),
         ("prefill_pieces", ctypes.c_int32),
+        ("prefill_item", ctypes.c_int32),
+        ("prefill_listed", ctypes.c_int32),
     ]
 
 

@@ -120,6 +120,32 @@ def test_prefill_grid_schedule_workspace(lib):
     assert plan.prefill_workgroups > 0 and plan.prefill_pieces == 0
 
 
+@pytest.mark.parametrize("sizes,kv,item,listed", [
+    # (tokens, sequences, longest chunk, longest context): few items, long contexts: cut; the
+    # longer the mean per CU the larger the items
+    ((64, 1, 64, 8064), 2, 64, 64),
+    ((512, 1, 512, 4512), 2, 64, 64),
+    ((1052, 29, 1024, 5024), 2, 128, 64),
+    ((512, 1, 512, 4512), 3, 128, 64),
+    ((1563, 32, 512, 4252), 3, 128, 64),
+    # short ones: whole, listed where decode rows would leave holes in the grid
+    ((512, 1, 512, 512), 2, 64, 0),
+    ((540, 29, 512, 700), 2, 64, 1),
+    ((1253, 33, 300, 2279), 2, 64, 1),
+    ((1563, 32, 512, 4252), 2, 64, 1),
+    # items for every CU: whole, larger over fp8
+    ((4096, 8, 512, 2048), 2, 64, 0),
+    ((4096, 8, 512, 2048), 3, 128, 0),
+    ((2048, 1, 2048, 2048), 3, 64, 0),
+])
+def test_pair_prefill_plan(lib, sizes, kv, item, listed):
+    """The pair kernel's items and whether they are listed and cut: batches on either side
+    of the planner's lines (16 query heads over 8, 256 CUs without a GPU)."""
+    tokens, seqs, max_q, max_ctx = sizes
+    plan = _plan(lib, tokens, seqs, 16, 8, 128, 16, max_q, max_ctx, 2, kv)
+    assert (plan.prefill_item, plan.prefill_listed) == (item, listed)
+
+
 def test_plan_options_are_explicit_and_checked(lib, monkeypatch):
     """The schedule depends on the sizes and the options only: no environment knob."""
     monkeypatch.setenv("MVLLM_DECODE_SCHEDULE", "2")

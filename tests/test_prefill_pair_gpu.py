@@ -26,6 +26,7 @@ def check(extension, contexts, lens, dtype, kv_dtype, options, hq=16):
     want = oracle(b.q, b.key_pool, b.value_pool, b.block_tables, b.cu_seqlens_q, b.context_lens,
                   b.scale, **({"k_scale": b.k_scale, "v_scale": b.v_scale} if kv_dtype else {}))
     assert_max_abs(got.float(), want, ATTN_ATOL[kv_dtype or dtype], f"{contexts} {lens}")
+    return got
 
 
 @pytest.mark.parametrize("options", [WHOLE, CUT], ids=["whole", "cut"])
@@ -72,6 +73,37 @@ def test_cut_items_of_many_sequences(extension, device):
 def test_the_default_cuts_a_lone_long_chunk(extension, device):
     """No options: 63 tokens after 6393 keys (8 items on 256 CUs)."""
     check(extension, [6456], [63], torch.bfloat16, None, None)
+
+
+# (chunk lengths, keys before each, decode rows, their contexts' bound, heads, pool, item, listed)
+ROUTES = {
+    "whole, last query tiles first": ([129, 64, 2, 200, 65], [0, 100, 62, 57, 191], 20, 300, 16, None, 64, 1),
+    "whole, by sequence": ([256, 255, 257], [2400, 2345, 2000], 5, 900, 32, None, 64, 1),
+    "whole, fp8 items of 128": ([390, 385, 388, 384], [500, 0, 127, 64], 6, 700, 32, F8, 128, 1),
+    "cut, items of 128": ([130, 257, 65, 500], [4870, 4000, 4800, 4500], 3, 900, 16, None, 128, 64),
+    "cut, fp8 items of 128": ([130, 257, 65, 500], [3870, 3000, 3800, 3500], 3, 900, 16, F8, 128, 64),
+    "whole, more than 64 sequences": ([100, 33], [0, 64], 66, 200, 16, None, 64, 0),
+    "cut, more than 64 sequences": ([63, 3], [6000, 900], 70, 200, 16, None, 64, 64),
+    "cut, fp8, more than 64 sequences": ([300, 200], [5000, 4000], 68, 200, 16, F8, 128, 64),
+}
+
+
+@pytest.mark.parametrize("route", ROUTES)
+def test_the_planner_s_own_routes(extension, device, route):
+    """Ragged chunks among decode rows, every query tile and key tile edge somewhere in them,
+    by each way the planner runs a batch when no option forces one; the same bits again."""
+    chunks, before, decodes, bound, hq, kv_dtype, item, listed = ROUTES[route]
+    gen = torch.Generator().manual_seed(len(route))
+    rows = [(int(c), 1) for c in torch.randint(1, bound, (decodes,), generator=gen)]
+    rows += [(n + b, n) for n, b in zip(chunks, before)]
+    rows = [rows[i] for i in torch.randperm(len(rows), generator=gen).tolist()]
+    contexts, lens = [c for c, _ in rows], [n for _, n in rows]
+    plan = extension.paged_attention_plan(sum(lens), len(lens), hq, 8, 128, 16, max(lens), max(contexts),
+                                          torch.bfloat16, kv_dtype or torch.bfloat16)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (plan["prefill_item"], plan["prefill_listed"]) == (item, listed)
+    first, again = (check(extension, contexts, lens, torch.bfloat16, kv_dtype, None, hq) for _ in range(2))
+    assert torch.equal(first, again)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

@@ -526,8 +526,8 @@ int mvllm_sampling_probabilities(float* probs, const void* logits, int64_t rows,
                                  int64_t row_stride, int32_t dtype,
                                  const mvllm_sampling_row* params, void* workspace,
                                  uint64_t workspace_bytes, void* stream);
-/* Its workspace (256-byte aligned, contents need not be initialised): about 2.4 bytes per
- * logit of at most 128 rows. */
+/* Its workspace (256-byte aligned, contents need not be initialised): 2.4 to 3.5 bytes
+ * per logit of at most 128 rows. */
 uint64_t mvllm_sampling_workspace_bytes(int64_t rows, int64_t vocab);
 
 /* Read-only HBM probe for the benchmark's bandwidth ceiling (no counterpart in the

@@ -21,8 +21,9 @@
 //   gather   the row's bins added up and scanned, the boundary bin found, and the
 //            segment's tokens in it listed
 //   write    the last kept token selected among the listed ones (every workgroup of the
-//            row does it again: a handful of tokens, cheaper than a launch), and the
-//            probabilities written in vocabulary order
+//            row does it again, cheaper than a launch: they are mostly a handful; see
+//            select_last for rows where they are not), and the probabilities written in
+//            vocabulary order
 // Bounds: the logits are read four times (10 MB at 32 x 151936 bf16, from L2 and the
 // last-level cache after the first) and the probabilities written once (19 MB); each
 // launch is a few microseconds of latency and of vector work (an IEEE division by the
@@ -358,18 +359,36 @@ __global__ __launch_bounds__(kThreads) void sampling_gather_kernel(const Rows ro
 }
 
 // The last kept token's rank and the mass of all kept ones: an exact selection among
-// the boundary bin's listed tokens. While more than kThreads remain, a pass of eight
-// bits of the rank narrows them (the same rule over 256 bins); then each thread takes
-// one and compares it with all. Ranks are unique, so eight passes leave one token.
-template <typename T, int kSegment>
+// the boundary bin's listed tokens. While more than kThreads remain, passes narrow them by the
+// rule of the bins; then each thread takes one and compares it with all.
+//   They are a handful, or the whole vocabulary: flat rows, and rows of which one token stands
+// out or all but a few are masked while top_k asks for more. The passes:
+//   - the listed values' range; none of them with a probability ends here (masked tokens:
+//     which are kept changes nothing)
+//   - 1024 bins of equal width over that range, where it is a usual one
+//   - digits of ten bits of the value, from the first that can differ
+//   - of one value left, the segments, then ten bits of the index within one
+// What bounds them is one CU's vector work and LDS atomics, 25 to 60 us a pass over 151936
+// tokens. us a call for 1 and 32 rows of 151936 bf16 logits, sorted by torch, with 8-bit digits
+// of the rank from its first on, now: one value everywhere 198, 908; 2970, 4280; 129, 192; N(0,
+// 1e-3) with top-p 201, 964; 703, 744; 192, 288; N(0, 2) and one 25 with top-k 50 202, 968; 701,
+// 757; 165, 244; all but 30 masked, top-k 50 198, 906; 2952, 4246; 76, 118.
+constexpr int kDigit = 10;
+constexpr int kDigitBins = 1 << kDigit;
+constexpr int kDigitCopies = 2;
+constexpr int kPerThread = kDigitBins / kThreads;
+static_assert(kMaxSegments <= kDigitBins && kLongestSegment <= 1 << 14, "");
+
+template <typename T, bool kVec, int kSegment>
 __device__ __forceinline__ uint64_t select_last(const RowState& s, const Boundary& b,
-                                                const Work& w, const T* row, int r, int segments,
-                                                float unit, uint64_t* lds, uint64_t& kept_mass) {
+                                                const Work& w, const T* row, int64_t v, int r,
+                                                int segments, float unit, uint64_t* lds, uint64_t& kept_mass) {
   __shared__ uint32_t start[kMaxSegments + 1];
-  __shared__ unsigned long long mass[256];
-  __shared__ uint32_t count[256];
+  __shared__ unsigned long long mass[kDigitCopies][kDigitBins];
+  __shared__ uint32_t count[kDigitCopies][kDigitBins];
   __shared__ uint64_t c_rank[kThreads], c_mass[kThreads];
   __shared__ uint32_t taken;
+  const int lane = threadIdx.x % kWave;
   const int64_t cell = static_cast<int64_t>(r) * segments;
   uint64_t total = 0;
   {
@@ -381,69 +400,199 @@ __device__ __forceinline__ uint64_t select_last(const RowState& s, const Boundar
   }
   __syncthreads();
   const uint32_t listed = static_cast<uint32_t>(total);
-  auto token = [&](uint32_t j, uint64_t& rank, uint64_t& m) __attribute__((always_inline)) {
-    int a = 0, e = segments;  // start[a] <= j < start[e]
-    while (e - a > 1) {
-      const int mid = (a + e) >> 1;
-      if (start[mid] <= j) a = mid; else e = mid;
+  // f(x, index in the row) for segment a's listed tokens; from the list, a thread's loads kAhead
+  // at a time, or where it holds a good part of the segment from the row itself (its chunks
+  // in order, no load waiting for another: 151936 tokens 90 us by the list, 30 so).
+  constexpr int kAhead = 4;
+  auto for_segment = [&](int a, auto f) __attribute__((always_inline)) {
+    const uint32_t n = start[a + 1] - start[a];
+    const int64_t lo = static_cast<int64_t>(a) * kSegment, hi = min(v, lo + kSegment);
+    if (8 * n >= hi - lo) {
+      for_each<T, kVec, kSegment>(row, lo, hi, [&](int64_t i, float l) __attribute__((always_inline)) {
+        const float x = l / s.t;
+        if (bin_of(s.max, x) == b.bin) f(x, static_cast<uint32_t>(i));
+      });
+      return;
     }
-    const uint32_t index = static_cast<uint32_t>(a * kSegment) +
-                           w.list[(cell + a) * kSegment + (j - start[a])];
-    const float x = Elem<T>::load(row, index) / s.t;
-    rank = rank_of(x, index);
-    m = mass_of(expf(x - s.max), unit);
+    const uint16_t* list = w.list + (cell + a) * kSegment;
+    for (uint32_t j0 = 0; j0 < n; j0 += kAhead * kThreads) {
+      uint32_t index[kAhead];
+      float x[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        index[u] = a * kSegment + list[min(j0 + u * kThreads + threadIdx.x, n - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) x[u] = Elem<T>::load(row, index[u]);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        if (j0 + u * kThreads + threadIdx.x < n) f(x[u] / s.t, index[u]);
+      }
+    }
   };
-  uint64_t prefix = 0, count_before = b.count, mass_before = b.mass;
-  int known = 0;  // bits of the rank fixed so far
+  uint64_t count_before = b.count, mass_before = b.mass;
   uint32_t left = listed;
-  while (left > kThreads) {
-    const int shift = 56 - known;
-    if (threadIdx.x < 256) {
-      mass[threadIdx.x] = 0;
-      count[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    for (uint32_t j = threadIdx.x; j < listed; j += kThreads) {
-      uint64_t rank, m;
-      token(j, rank, m);
-      if (known == 0 || rank >> (64 - known) == prefix) {
-        const int bin = static_cast<int>(rank >> shift) & 255;
-        atomicAdd(&mass[bin], static_cast<unsigned long long>(m));
-        atomicAdd(&count[bin], 1u);
+  float top = 0.0f, per_unit = 0.0f;
+  int bin_chosen = -1;   // equal-width bin
+  uint64_t prefix = 0;   // of the rank
+  int known = 0;         // its bits
+  int first = 0, last = segments;  // the segments left
+  auto width_bin = [&](float x) __attribute__((always_inline)) -> int {
+    return static_cast<int>(fminf((top - x) * per_unit, static_cast<float>(kDigitBins - 1)));
+  };
+  auto matches = [&](float x, uint64_t rank) __attribute__((always_inline)) -> bool {
+    return (bin_chosen < 0 || width_bin(x) == bin_chosen) &&
+           (known == 0 || rank >> (64 - known) == prefix);
+  };
+  // One pass: bin_of_token over the tokens left, the last bin whose first token is kept (the
+  // first non-empty one's is: it was chosen for it), and what comes before it.
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+#pragma unroll
+      for (int c = 0; c < kDigitCopies; ++c) {
+        mass[c][i * kThreads + threadIdx.x] = 0;
+        count[c][i * kThreads + threadIdx.x] = 0;
       }
     }
     __syncthreads();
-    const bool own = threadIdx.x < 256;
-    const uint64_t m = own ? mass[threadIdx.x] : 0, c = own ? count[threadIdx.x] : 0;
-    uint64_t unused;
-    const uint64_t mb = mass_before + block_exclusive_scan64(m, lds, unused);
-    const uint64_t cb = count_before + block_exclusive_scan64(c, lds, unused);
-    // (the first non-empty bin's first token is kept: its bin was chosen for it)
-    const bool mine = c > 0 && (cb == count_before || keeps(cb, mb, s.k, b.limit));
-    const int bin = static_cast<int>(block_max64(mine ? threadIdx.x : 0, lds));
+  };
+  auto choose = [&]() __attribute__((always_inline)) -> int {
     __syncthreads();
-    if (static_cast<int>(threadIdx.x) == bin) {
-      lds[0] = mb;
-      lds[1] = cb;
-      lds[2] = c;
+    uint64_t bm[kPerThread], bc[kPerThread], m = 0, c = 0, unused;
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {  // thread t owns bins kPerThread t and on
+      bm[i] = bc[i] = 0;
+#pragma unroll
+      for (int k = 0; k < kDigitCopies; ++k) {
+        bm[i] += mass[k][kPerThread * threadIdx.x + i];
+        bc[i] += count[k][kPerThread * threadIdx.x + i];
+      }
+      m += bm[i];
+      c += bc[i];
+    }
+    uint64_t mb = mass_before + block_exclusive_scan64(m, lds, unused);
+    uint64_t cb = count_before + block_exclusive_scan64(c, lds, unused);
+    uint64_t my_bin = 0, my_mb = 0, my_cb = 0, my_c = 0;
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      if (bc[i] > 0 && (cb == count_before || keeps(cb, mb, s.k, b.limit))) {
+        my_bin = kPerThread * threadIdx.x + i;
+        my_mb = mb;
+        my_cb = cb;
+        my_c = bc[i];
+      }
+      mb += bm[i];
+      cb += bc[i];
+    }
+    const uint64_t bin = block_max64(my_c > 0 ? my_bin : 0, lds);
+    __syncthreads();
+    if (my_c > 0 && my_bin == bin) {
+      lds[0] = my_mb;
+      lds[1] = my_cb;
+      lds[2] = my_c;
     }
     __syncthreads();
     mass_before = lds[0];
     count_before = lds[1];
     left = static_cast<uint32_t>(lds[2]);
-    prefix = (prefix << 8) | static_cast<uint64_t>(bin);
-    known += 8;
     __syncthreads();
+    return static_cast<int>(bin);
+  };
+  auto pass = [&](auto bin_of_token) __attribute__((always_inline)) -> int {
+    clear();
+    for (int a = first; a < last; ++a) {
+      for_segment(a, [&](float x, uint32_t index) __attribute__((always_inline)) {
+        const uint64_t rank = rank_of(x, index);
+        if (matches(x, rank)) {
+          const int bin = bin_of_token(x, rank);
+          atomicAdd(&mass[lane % kDigitCopies][bin],
+                    static_cast<unsigned long long>(mass_of(expf(x - s.max), unit)));
+          atomicAdd(&count[lane % kDigitCopies][bin], 1u);
+        }
+      });
+    }
+    return choose();
+  };
+  if (left > kThreads) {
+    uint64_t low = ~uint64_t{0}, high = 0;  // of the values' halves of the ranks
+    for (int a = 0; a < segments; ++a) {
+      for_segment(a, [&](float x, uint32_t) __attribute__((always_inline)) {
+        const uint64_t value = rank_of(x, 0) >> 32;
+        low = min(low, value);
+        high = max(high, value);
+      });
+    }
+    low = ~block_max64(~low, lds);
+    high = block_max64(high, lds);
+    top = key_value(~static_cast<uint32_t>(low));
+    if (expf(top - s.max) == 0.0f) {
+      kept_mass = b.mass;
+      return ~uint64_t{0};
+    }
+    const float range = top - key_value(~static_cast<uint32_t>(high));
+    if (range > 0.0f && range < 1024.0f) {
+      per_unit = static_cast<float>(kDigitBins) / range;
+      if (per_unit < 1e30f) bin_chosen = pass([&](float x, uint64_t) { return width_bin(x); });
+    }
+    known = low == high ? 32 : __builtin_clzll(low ^ high) - 32;
+    prefix = low >> (32 - known);
+  }
+  while (left > kThreads && known < 64) {  // (all 64 bits known leave one)
+    if (known == 32) {
+      // One value: its count in each segment.
+      clear();
+      const uint64_t m = mass_of(expf(key_value(~static_cast<uint32_t>(prefix)) - s.max), unit);
+      for (int a = 0; a < segments; ++a) {
+        int mine = 0;
+        for_segment(a, [&](float x, uint32_t index) __attribute__((always_inline)) {
+          mine += matches(x, rank_of(x, index)) ? 1 : 0;
+        });
+        const uint32_t n = __builtin_amdgcn_readlane(wave_inclusive_scan(mine), kWave - 1);
+        if (lane == 0) {
+          atomicAdd(&mass[0][a], static_cast<unsigned long long>(m * n));
+          atomicAdd(&count[0][a], n);
+        }
+      }
+      first = choose();
+      last = first + 1;
+      constexpr int kIndexBits = __builtin_ctz(kSegment);
+      prefix = (prefix << (32 - kIndexBits)) | static_cast<uint64_t>(first);
+      known = 64 - kIndexBits;
+      continue;
+    }
+    const int width = min(kDigit, (known < 32 ? 32 : 64) - known);
+    const int shift = 64 - known - width;
+    const int bin = pass([&](float, uint64_t rank) __attribute__((always_inline)) {
+      return static_cast<int>(rank >> shift) & ((1 << width) - 1);
+    });
+    prefix = (prefix << width) | static_cast<uint64_t>(bin);
+    known += width;
   }
   if (threadIdx.x == 0) taken = 0;
   __syncthreads();
-  for (uint32_t j = threadIdx.x; j < listed; j += kThreads) {
-    uint64_t rank, m;
-    token(j, rank, m);
-    if (known == 0 || rank >> (64 - known) == prefix) {
-      const uint32_t at = atomicAdd(&taken, 1u);
-      c_rank[at] = rank;
-      c_mass[at] = m;
+  auto take = [&](float x, uint32_t index) __attribute__((always_inline)) {
+    const uint64_t rank = rank_of(x, index);
+    if (!matches(x, rank)) return;
+    const uint32_t at = atomicAdd(&taken, 1u);
+    if (at >= kThreads) return;  // (`left` of them)
+    c_rank[at] = rank;
+    c_mass[at] = mass_of(expf(x - s.max), unit);
+  };
+  if (listed <= kThreads) {
+    const uint32_t j = threadIdx.x;
+    if (j < listed) {
+      int a = 0, e = segments;  // start[a] <= j < start[e]
+      while (e - a > 1) {
+        const int mid = (a + e) >> 1;
+        if (start[mid] <= j) a = mid; else e = mid;
+      }
+      const uint32_t index = a * kSegment + w.list[(cell + a) * kSegment + (j - start[a])];
+      take(Elem<T>::load(row, index) / s.t, index);
+    }
+  } else {
+    for (int a = first; a < last; ++a) {
+      for_segment(a, take);
     }
   }
   __syncthreads();
@@ -496,7 +645,7 @@ __global__ __launch_bounds__(kThreads) void sampling_write_kernel(const Rows row
   } else {
     const Boundary b = find_boundary(s, w, r, segments, lds);
     uint64_t kept_mass = 0;
-    last = select_last<T, kSegment>(s, b, w, row, r, segments, unit, lds, kept_mass);
+    last = select_last<T, kVec, kSegment>(s, b, w, row, v, r, segments, unit, lds, kept_mass);
     sum = static_cast<float>(kept_mass) * inv_unit;
   }
   // Tokens whose approximate quotient is below the last kept value by more than the two can

@@ -69,6 +69,62 @@ def test_many_tokens_at_the_boundary(device, vocab):
     check(torch.stack([flat, flat, close, close, peak, peak]).to(device), rows)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("vocab", [513, 20000, 151936, 1048576])
+def test_the_boundary_among_most_of_the_vocabulary(device, vocab, dtype):
+    """Rows whose last kept token lies among most of the vocabulary's: one value everywhere,
+    negative ones, values of both signs far below one peak, two interleaved values, and rows
+    of which all but a few tokens are masked, with -inf or the type's lowest, while top_k asks
+    for more of them."""
+    gen = torch.Generator().manual_seed(vocab)
+    x = torch.randn(8, vocab, generator=gen)
+    allowed = torch.randperm(vocab, generator=gen)[:30]
+    x[0] = -3.25
+    x[1] *= 1e-3
+    x[2, 77] = 25.0
+    x[3] = torch.tensor([2.0, -2.0]).repeat(-(-vocab // 2))[:vocab]
+    x[3, 5] = 40.0
+    for row, mask in ((4, -torch.inf), (5, torch.finfo(dtype).min)):
+        kept = x[row, allowed].clone()
+        x[row] = mask
+        x[row, allowed] = kept
+    x[6] = -x[6].abs() - 20.0
+    x[6, -1] = 1.0
+    x[7] = 5.0 - torch.arange(vocab) * 2.0 ** -14
+    rows = [SamplingParams(0.7, 0, 0.61), SamplingParams(1.0, vocab // 3, 1.0),
+            SamplingParams(1.0, 50, 1.0), SamplingParams(1.0, vocab // 2 + 9, 1.0),
+            SamplingParams(1.0, 50, 1.0), SamplingParams(0.6, 50, 0.999),
+            SamplingParams(1.0, 501, 1.0), SamplingParams(1.3, vocab - 1, 0.9)]
+    check(x.to(dtype).to(device), rows)
+
+
+def test_no_row_costs_many_times_another(device):
+    """A call's time on rows whose boundary lies among the whole vocabulary, against a call on
+    ordinary rows beside it: the selection's few passes over one row's tokens (3 to 6 times,
+    measured), not its steps for every token one after another (20 to 80 times)."""
+    gen = torch.Generator(device=device).manual_seed(4)
+    x = torch.randn(1, 151936, generator=gen, device=device)
+
+    def fastest(logits, params):
+        best = float("inf")
+        for _ in range(8):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(10):
+                ops.sampling_probabilities(logits, params, use_cuda=True)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+    params = [SamplingParams(1.0, 50, 1.0)]
+    ordinary = fastest(x, params)
+    peaked, masked = x.clone(), torch.full_like(x, -torch.inf)
+    peaked[0, 9] = 25.0
+    masked[0, :30] = x[0, :30]
+    for odd in (torch.full_like(x, 1.5), peaked, masked):
+        assert fastest(odd, params) < 12 * ordinary
+
+
 def test_strided_rows_many_rows_and_signed_zeros(device):
     base = torch.randn(300, 1203, device=device)
     base[:, ::2] = 0.0

@@ -164,6 +164,10 @@ __device__ __forceinline__ void for_each(const T* row, int64_t lo, int64_t hi, F
   for (int64_t i = done + threadIdx.x; i < hi; i += kThreads) f(i, Elem<T>::load(row, i));
 }
 
+// An approximate quotient below it errs by more than its own few 2^-23: subnormals (one of
+// temperatures near the largest float) by up to their spacing.
+constexpr float kTinyQuotient = 1e-37f;
+
 // What a workgroup knows of its row before it looks at a logit.
 struct RowState {
   float t, p, max;   // temperature, top_p, the scaled maximum
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(kThreads) void sampling_gather_kernel(const Rows ro
   uint16_t* list = w.list + cell * kSegment;
   // The approximate distance d' = max - l * inv_t is within slack + d' * 1e-6 of the exact
   // one, so a token whose d' misses the bin by more is not in it.
-  const float slack = fabsf(s.max) * 1e-6f;
+  const float slack = fabsf(s.max) * 1e-6f + kTinyQuotient;
   const float near = static_cast<float>(b.bin) / kBinsPerNat * (1.0f - 1e-5f) - slack;
   const float far = b.bin == kBins - 1 ? INFINITY
                                        : static_cast<float>(b.bin + 1) / kBinsPerNat * (1.0f + 1e-5f) + slack;
@@ -652,7 +656,7 @@ __global__ __launch_bounds__(kThreads) void sampling_write_kernel(const Rows row
   // differ are not kept.
   const float value = key_value(~static_cast<uint32_t>(last >> 32));
   const float below = s.mode == kTruncate && s.finite && s.approx
-                          ? value - (fabsf(value) + fabsf(s.max)) * 1e-6f
+                          ? value - ((fabsf(value) + fabsf(s.max)) * 1e-6f + kTinyQuotient)
                           : -INFINITY;
   auto prob = [&](int64_t i, float l) __attribute__((always_inline)) -> float {
     if (s.mode == kGreedy) return static_cast<uint32_t>(i) == s.best ? 1.0f : 0.0f;

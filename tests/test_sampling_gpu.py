@@ -151,6 +151,20 @@ def test_non_finite_rows(device):
         x[keep].to(device), [rows[i] for i in keep], use_cuda=True).cpu())
 
 
+@pytest.mark.parametrize("temperature", [1e30, 1e38, 2.5e38])
+def test_quotients_below_the_normal_range(device, temperature):
+    """Temperatures so large that the scaled logits are subnormal: many tie, and the kept ones
+    are still the first of the order by value, then index. (All are 1 / k: their differences
+    are far below fp32.)"""
+    x = torch.rand(1, 20000, generator=torch.Generator().manual_seed(1)) * 0.05
+    k = 7001
+    got = ops.sampling_probabilities(x.to(device), [SamplingParams(temperature, k, 1.0)], use_cuda=True)
+    order = (x / temperature).sort(dim=-1, descending=True, stable=True).indices[:, :k]
+    want = torch.zeros_like(x).scatter_(1, order, 1.0 / k)
+    assert torch.equal(got.cpu() > 0, want > 0)
+    assert torch.allclose(got.cpu(), want, rtol=1e-6)
+
+
 def test_what_stays_on_the_torch_path(device):
     """Autograd, float64 and parameters outside float32 keep the torch path and its
     results."""

@@ -155,14 +155,17 @@ def test_non_finite_rows(device):
 def test_quotients_below_the_normal_range(device, temperature):
     """Temperatures so large that the scaled logits are subnormal: many tie, and the kept ones
     are still the first of the order by value, then index. (All are 1 / k: their differences
-    are far below fp32.)"""
-    x = torch.rand(1, 20000, generator=torch.Generator().manual_seed(1)) * 0.05
-    k = 7001
-    got = ops.sampling_probabilities(x.to(device), [SamplingParams(temperature, k, 1.0)], use_cuda=True)
-    order = (x / temperature).sort(dim=-1, descending=True, stable=True).indices[:, :k]
-    want = torch.zeros_like(x).scatter_(1, order, 1.0 / k)
-    assert torch.equal(got.cpu() > 0, want > 0)
-    assert torch.allclose(got.cpu(), want, rtol=1e-6)
+    are far below fp32.) Many top_k, so that tokens of the last kept value whose approximate
+    quotient is off are among them."""
+    x = torch.rand(1, 20000, generator=torch.Generator().manual_seed(1)) * 1e-4 + 0.0499
+    ks = range(150, 19500, 151)
+    got = ops.sampling_probabilities(x.expand(len(ks), -1).contiguous().to(device),
+                                     [SamplingParams(temperature, k, 1.0) for k in ks], use_cuda=True)
+    order = (x / temperature).sort(dim=-1, descending=True, stable=True).indices
+    for row, k in zip(got.cpu(), ks):
+        want = torch.zeros(20000).scatter_(0, order[0, :k], 1.0 / k)
+        assert torch.equal(row > 0, want > 0)
+        assert torch.allclose(row, want, rtol=1e-6)
 
 
 def test_what_stays_on_the_torch_path(device):

@@ -45,6 +45,8 @@ from contextlib import contextmanager
 from dataclasses import dataclass
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from mini_vllm import torch_path
 from mini_vllm.kernels.extension import load_extension
@@ -378,10 +380,20 @@ def sampling_probabilities(logits: torch.Tensor, rows, use_cuda: bool = False) -
     return ext.sampling_probabilities(logits, params)
 
 
+def _modes() -> bool:
+    """Whether a dispatch or function mode is to see torch's calls (the one that only picks
+    new tensors' device aside)."""
+    if torch._C._len_torch_dispatch_stack():
+        return True
+    return torch._C._len_torch_function_stack() > 0 and not all(
+        isinstance(m, DeviceContext) for m in _get_current_function_mode_stack())
+
+
 def _plain(x: torch.Tensor) -> bool:
     """A tensor whose memory a kernel may read in torch's place: not a subclass or a
-    functorch wrapper, not under a trace, and with no derivative asked for."""
+    functorch wrapper, not under a trace or a mode, and with no derivative asked for."""
     return (type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing() and not _modes()
             and not torch._C._functorch.is_functorch_wrapped_tensor(x)
             and torch.autograd.forward_ad._current_level < 0
             and not (x.requires_grad and torch.is_grad_enabled()))

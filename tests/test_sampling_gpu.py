@@ -9,6 +9,9 @@ from __future__ import annotations
 import pytest
 import torch
 
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
 from mini_vllm.kernels import ops
 from mini_vllm.sampler import SamplingParams, sampling_probabilities
 from oracle import sampler as oracle
@@ -180,3 +183,34 @@ def test_what_stays_on_the_torch_path(device):
     assert ops.sampling_probabilities(x.double(), rows, use_cuda=True) is None
     for odd in (SamplingParams(1e-40), SamplingParams(1e39), SamplingParams(1.0, 0, 1e-40)):
         assert ops.sampling_probabilities(x, [odd, odd], use_cuda=True) is None
+
+
+def test_modes_and_traces_see_the_torch_path(device):
+    """A dispatch or function mode and a trace see every step, as they did before there were
+    kernels; the mode that only picks new tensors' device hides none."""
+    class Dispatch(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        seen = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen += 1
+            return func(*args, **(kwargs or {}))
+    x = torch.randn(3, 500, device=device)
+    rows = [SamplingParams(0.7, 5, 0.9), SamplingParams(), SamplingParams(1.0, 0, 0.8)]
+    want = sampling_probabilities(x, rows)
+    for mode in (Dispatch(), Function()):
+        with mode:
+            assert ops.sampling_probabilities(x, rows, use_cuda=True) is None
+            got = sampling_probabilities(x, rows)
+        assert mode.seen > 5 and torch.allclose(got, want, rtol=1e-5)
+    with torch.device(device):
+        assert torch.equal(ops.sampling_probabilities(x, rows, use_cuda=True), want)
+    traced = torch.jit.trace(lambda t: sampling_probabilities(t, rows), (x,), check_trace=False)
+    y = torch.randn_like(x)
+    assert torch.allclose(traced(y), sampling_probabilities(y, rows), rtol=1e-5)

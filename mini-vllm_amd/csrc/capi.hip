@@ -74,6 +74,7 @@ struct Options {
   int prefill_share_tiles = mvllm::kPrefillShareTiles;
   int prefill_staging = 0;
   int prefill_pieces = mvllm::kSplitDefaultPieces;
+  uint64_t scratch_bytes = 0;  // > 0: the workspace is this fixed one
   bool share_tiles_given = false;
   bool pieces_given = false;  // prefill_pieces is the caller's, not the default
   int prefill_piece_pct = mvllm::kSplitDefaultPct;
@@ -416,14 +417,22 @@ void plan_decode(Plan& plan, int32_t num_tokens, int32_t num_seqs, int32_t hq, i
     // more workgroups than there are smallest shares in the largest possible batch.
     int64_t wgs = static_cast<int64_t>(o.decode_wgs_per_cu) * device_cus();
     const int64_t least = mvllm::decode_min_share_keys(element_bytes(kv_dtype), d);
-    const int64_t by_size = (static_cast<int64_t>(num_seqs) * max_ctx + least - 1) / least;
+    const int64_t keys = static_cast<int64_t>(num_seqs) * max_ctx;
+    const int64_t by_size = (keys + least - 1) / least;
     if (wgs > by_size) wgs = by_size;
     if (wgs > mvllm::kMaxDecodeShares) wgs = mvllm::kMaxDecodeShares;
     if (wgs < 1) wgs = 1;
-    plan.pub.decode_workgroups = static_cast<int32_t>(wgs);
     // [prefix: num_seqs + 1 int32][O partials][(m, l) partials]
-    const uint64_t entries = static_cast<uint64_t>(wgs + num_seqs) * hq;
     const uint64_t head = align256(static_cast<uint64_t>(num_seqs + 1) * sizeof(int));
+    if (o.scratch_bytes > head + 512) {
+      // A fixed workspace: fewer and so larger shares where their partials need it, up to 64 keys.
+      const int64_t fit = static_cast<int64_t>((o.scratch_bytes - head - 512) / sizeof(float) /
+                                               (static_cast<uint64_t>(hq) * (d + 2))) - num_seqs;
+      const int64_t fewest = (keys + 63) / 64 < 1 ? 1 : (keys + 63) / 64;
+      if (wgs > fit) wgs = fit > fewest ? fit : (wgs < fewest ? wgs : fewest);
+    }
+    plan.pub.decode_workgroups = static_cast<int32_t>(wgs);
+    const uint64_t entries = static_cast<uint64_t>(wgs + num_seqs) * hq;
     plan.off_o = head;
     plan.off_ml = plan.off_o + align256(entries * d * sizeof(float));
     plan.pub.workspace_bytes = plan.off_ml + align256(entries * 2 * sizeof(float));
@@ -727,6 +736,7 @@ int paged_attention_entry(const char* name, void* out, const void* q, const void
   Options o;
   rc = read_options(options, o);
   if (rc != MVLLM_OK) return rc;
+  if (static_scratch) o.scratch_bytes = workspace_bytes;
   if (num_tokens == 0 || num_seqs == 0) return MVLLM_OK;
   if (out == nullptr || q == nullptr || key_pool == nullptr ||
       value_pool == nullptr || block_tables == nullptr || cu_seqlens_q == nullptr ||

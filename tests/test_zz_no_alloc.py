@@ -79,6 +79,24 @@ def test_noalloc_mixed_batch_with_the_grid_prefill(extension, device):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("seqs,context,served", [(260, 60, True), (300, 30, True), (400, 1000, False)])
+def test_noalloc_decode_shares_fit_the_scratch(extension, device, seqs, context, served):
+    """Short contexts of many sequences at head dim 256 and 32 heads, whose smallest shares'
+    partials pass the static scratch: served in larger shares, as long as shares of 64 keys
+    do fit."""
+    b = build_batch([1 + (i * 7) % context for i in range(seqs)], [1] * seqs, dtype=torch.float16,
+                    num_q_heads=32, num_kv_heads=8, head_dim=256, seed=26, device=device)
+    out = torch.full_like(b.q, float("nan"))
+    rc = _noalloc(extension, b, out)
+    torch.cuda.synchronize()
+    if not served:
+        assert rc == 2 and "scratch" in extension.lib.mvllm_last_error().decode()
+        return
+    assert rc == 0, extension.lib.mvllm_last_error().decode()
+    want = extension.paged_attention(*b.args())
+    assert (out.float() - want.float()).abs().max().item() <= 2e-3  # another cut, one fp16 rounding
+
+
 def test_noalloc_refuses_a_plan_larger_than_its_scratch(extension, device):
     b = build_batch([4000], [512], dtype=torch.bfloat16, num_q_heads=16, num_kv_heads=8,
                     head_dim=128, seed=25, device=device)

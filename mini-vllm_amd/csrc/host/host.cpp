@@ -439,6 +439,10 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "mvllm_host", nullptr, -1, kMethod
 
 }  // namespace
 
+// The build's identity, also to be read off the file before it is loaded.
+extern "C" __attribute__((used, visibility("default"))) const char mvllm_host_id[] =
+    "mvllm-host-id:" MVLLM_SOURCE_HASH;
+
 PyMODINIT_FUNC PyInit_mvllm_host() {
   PyObject* m = PyModule_Create(&kModule);
   if (m != nullptr) PyModule_AddStringConstant(m, "source_hash", MVLLM_SOURCE_HASH);

@@ -24,6 +24,8 @@ import importlib.machinery
 import importlib.util
 import math
 import os
+import re
+import shutil
 import struct
 import subprocess
 import sys
@@ -137,14 +139,26 @@ def host_hash() -> str | None:
     return h.hexdigest()[:16]
 
 
-def build_host() -> Path:
-    """Compile ``csrc/host/host.cpp`` (no device code) against torch into ``lib/``."""
+def build_host() -> Path | None:
+    """Compile ``csrc/host/host.cpp`` (no device code) against torch into ``lib/``; None, with
+    a warning, where there is no host compiler or no headers to compile it with: the ops'
+    Python bodies need neither. A compile error raises."""
     include = Path(torch.__file__).resolve().parent / "include"
+    python_include = sysconfig.get_paths()["include"]
+    missing = [what for what, there in (
+        (f"the compiler {CXX}", shutil.which(CXX)),
+        ("torch's headers", (include / "torch/csrc/Exceptions.h").exists()),
+        ("Python's headers", (Path(python_include) / "Python.h").exists())) if not there]
+    if missing:
+        HOST_PATH.unlink(missing_ok=True)
+        print(f"warning: {HOST_SOURCE.name} is not built ({' and '.join(missing)} not found); "
+              "the ops' Python bodies serve its calls", file=sys.stderr)
+        return None
     lib = include.parent / "lib"
     tmp = HOST_PATH.with_suffix(f".so.tmp{os.getpid()}")
     cmd = [CXX, *HOST_FLAGS, f'-DMVLLM_SOURCE_HASH="{host_hash()}"',
            f"-I{INCLUDE_DIR}", f"-I{include}", f"-I{include}/torch/csrc/api/include",
-           "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", str(HOST_SOURCE),
+           "-I/opt/rocm/include", f"-I{python_include}", str(HOST_SOURCE),
            "-o", str(tmp), f"-L{lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
            "-ltorch_python"]
     result = subprocess.run(cmd, capture_output=True, text=True)
@@ -155,24 +169,34 @@ def build_host() -> Path:
 
 
 def open_host():
-    """The host module (``csrc/host/host.cpp``), or None where it is not built: the ops'
-    Python bodies then do its work. One built from other sources is refused."""
+    """The host module (``csrc/host/host.cpp``), or None where it is not built, or, with a
+    warning, where it is not of these sources and this torch (its identity is read before it
+    is loaded: one built against another torch may not load at all): the ops' Python bodies
+    then do its work."""
     if not HOST_PATH.exists():
         return None
-    loader = importlib.machinery.ExtensionFileLoader("mvllm_host", str(HOST_PATH))
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mvllm_host", loader))
-    loader.exec_module(module)
     current = host_hash()
-    if current is not None and module.source_hash != current:
-        raise ToolchainError(f"{HOST_PATH} was built from other sources or for another torch "
-                             f"(build id {module.source_hash}, sources {current}); rebuild it: "
-                             "__graft_entry__.build()")
-    return module
+    found = re.search(rb"mvllm-host-id:([0-9a-f]{16})", HOST_PATH.read_bytes())
+    built = None if found is None else found.group(1).decode()
+    reason = f"build id {built}, sources {current}"
+    if current is None or built == current:
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("mvllm_host", str(HOST_PATH))
+            module = importlib.util.module_from_spec(
+                importlib.util.spec_from_loader("mvllm_host", loader))
+            loader.exec_module(module)
+            return module
+        except ImportError as e:
+            reason = str(e)
+    print(f"warning: {HOST_PATH} was built from other sources or for another torch ({reason}); "
+          "the ops' Python bodies serve its calls until it is rebuilt: __graft_entry__.build()",
+          file=sys.stderr)
+    return None
 
 
 def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every ``csrc/*.hip`` for gfx950 and link ``lib/libminivllm_hip.so``, and
-    build the host module beside it.
+    build the host module beside it (:func:`build_host`).
 
     Always compiles (this is the "does it build" check); objects go to ``_build/``
     and the library is replaced atomically so a running process never maps a

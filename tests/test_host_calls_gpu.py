@@ -55,10 +55,10 @@ def assert_same(native, python):
 
 
 def test_the_built_module_matches_its_source():
-    host = ext_module.open_host()  # refuses a stale build itself
-    if host is None:
+    if not ext_module.HOST_PATH.exists():
         pytest.skip("the host module is not built")
-    assert host.source_hash == ext_module.host_hash()
+    host = ext_module.open_host()  # None for a stale build
+    assert host is not None and host.source_hash == ext_module.host_hash()
     x = torch.zeros(2, 64, dtype=torch.bfloat16)  # host memory: not a call it serves
     entries = host.entries(*[0] * 7)
     assert host.linear_swiglu(entries, {}, x, x, 32) is None
@@ -78,6 +78,35 @@ def test_the_module_has_no_thread_local_storage():
     size, count = struct.unpack_from("<HH", elf, 54)
     kinds = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(count)]
     assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
+
+
+def test_a_module_that_is_not_this_build_is_left_alone(tmp_path, monkeypatch, capsys):
+    """Other sources' or another torch's (told by its id, before it is loaded), or a file that
+    does not load: no module and a warning, and the Python bodies serve, as where there is
+    none."""
+    if not ext_module.HOST_PATH.exists():
+        pytest.skip("the host module is not built")
+    built = ext_module.HOST_PATH.read_bytes()
+    ident = b"mvllm-host-id:" + ext_module.host_hash().encode()
+    assert built.count(ident) == 1
+    path = tmp_path / "mvllm_host.so"
+    monkeypatch.setattr(ext_module, "HOST_PATH", path)
+    assert ext_module.open_host() is None and capsys.readouterr().err == ""  # not built
+    for content in (built.replace(ident, b"mvllm-host-id:0123456789abcdef"), b"not a library",
+                    b"not a library but " + ident):
+        path.write_bytes(content)
+        assert ext_module.open_host() is None
+        assert "rebuilt" in capsys.readouterr().err
+
+
+def test_no_host_compiler_is_no_build_error(tmp_path, monkeypatch, capsys):
+    """Without one the module is left out, a stale one with it, and the library is built."""
+    path = tmp_path / "mvllm_host.so"
+    path.write_bytes(b"stale")
+    monkeypatch.setattr(ext_module, "HOST_PATH", path)
+    monkeypatch.setattr(ext_module, "CXX", "no-such-compiler")
+    assert ext_module.build_host() is None and not path.exists()
+    assert "no-such-compiler" in capsys.readouterr().err
 
 
 @gpu

@@ -3,6 +3,7 @@ where both serve a call, and the Python body's answer or refusal everywhere else
 
 from __future__ import annotations
 
+import math
 import struct
 from contextlib import contextmanager
 
@@ -128,7 +129,13 @@ def test_paged_attention(extension, contexts, lens, dtype, kv):
     served = extension._host.paged_served(q, kp, vp, tables, cu, ctx, seq, mq, mc, 0.1,
                                           b.k_scale, b.v_scale)
     assert served
-    assert_same(*both(extension, op(*args)))
+    native, python = both(extension, op(*args))
+    assert_same(native, python)
+    own = extension._host.paged_attention(  # the native body itself, its workspace there by now
+        extension._entries, extension._workspaces, q, kp, vp, tables, cu, ctx, seq, mq, mc,
+        1.0 / math.sqrt(q.shape[-1]), b.k_scale, b.v_scale)
+    assert own is not None
+    assert_same(own, python)
     stream = torch.cuda.Stream()  # a workspace of its own, not there at the first call
     stream.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(stream):
@@ -160,11 +167,22 @@ def test_projections(extension, m, k, n):
     w = ops.pack_weight(rand(n, k), use_cuda=True)
     wide = rand(m, 2 * k)[:, ::2]  # a strided input
     for a in (x, wide, x.half()):
+        taken = a is x and m <= 64  # the calls that the native bodies are to serve
         def residual_norm(a=a):
             return ops.linear_residual_rmsnorm(a, w, residual, norm, 1e-6, use_cuda=True)
-        assert_same(*both(extension, residual_norm))
+        native, python = both(extension, residual_norm)
+        assert_same(native, python)
+        own = extension.try_linear_residual_rmsnorm(a, w.packed, n, residual, norm, 1e-6)
+        assert (own is not None) == (taken and k > 1024 and n % 512 == 0)
+        if own is not None:
+            assert_same(own, python)
         if n % 32 == 0 and a.dtype == x.dtype:
-            assert_same(*both(extension, lambda a=a: ops.linear_swiglu(a, w, use_cuda=True)))
+            native, python = both(extension, lambda a=a: ops.linear_swiglu(a, w, use_cuda=True))
+            assert_same(native, python)
+            own = extension.try_linear_swiglu(a, w.packed, n)
+            assert (own is not None) == taken
+            if own is not None:
+                assert_same(own, python)
     with extension.recording_workspaces() as held:  # the buffers that a graph keeps alive
         ops.linear_residual_rmsnorm(x, w, residual, norm, 1e-6, use_cuda=True)
     assert bool(held) == (m <= 64 and k > 1024 and n % 512 == 0)
@@ -194,9 +212,20 @@ def test_the_fused_decode_step(extension, contexts, dtype):
                 q, k, v, qw, kw, cos, sin, 1e-6, kp, vp, tables, cu, ctx, seq, max_context,
                 0.09, use_cuda=True), kp, vp
         return call
-    assert_same(*both(extension, op(*views)))
-    assert_same(*both(extension, op(*(t.contiguous() for t in views))))
+    def native_serves(q, k, v, qw=qw):
+        kp2, vp2 = kp.clone(), vp.clone()
+        out = extension.try_paged_decode_qk_norm_rope(q, k, v, qw, kw, cos, sin, 1e-6, kp2, vp2, tables,
+                                                      cu, ctx, seq, mc, 0.09)
+        return None if out is None else (out, kp2, vp2)
+    for rows in (views, [t.contiguous() for t in views]):
+        native, python = both(extension, op(*rows))
+        assert_same(native, python)
+        own = native_serves(*rows)
+        assert own is not None
+        assert_same(own, python)
     q, k, v = views
+    assert native_serves(q, k[:, :-1], v) is None
+    assert native_serves(q, k, v, qw=qw.float()) is None
     assert_same(*both(extension, op(q, k, v.contiguous())))       # k and v apart
     assert_same(*both(extension, op(q, k, v, qw=qw.float())))     # not the kernel's dtype
     assert_same(*both(extension, op(q, k[:, :-1], v)))

@@ -113,6 +113,7 @@ constexpr float kRescaleSlack = 8.0f;
 constexpr int kExactTiles = 12;
 constexpr int kExactEvery = 4;
 
+constexpr int kMaxDecodeWaves = 8;        // of a stream decode workgroup
 constexpr int kMaxDecodeShares = 65535;  // DecodeShares' 32-bit products
 
 // The stream decode's shares: share w owns keys [begin(w), begin(w + 1)) of the `total` laid

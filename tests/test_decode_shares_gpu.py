@@ -41,6 +41,19 @@ def test_sequence_counts_and_smallest_shares(extension, device, dtype, kv_dtype,
     check(extension, b, kv_dtype or dtype)
 
 
+@pytest.mark.parametrize("seqs,kv_heads", [(66, 1), (257, 1), (512, 8), (513, 8), (2049, 2), (4096, 8)])
+def test_prefix_sums_of_many_sequences(extension, device, seqs, kv_heads):
+    """Past 64 sequences each wave of a workgroup (one per kv head here) sums a run of them:
+    runs that end within 64, empty last ones, up to the most sequences a launch takes, prompt
+    chunks, which have no decode keys, among them."""
+    rng = random.Random(seqs)
+    lens = [3 if i % 97 == 50 else 1 for i in range(seqs)]
+    contexts = [rng.choice([3, 16, 17, 31, 40]) for _ in range(seqs)]
+    b = build_batch(contexts, lens, dtype=torch.bfloat16, num_q_heads=2 * kv_heads,
+                    num_kv_heads=kv_heads, head_dim=128, seed=seqs, device="cuda")
+    check(extension, b, torch.bfloat16)
+
+
 @pytest.mark.parametrize("wgs_per_cu", [1, 3, 300])
 @pytest.mark.parametrize("contexts", [[5000], [1, 4999], [4099, 2, 8191], [17] * 40])
 def test_share_division(extension, device, contexts, wgs_per_cu):

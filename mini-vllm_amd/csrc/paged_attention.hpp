@@ -156,9 +156,6 @@ __host__ __device__ inline int64_t share_begin(int64_t w, int64_t total, int64_t
 __host__ __device__ inline int64_t share_owner(int64_t x, int64_t total, int64_t wgs) {
   return ((x + 1) * wgs - 1) / total;
 }
-__host__ __device__ inline bool share_nonempty(int64_t w, int64_t total, int64_t wgs) {
-  return (w * total) / wgs < ((w + 1) * total) / wgs;
-}
 
 // Query heads per decode wave for a GQA group of `group` heads.
 __host__ __device__ inline int decode_group_chunk(int group) {

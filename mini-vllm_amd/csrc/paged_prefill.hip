@@ -6,7 +6,10 @@
 // keys being gathered through the sequence's block table. GQA: query head h reads kv
 // head h / (H_q / H_k).
 //
-// Design (this library's own):
+// Three kernels: the pair kernel (further down, with its own schedule) for GQA pairs at D =
+// 128 over pages of at least 16 keys with a positive scale, which is every prefill of the 0.6B
+// shapes; paged_prefill_lds_kernel for odd groups at D = 128 over 16-bit pools; and
+// paged_prefill_kernel for the rest. Design of the latter two (this library's own):
 //
 //  * work item = (sequence, column, query tile): 128 query positions of HW query heads
 //    (HW = 2 heads of one GQA group when the group is even) against one kv head. Its
@@ -17,8 +20,8 @@
 //    share of all key tiles, whatever the spread of prefix lengths; an item cut
 //    between workgroups leaves (m, l, O) partials that paged_prefill_merge_kernel
 //    combines. A share's partial pieces are at most its first and its last, stored
-//    in slots 2w and 2w + 1. Shares are assigned XCD by XCD. Grid schedule (more than kMaxStreamSeqs sequences): one
-//    workgroup per item, whole.
+//    in slots 2w and 2w + 1. Shares are assigned XCD by XCD. Grid schedule (items for half
+//    the CUs, or more than kMaxStreamSeqs sequences): one workgroup per item, whole.
 //  * workgroup = 4 x HS waves: wave (hs, w) owns query positions 32w .. 32w+31 of
 //    HCW = HW / HS heads. The launches use HS = HW (one head per wave): for a GQA
 //    pair, 8 waves, two per SIMD, one's softmax under the other's MFMAs.
@@ -925,24 +928,23 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_kernel(const PagedPara
 //    instruction, lane i to byte 16 i): no registers, no LDS store instructions. Rows
 //    are 256 B; chunk c of key r is stored at chunk c ^ (r & 7), so the eight keys an
 //    MFMA fragment read serves per LDS cycle fall in distinct banks.
-//  * V is loaded into registers two tiles ahead and written transposed (v_perm pairs)
-//    into V^T rows of 64 keys, ordered as the P^T operand lists them (per 16 keys:
-//    4h..4h+3 then 8+4h..8+4h+3 in chunk 2ks + h), so a PV operand is one
-//    ds_read_b128; the chunks of row d are XOR-swizzled by (d ^ d >> 3) & 7.
-//  * three K buffers, three V^T buffers and three V register sets, each a separate
-//    array picked at compile time (the loop is unrolled by three): the compiler's
+//  * V is copied the same way, rows as they are; the wave that copied them then writes
+//    them transposed (v_perm pairs) into V^T rows of 64 keys, ordered as the P^T operand
+//    lists them (per 16 keys: 4h..4h+3 then 8+4h..8+4h+3 in chunk 2ks + h), so a PV
+//    operand is one ds_read_b128; the chunks of row d are XOR-swizzled by (d ^ d >> 3) & 7.
+//  * three buffers of K rows and three of V rows, each a separate array picked at
+//    compile time (the loop is unrolled by three): the compiler's
 //    wait-count pass then sees that the copies in flight write other arrays than
 //    the ones a step reads and writes, and does not drain them before every LDS
 //    access. Tiles t + 1 and t + 2 are in flight while t is computed.
 //  * before a tile's barrier each wave waits (vmcnt) for its own copies of that tile
 //    only, so the barrier publishes the whole tile.
-template <typename TQ, int HS, bool kStream>
-__global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const PagedParams p) {
+template <typename TQ, bool kStream>
+__global__ __launch_bounds__(256) void paged_prefill_lds_kernel(const PagedParams p) {
   constexpr int D = 128;
-  constexpr int kThreads = 256 * HS;
-  constexpr int kWaves = 4 * HS;
-  constexpr int HW = HS;                  // query heads per work item, one per wave set
-  constexpr int KW = kTileKeys / kWaves;  // keys of a tile staged by one wave (16 or 8)
+  constexpr int kThreads = 256;
+  constexpr int kWaves = 4;
+  constexpr int KW = kTileKeys / kWaves;  // keys of a tile staged by one wave
   constexpr int kCopies = KW / 4;         // 1 KB direct loads per wave per tile
   constexpr int KV = KW / 4;              // V keys per lane: 4 key groups x 16 dim chunks
   constexpr int kKSteps = D / 16;
@@ -954,7 +956,7 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
   // tile loop is untracked asm and the stages are issued in tile order, so waiting down
   // to kStageOps outstanding completes everything but the newest stage.
   constexpr int kStageOps = 2 * kCopies;
-  static_assert(KV == 2 || KV == 4, "V staging map");
+  static_assert(KV == 4, "V staging map");
   static_assert(kTileKeys == kPrefillKeyTile && 32 * 4 == kPrefillQueryTile, "tile sizes");
 
   __shared__ __align__(16) char k_lds0[kTileBytes];
@@ -979,13 +981,9 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
   const int lane = tid % kWave;
   const int l32 = lane & 31;
   const int hsel = lane >> 5;
-  const int hs = wave / 4;  // head of the pair
-  const int wq = wave % 4;  // 32-position query block
 
   const int n = p.num_seqs;
-  const int group = p.hq / p.hk;
-  const int chunks = group / HW;
-  const int cols = p.hk * chunks;
+  const int cols = p.hq;  // one head per work item: column c is query head c
   // Compiled per schedule: the grid's kernel carries none of the stream's cursor
   // seeking (whose registers otherwise spill into the tile loop).
   constexpr bool stream = kStream;
@@ -1085,7 +1083,6 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
   // dims 8 * v_chunk .. +7 per lane) into V^T buffer `vbuf`. Row 8 * v_chunk + e holds
   // them in chunk vt_chunk ^ e: a V^T address has the chunk in bits 4..6 and nothing
   // else there, so the swizzle is one XOR of the lane's row-0 address.
-  typedef __attribute__((address_space(3))) uint32_t lds_u32;
   typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
   auto store_v = [&](auto slot, int vbuf) __attribute__((always_inline)) {
     const char* raw = r_arr(slot) + v_key * kRow + v_chunk * 16;
@@ -1099,12 +1096,8 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
       // dwords, the first operand's in the upper half of the result.
       const uint32_t sel = (e & 1) == 0 ? 0x05040100u : 0x07060302u;
       const uint32_t addr = (row0 ^ (e * 16)) + e * kVRow;
-      if constexpr (KV == 2) {
-        *reinterpret_cast<lds_u32*>(addr) = __builtin_amdgcn_perm(vr[1][e >> 1], vr[0][e >> 1], sel);
-      } else {
-        *reinterpret_cast<lds_u32x2*>(addr) = u32x2{__builtin_amdgcn_perm(vr[1][e >> 1], vr[0][e >> 1], sel),
-                                                    __builtin_amdgcn_perm(vr[3][e >> 1], vr[2][e >> 1], sel)};
-      }
+      *reinterpret_cast<lds_u32x2*>(addr) = u32x2{__builtin_amdgcn_perm(vr[1][e >> 1], vr[0][e >> 1], sel),
+                                                  __builtin_amdgcn_perm(vr[3][e >> 1], vr[2][e >> 1], sel)};
     }
   };
 
@@ -1118,7 +1111,7 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
 
   auto begin_piece = [&]() __attribute__((always_inline)) {
     const int offset = cur.context - cur.len;
-    const int w_first = cur.q * kPrefillQueryTile + 32 * wq;
+    const int w_first = cur.q * kPrefillQueryTile + 32 * wave;
     w_active = w_first < cur.len;
     w_kv_end = offset + min(w_first + 32, cur.len);
     w_kv_full = offset + w_first + 1;
@@ -1126,7 +1119,7 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
     my_valid = my_local < cur.len;
     my_visible = offset + my_local + 1;
     row_base = sload(p.cu_seqlens_q + cur.s);
-    head0 = (cur.c / chunks) * group + (cur.c % chunks) * HW + hs;
+    head0 = cur.c;
     piece_t0 = cur.t;
     piece_u0 = cur.u;
     const int local = min(my_local, cur.len - 1);
@@ -1256,7 +1249,7 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
       }
     } else {
       const int64_t slot = 2 * static_cast<int64_t>(share) + (piece_u0 == u0 ? 0 : 1);
-      const int64_t prow = (slot * HW + hs) * kPrefillQueryTile + (my_local - cur.q * kPrefillQueryTile);
+      const int64_t prow = slot * kPrefillQueryTile + (my_local - cur.q * kPrefillQueryTile);
       float* po = p.pf_o + prow * D;
 #pragma unroll
       for (int db = 0; db < kDBlocks; ++db) {
@@ -1334,7 +1327,9 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
 
 // The kernel of GQA pairs at D = 128 (pages of >= 16 keys, a positive scale, 16-bit and fp8
 // pools): a work item is kWaves * 16 query positions of two heads against one kv head, one
-// wave per (head, 32 positions).
+// wave per (head, 32 positions). Which items are of 64 and which of 128 positions, whole or cut,
+// on the grid or in the order of a list, is the host's choice (pair_mode and plan_whole in
+// capi.hip, with both sides' times).
 //
 // What bounds it: per wave and 64-key tile 32 MFMAs (1024 matrix cycles), ~130 vector
 // instructions of softmax (32 of them v_exp_f32), and 32 KB of K/V fragments from LDS, no two
@@ -1344,8 +1339,8 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
 // copies of its tiles.
 //
 // Why this layout:
-//  * workgroups of four waves and 64 KB of LDS, two to a CU, not one of eight: twice the items
-//    (a 512-token chunk is 64 of them, not 32), one workgroup's waits, barriers, prologue
+//  * workgroups of four waves and 64 KB of LDS (80 over fp8), two to a CU, not one of eight: twice
+//    the items (a 512-token chunk is 64 of them, not 32), one workgroup's waits, barriers, prologue
 //    and epilogue run beside the other's MFMAs, and four waves meet at a barrier
 //    instead of eight. Against the eight-wave kernel it replaced, which kept three staged tiles
 //    and a transposed copy of V in 128 KB: 8 x 512 tokens after up to 1536 keys 59.6 -> 52
@@ -1362,7 +1357,9 @@ __global__ __launch_bounds__(256 * HS) void paged_prefill_lds_kernel(const Paged
 //  * tried, no faster: copies with a step and a half to land (a second barrier per tile), six
 //    fragments read ahead, a raised wave priority in the MFMA phases.
 //  * fp8 pools: each wave's own rows are staged as codes and converted, times the page's
-//    scale, into the same buffers before the barrier.
+//    scale, into the same buffers before the barrier. With eight waves a tile is converted for
+//    twice the positions: five chunks of 61-512 tokens beside 28 decodes 93 -> 80 us a call,
+//    with the schedule's balance.
 template <typename TQ, typename TKV, int kWaves, bool kSplit>
 __global__ __launch_bounds__(kWaves * kWave, 2) void paged_prefill_pair_kernel(const PagedParams p) {
   constexpr bool kFp8 = std::is_same_v<TKV, fp8_t>;
@@ -2121,11 +2118,11 @@ void launch_prefill_pair(const PagedParams& p, int max_query_len, hipStream_t st
 template <typename TQ>
 void launch_prefill_lds(const PagedParams& p, int max_query_len, hipStream_t stream) {
   if (p.pf_wgs > 0) {
-    paged_prefill_lds_kernel<TQ, 1, true><<<p.pf_wgs, 256, 0, stream>>>(p);
+    paged_prefill_lds_kernel<TQ, true><<<p.pf_wgs, 256, 0, stream>>>(p);
     paged_prefill_merge_kernel<TQ, 128, 1><<<kMergeSub * p.pf_wgs, kMergeThreads, 0, stream>>>(p);
   } else {
     const int qtiles = (max_query_len + kPrefillQueryTile - 1) / kPrefillQueryTile;
-    paged_prefill_lds_kernel<TQ, 1, false><<<dim3(p.hq, p.num_seqs, qtiles), 256, 0, stream>>>(p);
+    paged_prefill_lds_kernel<TQ, false><<<dim3(p.hq, p.num_seqs, qtiles), 256, 0, stream>>>(p);
   }
 }
 

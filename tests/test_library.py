@@ -88,14 +88,16 @@ def _plan(lib, *args, options=None):
     return plan
 
 
-SLOT_BYTES = 8 * 64 * 66 * 4  # one piece's (m, l, O) partial: 8 waves x 64 lanes
+# One piece's (m, l, O) partial: two heads x 128 query positions x 130 floats (133120 bytes),
+# rounded up to 8 waves x 64 lanes x 66 floats.
+SLOT_BYTES = 8 * 64 * 66 * 4
 
 
 def test_prefill_grid_schedule_workspace(lib):
-    """Enough 128-query items to fill the CUs: the grid schedule. Where the pipelined
+    """Enough 128-query items to fill the CUs: the grid schedule. Where the pair
     kernel runs it (D 128, GQA pairs, 16-bit or fp8 pools, <= 64 items) it may cut long
     items into pieces, whose partial slots are the only workspace it needs; with
-    prefill_pieces = 1 (or where the pipelined kernel does not run) it needs none."""
+    prefill_pieces = 1 (or where the pair kernel does not run) it needs none."""
     plan = _plan(lib, 4096, 8, 16, 8, 128, 16, 512, 2048, 2, 2)
     assert plan.prefill_mfma == 1 and plan.prefill_workgroups == 0
     assert plan.prefill_pieces == 8

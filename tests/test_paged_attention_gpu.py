@@ -239,7 +239,7 @@ def test_prefill_schedules_in_a_mixed_fp8_batch(extension, device, schedule):
 
 @pytest.mark.parametrize("block_size", [16, 32, 64])
 def test_fp8_prefill_on_the_pipelined_grid_kernel(extension, device, block_size):
-    """fp8 pools on the grid schedule take the pipelined kernel (codes staged straight
+    """fp8 pools on the grid schedule take the pair kernel (codes staged straight
     into LDS, dequantised there with each page's scale): ragged prefixes, partial last
     tiles, a decode row, pages of 16 to 64 keys."""
     b = case([1500, 700, 130, 65, 3000], [512, 300, 130, 1, 200], device, dtype=torch.bfloat16,
@@ -256,10 +256,10 @@ def _split(pieces, share_tiles=1):
 @pytest.mark.parametrize("pieces", [2, 3, 16])
 @pytest.mark.parametrize("kv_dtype", [torch.bfloat16, torch.float8_e4m3fn])
 def test_split_grid_cuts_long_items(extension, device, pieces, kv_dtype):
-    """The grid cuts items longer than ~1.2x the mean work per CU into key ranges run by
-    workgroups of their own in the same launch, the last piece to finish merging the
-    others: a 6000-key prefix beside short chunks (its items cut into up to 5 pieces),
-    ragged chunk ends, a decode row, an fp8 pool."""
+    """Items longer than a set part of the mean work per CU are cut into key ranges run by
+    workgroups of their own, which a second launch merges: a 6000-key prefix beside short
+    chunks (its items cut into up to `pieces` pieces), ragged chunk ends, a decode row,
+    an fp8 pool."""
     b = case([6000, 700, 130, 65, 3000], [512, 300, 130, 1, 200], device, dtype=torch.bfloat16,
              kv_dtype=kv_dtype, num_q_heads=16, num_kv_heads=8, head_dim=128)
     plan = extension.paged_attention_plan(b.q.shape[0], 5, 16, 8, 128, 16, 512, 6000,
@@ -270,10 +270,9 @@ def test_split_grid_cuts_long_items(extension, device, pieces, kv_dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_split_grid_one_long_prompt(extension, device, dtype):
-    """One sequence alone: every item long against the mean, so each is cut (up to 7
-    pieces of ~13 tiles); whichever piece finishes last folds them in piece order, so
-    three calls in a row give the same bits (and each finds the arrival counters left
-    at zero by the one before)."""
+    """One sequence alone: every item long against the mean, so each is cut; the merge
+    folds the pieces in piece order whatever order they finished in, so three calls in a
+    row give the same bits."""
     b = case([6100], [512], device, dtype=dtype, num_q_heads=16, num_kv_heads=8, head_dim=128)
     want = oracle(b)
     first = None
@@ -590,10 +589,9 @@ def test_the_torch_path_runs_on_device_without_cuda_requested(extension, device)
 
 
 def test_a_captured_split_prefill_runs_items_whole(extension, device):
-    """A split-grid prefill captured into a graph must not name its stream's arrival
-    counters (a replay on another stream could overlap a launch on the capture stream):
-    captured, it runs every item whole - counted by split_stats - and each replay, also
-    on another stream, matches the oracle and the eager whole-item call's bits."""
+    """A split-grid prefill captured into a graph runs every item whole - counted by
+    split_stats - and each replay, also on
+    another stream, matches the oracle and the eager whole-item call's bits."""
     b = case([6000, 700], [512, 300], device, dtype=torch.bfloat16, num_q_heads=16,
              num_kv_heads=8, head_dim=128)
     opts = _split(8)

@@ -265,8 +265,10 @@ PairWork pair_work(int32_t num_tokens, int32_t num_seqs, int32_t hq, int32_t max
 // 160 up to 84 96 and 83, 200 up to 88 95 and 107; fp8, 144 up to 34 68 and 60, 200 up to 25
 // 49 and 59, 232 up to 55 102 and 93, 256 up to 32 60 and 64, up to 126 205 and 167.
 // More still: whole. 128 positions over fp8 from one and a half a CU, but for chunks that
-// are long against their context (their items differ so much that fewer pair badly): 440 items
-// of 8 chunks 73 and 65 us, 400 of one fresh chunk of 1600 tokens 48 and 55.
+// are long against their context (their items differ so much that fewer pair badly) up to two
+// and a half: 440 items of 8 chunks 73 and 65 us, 400 of one fresh chunk of 1600 tokens 48 and 55,
+// 512 of two of 2048 63 and 71, 768 of three 84 and 75, 1024 of one of 8192 350 and 304. Never
+// for chunks of at most 64 tokens, which fill half of such an item: 384 of 48 chunks 67 and 100.
 struct PairMode {
   int tile;
   bool cut;
@@ -275,7 +277,8 @@ PairMode pair_mode(const PairWork& w, int32_t num_seqs, int32_t hq, int32_t max_
   const bool fp8 = kv_dtype == mvllm::kFP8E4M3;
   // A grid of very many positions is halved (1500 decodes and 2048 tokens, 384K: 738 -> 700 us).
   const bool vast = static_cast<int64_t>(num_seqs) * ((max_q + 63) / 64) * (hq / 2) >= 128 * 1024;
-  const PairMode whole{vast || (fp8 && 2 * w.wgs >= 3 * cus && max_q <= 32 * w.n) ? 128 : 64, false};
+  const bool wide = fp8 && ((2 * w.wgs >= 3 * cus && max_q <= 32 * w.n) || 2 * w.wgs >= 5 * cus);
+  const PairMode whole{max_q > 64 && (vast || wide) ? 128 : 64, false};
   // Past 64 sequences the schedule is a launch of its own, and the list and the merge have a
   // position per sequence and column: about 6 us and 1.5 ns each.
   const int64_t n = w.n - (num_seqs > 64 ? 6 + static_cast<int64_t>(num_seqs) * hq / 1333 : 0);

@@ -139,6 +139,11 @@ def test_prefill_grid_schedule_workspace(lib):
     ((4096, 8, 512, 2048), 2, 64, 0),
     ((4096, 8, 512, 2048), 3, 128, 0),
     ((2048, 1, 2048, 2048), 3, 64, 0),
+    ((4096, 2, 2048, 2048), 3, 64, 0),
+    ((8192, 4, 2048, 2048), 3, 128, 0),
+    # chunks that would fill half of a larger item
+    ((3072, 48, 64, 2064), 3, 64, 0),
+    ((4160, 64, 65, 2064), 3, 128, 0),
 ])
 def test_pair_prefill_plan(lib, sizes, kv, item, listed):
     """The pair kernel's items and whether they are listed and cut: batches on either side

@@ -300,16 +300,20 @@ PairMode pair_mode(const PairWork& w, int32_t num_seqs, int32_t hq, int32_t max_
 // scan. Past one item a CU a sequence's items run one after another from contexts of 44 tiles
 // on, by the schedule in any case, so that they meet in the L2 (320 items of up to 84 tiles: 119
 // us and 130 with all sequences' last query tiles first, over fp8 156 and 168), before
-// that the longest of all first (440 of up to 27 tiles over fp8: 68 and 73).
+// that the longest of all first (440 of up to 27 tiles over fp8: 68 and 73). Chunks of unequal
+// length, whose grid has a few holes, one after another whatever their contexts: 864 items of 16
+// chunks of 256-512 tokens after up to 1536 keys 82 us on the grid, 70 so, over fp8 106 and 86; 760
+// of 8 chunks of 512-1020 88 and 76, over fp8 110 and 92.
 void plan_whole(Plan& plan, const PairWork& w, int32_t num_tokens, int32_t num_seqs, int32_t hq,
                 int32_t max_q, int tile, int cus) {
   plan.split_tile = tile;
   plan.split_pieces = 0;
   const int64_t grid = static_cast<int64_t>(num_seqs) * ((max_q + tile - 1) / tile);
   const int64_t live = (w.tokens + tile - 1) / tile + w.chunks / 2;
-  plan.split_by_seq = w.n >= 44;
-  if ((grid >= 2 * live || (w.wgs > cus && plan.split_by_seq && num_seqs > 1)) &&
-      num_seqs <= 64) {
+  const bool holes = grid >= 2 * live;
+  const bool ragged = 20 * grid >= 21 * live;
+  plan.split_by_seq = w.n >= 44 || !holes;
+  if ((holes || (w.wgs > cus && num_seqs > 1 && (w.n >= 44 || ragged))) && num_seqs <= 64) {
     plan_ranked(plan, num_tokens, num_seqs, hq, max_q, tile, cus, 100, 1);
   }
 }

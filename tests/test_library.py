@@ -141,6 +141,9 @@ def test_prefill_grid_schedule_workspace(lib):
     ((2048, 1, 2048, 2048), 3, 64, 0),
     ((4096, 2, 2048, 2048), 3, 64, 0),
     ((8192, 4, 2048, 2048), 3, 128, 0),
+    # unequal chunks: the grid has a few holes
+    ((6404, 16, 512, 2048), 2, 64, 1),
+    ((6404, 16, 512, 2048), 3, 128, 1),
     # chunks that would fill half of a larger item
     ((3072, 48, 64, 2064), 3, 64, 0),
     ((4160, 64, 65, 2064), 3, 128, 0),

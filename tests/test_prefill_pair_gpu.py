@@ -79,6 +79,7 @@ def test_the_default_cuts_a_lone_long_chunk(extension, device):
 ROUTES = {
     "whole, last query tiles first": ([129, 64, 2, 200, 65], [0, 100, 62, 57, 191], 20, 300, 16, None, 64, 1),
     "whole, by sequence": ([256, 255, 257], [2400, 2345, 2000], 5, 900, 32, None, 64, 1),
+    "whole, a few holes": ([512, 300, 201, 449], [0, 65, 500, 127], 0, 300, 32, None, 64, 1),
     "whole, fp8 items of 128": ([390, 385, 388, 384], [500, 0, 127, 64], 6, 700, 32, F8, 128, 1),
     "cut, items of 128": ([130, 257, 65, 500], [4870, 4000, 4800, 4500], 3, 900, 16, None, 128, 64),
     "cut, fp8 items of 128": ([130, 257, 65, 500], [3870, 3000, 3800, 3500], 3, 900, 16, F8, 128, 64),

@@ -4,9 +4,9 @@
 // What bounds a small eager call is the host, not the GPU: in Python the same work (some eighty
 // attribute reads, two ctypes calls of up to thirty arguments) took 8-11 us a call. Measured in
 // back-to-back eager calls, with the Python body and with this one: a lone sequence's fused
-// decode attention 21.1 -> 16.4 us (its kernels alone: 16.5), the two MLP
-// launches of 32 rows 22 -> 15.1 us (kernels alone: 13.5), four float32 sequences' decode
-// attention 16.7 -> 15.5 us (kernels: 15.6).
+// decode attention 21.1 -> 16.3 us (its kernels alone: 16.2), the MLP's three
+// launches of 32 rows 22 -> 13.4 us (kernels alone: 13.2), four float32 sequences' decode
+// attention 16.7 -> 15.2 us (kernels: 14.9).
 //
 // Every function serves the calls whose arguments are exactly what the kernels take and
 // answers None to anything else - another type, dtype, shape, stride, device or integer kind, a

@@ -762,7 +762,7 @@ int paged_attention_entry(const char* name, void* out, const void* q, const void
   Plan plan = make_plan(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim, block_size,
                         max_query_len, max_context_len, q_dtype, kv_dtype, o);
   if (static_scratch && plan.pub.workspace_bytes > workspace_bytes && plan.pub.prefill_pieces > 1) {
-    // The split grid's partial slots do not fit the static scratch: items stay whole.
+    // The cut items' partial slots do not fit the static scratch: items stay whole.
     o.prefill_pieces = 1;
     plan = make_plan(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim, block_size,
                      max_query_len, max_context_len, q_dtype, kv_dtype, o);

@@ -11,10 +11,9 @@ and leave these paths idle, so here they are driven on purpose:
 * decode: the stream schedule (a sequence cut into many shares, merged by the merge
   kernel) with the spike in its first, a middle and its last share, and the grid
   schedule (splits of 64-1024 keys, its own merge);
-* prefill: the item grid, the split grid (long items cut into key-range pieces in one
-  launch, the last piece folding the others), the stream schedule (shares of all key
-  tiles, cut items merged after), the register-staged kernel, and fp32 rows (the
-  decode kernel run by row);
+* prefill: the item grid, the split grid (long items cut into key-range pieces, merged
+  by a second launch), the stream schedule (items cut for equal work per CU, merged
+  after), the register-staged kernel, and fp32 rows (the decode kernel run by row);
 * the prefill kernels' lazy rescale: the running max is raised only when a tile's max
   exceeds it by more than 8 log2 units, so a staircase of scores with steps just below
   and just above that slack, placed in different tiles, split pieces and stream shares,

@@ -284,12 +284,15 @@ def test_split_grid_one_long_prompt(extension, device, dtype):
 
 
 def test_split_grid_matches_the_whole_item_grid(extension, device):
-    """Config 3's shape on the split grid (the default) and with every item whole: both
-    within tolerance of the oracle and of each other."""
+    """Config 3's shape with its long items cut and with every item whole (what the planner
+    picks for it): within tolerance of each other, and not the same run."""
     b = config_batch(3, device=device)
     whole = kernel(extension, b, {"prefill_schedule": "grid", "prefill_pieces": 1})
-    split = kernel(extension, b, {"prefill_schedule": "grid"})
+    split = kernel(extension, b, {"prefill_schedule": "grid", "prefill_pieces": 8,
+                                  "prefill_piece_pct": 50})
     assert_max_abs(split.float(), whole.float(), 2 * ATTN_ATOL[torch.bfloat16], "split vs whole")
+    assert not torch.equal(split, whole)
+    assert torch.equal(kernel(extension, b, {"prefill_schedule": "grid"}), whole)
 
 
 def test_split_grid_piece_lengths_and_bounds(extension, device):

@@ -153,7 +153,7 @@ CONFIGS = {
 
 def config_batch(index: int, device: torch.device | str = "cpu", seed: int = 0,
                  generator_device: str = "cpu", kv_dtype: torch.dtype | None = None) -> PagedBatch:
-    """The BASELINE.json config ``index`` (1-4), GQA 16q/8kv, D=128, 16-token pages.
+    """The benchmark workload ``index`` (1-4), GQA 16q/8kv, D=128, 16-token pages.
 
     Lengths are drawn from their own generator (seed ``seed``) so the shapes do not
     depend on the tensor draws; pools for configs 2-4 hold the needed pages + 10%.
